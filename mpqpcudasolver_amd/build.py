@@ -4,11 +4,18 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 _DIR = os.path.dirname(os.path.abspath(__file__))
-SOURCES = [os.path.join(_DIR, "csrc", "mpqp_hip.hip")]
-DEPS = [os.path.join(_DIR, "csrc", f) for f in ("lp_engine.hpp", "kernels.hpp", "opt_kernel.hpp", "regions.hpp")] + [
+_CSRC = os.path.join(_DIR, "csrc")
+DEPS = [os.path.join(_CSRC, f) for f in ("lp_engine.hpp", "kernels.hpp", "opt_kernel.hpp", "reg_kernel.hpp", "opt_fn.hpp",
+                                         "regions.hpp")] + [
     os.path.join(os.path.dirname(_DIR), "include", "mpqp_hip.h")]
+# (source, extra flags): the library's host code and small kernels, then the
+# groups of optimality kernels (csrc/opt_fn.hpp), longest compilations first
+UNITS = [(os.path.join(_CSRC, "opt_fn.hip"), [f"-DMPQP_PART={p}"]) for p in (2, 3, 6, 7, 1, 0, 13, 12, 5, 4, 11, 10, 9, 8)] + [
+    (os.path.join(_CSRC, "mpqp_hip.hip"), [])]
 OUT = os.path.join(_DIR, "libmpqp_hip.so")
 
 HIPCC_FLAGS = [
@@ -32,16 +39,28 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
-def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
-    """Compiles the HIP sources into libmpqp_hip.so; returns its path."""
-    tmp = OUT + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, *(extra_flags or []), "-o", tmp, *SOURCES]
+def _run(cmd: list[str], verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed ({r.returncode}):\n{r.stderr[-8000:]}")
-    os.replace(tmp, OUT)
+
+
+def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
+    """Compiles the HIP sources side by side and links libmpqp_hip.so;
+    returns its path."""
+    compile_flags = [f for f in HIPCC_FLAGS if f != "-shared"]
+    workers = max(1, min(len(UNITS), int(os.environ.get("MAX_JOBS") or os.cpu_count() or 1)))
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(workers) as pool:
+        objs = [os.path.join(tmp, f"unit{i}.o") for i in range(len(UNITS))]
+        jobs = [pool.submit(_run, [hipcc(), *compile_flags, *flags, *(extra_flags or []), "-c", "-o", obj, src], verbose)
+                for obj, (src, flags) in zip(objs, UNITS)]
+        for j in jobs:
+            j.result()
+        out = OUT + ".tmp"
+        _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *objs], verbose)
+    os.replace(out, OUT)
     return OUT
 
 

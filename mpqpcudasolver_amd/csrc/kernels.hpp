@@ -57,6 +57,7 @@ struct OptArgs {
     unsigned char *gtab;  // split tableaus: rows [split_rows, M2) of each workgroup's in global
     long long gtab_stride;  // memory (the tableau does not fit in LDS), or null
     int split_rows;       // rows of a split tableau held in LDS (even), with the cost row
+    int stage_passes;     // register tableau: passes that stage its rows through LDS
 };
 
 // Byte layout of one stored state: T (rows x cols doubles, contiguous) then
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(NT) void feas_kernel(FeasArgs a) {
 // ascending, as the host enumeration), and the list of feasible candidates.
 // Counts are turned into offsets by an exclusive scan between the kernels.
 // ---------------------------------------------------------------------
-__global__ void child_count(const DevRecord *prec, const int *psets, int pn, int kw, int level, int n_c, int *cnt) {
+static __global__ void child_count(const DevRecord *prec, const int *psets, int pn, int kw, int level, int n_c, int *cnt) {
     const int pi = blockIdx.x * blockDim.x + threadIdx.x;
     if (pi >= pn) return;
     const int mx = level >= 2 ? psets[(long long)pi * kw + level - 2] : -1;
@@ -258,7 +259,7 @@ __global__ void child_count(const DevRecord *prec, const int *psets, int pn, int
 
 // p1par[child] = parent whenever the parent's phase 1 ended optimal (its
 // phase-1 state warm-starts the child), else -1
-__global__ void child_write(const DevRecord *prec, const int *psets, const int *off, const int *cnt, int pn, int kw,
+static __global__ void child_write(const DevRecord *prec, const int *psets, const int *off, const int *cnt, int pn, int kw,
                             int level, int *sets, int *par, int *p1par) {
     const int pi = blockIdx.x * blockDim.x + threadIdx.x;
     if (pi >= pn) return;
@@ -279,7 +280,7 @@ __global__ void child_write(const DevRecord *prec, const int *psets, const int *
 // child_write over parents [p0, p0 + pn) of a chunk: off[t] is parent
 // p0 + t's first child relative to the range; par holds chunk-wide parent
 // indices (their rows in the parent chunk's state stores)
-__global__ void child_write_range(const DevRecord *prec, const int *psets, const int *off, int p0, int pn, int kw,
+static __global__ void child_write_range(const DevRecord *prec, const int *psets, const int *off, int p0, int pn, int kw,
                                   int level, int n_c, int *sets, int *par, int *p1par) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= pn) return;
@@ -299,7 +300,7 @@ __global__ void child_write_range(const DevRecord *prec, const int *psets, const
 }
 
 // rows[t] = sets[idx[t]] widened to nx entries, -1 padded (t < cnt)
-__global__ void gather_rows_nx(const int *sets, const int *idx, int cnt, int kw, int nx, int *rows) {
+static __global__ void gather_rows_nx(const int *sets, const int *idx, int cnt, int kw, int nx, int *rows) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e < cnt * nx) {
         const int t = e / nx, u = e - t * nx;
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(NT) void gram_solve(double *W, int n_x, int ld, int
 // Lane l supplies A[i0 + l % 16][k + l / 16] and Y[k + l / 16][j0 + l % 16]
 // and receives G[i0 + 4 r + l / 16][j0 + l % 16] in result register r = 0..3
 // (the result layout of this instruction, measured on gfx950).
-__global__ __launch_bounds__(64) void gram_mfma(const double *A, const double *Y, int n_c, int n_x, int ldy,
+static __global__ __launch_bounds__(64) void gram_mfma(const double *A, const double *Y, int n_c, int n_x, int ldy,
                                                  double *G) {
     typedef double v4d __attribute__((ext_vector_type(4)));
     const int tiles = (n_c + 15) / 16;
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(64) void licq_screen(const double *G, int n_c, cons
     if (live && r == 0) fail[c] = bad ? 1 : 0;
 }
 
-__global__ void feasible_flag(const DevRecord *rec, int n, int *flag) {
+static __global__ void feasible_flag(const DevRecord *rec, int n, int *flag) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c < n) flag[c] = rec[c].feasible ? 1 : 0;
 }
@@ -390,7 +391,7 @@ __global__ void feasible_flag(const DevRecord *rec, int n, int *flag) {
 // the final-set flags.  out[0] feasibility pivots; [1] phase-1 / [2] phase-2
 // pivots of the optimality LPs kept in the first precision; [3] / [4] those
 // of the LPs re-solved in FP64; [5] re-solves.  One atomic per block and sum.
-__global__ void level_summary(const DevRecord *rec, int n, unsigned long long *out, int *flag) {
+static __global__ void level_summary(const DevRecord *rec, int n, unsigned long long *out, int *flag) {
     __shared__ unsigned long long s[6];
     if (threadIdx.x < 6) s[threadIdx.x] = 0ull;
     __syncthreads();
@@ -409,7 +410,7 @@ __global__ void level_summary(const DevRecord *rec, int n, unsigned long long *o
 }
 
 // rows[t] = sets[idx[t]] (kw ints each) for t < cnt
-__global__ void gather_rows(const int *sets, const int *idx, int cnt, int kw, int *rows) {
+static __global__ void gather_rows(const int *sets, const int *idx, int cnt, int kw, int *rows) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e < cnt * kw) {
         const int t = e / kw, u = e - t * kw;
@@ -417,7 +418,7 @@ __global__ void gather_rows(const int *sets, const int *idx, int cnt, int kw, in
     }
 }
 
-__global__ void list_write(const int *flag, const int *pos, int n, int *list) {
+static __global__ void list_write(const int *flag, const int *pos, int n, int *list) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c < n && flag[c]) list[pos[c]] = c;
 }
@@ -475,6 +476,7 @@ struct P2Pred {  // min_idx_kernel_optimal, batched_simplex.cu:343-344
 };
 
 #include "opt_kernel.hpp"
+#include "reg_kernel.hpp"
 
 // ---------------------------------------------------------------------
 // Root: S = {} KKT basis tableau (one workgroup, tableau in global memory)
@@ -488,6 +490,7 @@ struct RootArgs {
     int *rowof;       // N2
     int *slotof;      // N2
     double *root;     // M2 x (K2+2)
+    float *root32;    // the same in FP32, as a stored phase-1 state, or null
     int *root_basis;  // M2
     int *root_nonb;   // K2
     int *root_ok;
@@ -593,7 +596,14 @@ __global__ __launch_bounds__(NT) void root_kernel(RootArgs a) {
             const int pp = e / ld, kk = e - pp * ld;
             const int src = a.rowof[a.root_basis[pp]];
             const int sc = kk < K ? a.slotof[a.root_nonb[kk]] : kk;
-            a.root[e] = G[src * ld + sc];
+            const double v = G[src * ld + sc];
+            a.root[e] = v;
+            if (a.root32) a.root32[pp * opt_ld<float>(K) + kk] = (float)v;
+        }
+        if (a.root32) {
+            int *db = reinterpret_cast<int *>(a.root32 + (long long)opt_tw<float>(M, K));
+            for (int i = tid; i < M; i += NT) db[i] = a.root_basis[i];
+            for (int kk = tid; kk < K; kk += NT) db[M + kk] = a.root_nonb[kk];
         }
     }
     if (tid == 0) *a.root_ok = sh_ok;

@@ -74,6 +74,7 @@ struct DevProb {
     const int *root_basis;   // M2
     const int *root_nonb;    // K2
     const int *root_ok;      // 1 int
+    const float *root32;     // the root rounded to FP32, laid out as a stored phase-1 state
     double cert_ptol;        // primal certification: 1e-12 * (1 + max|xb2|)
     // A2 (column-major, M2 x N2) in sparse form for the FP64 certification,
     // without the stationarity-row entries of the w columns in the row lists.
@@ -154,15 +155,15 @@ __device__ __forceinline__ int shfl_down_i(int v, int d) {
 
 // lane_down<I>(x): lane t receives lane t + I (valid for t < I <= 32, the
 // only lanes the reference tree reads), without an LDS round trip:
-// DPP row_shl for I <= 8 (inside a 16-lane row), ds_swizzle SWAP16 for 16,
-// v_permlane32_swap (gfx950) for 32.
+// DPP row_shl for I <= 8 (inside a 16-lane row), v_permlane16_swap and
+// v_permlane32_swap (gfx950) for 16 and 32.
 template <int I>
 __device__ __forceinline__ int lane_down_i(int x) {
     static_assert(I == 1 || I == 2 || I == 4 || I == 8 || I == 16 || I == 32, "stride");
     if constexpr (I <= 8) {
         return __builtin_amdgcn_update_dpp(x, x, 0x100 + I, 0xf, 0xf, false);
     } else if constexpr (I == 16) {
-        return __builtin_amdgcn_ds_swizzle(x, 0x401F);
+        return __builtin_amdgcn_permlane16_swap(x, x, false, false)[1];
     } else {
         return __builtin_amdgcn_permlane32_swap(x, x, false, false)[1];
     }
@@ -191,7 +192,7 @@ __device__ __forceinline__ double max_step(double v, int lane) {
     return ((lane < I) & (o > v)) ? o : v;
 }
 
-// Wave maximum (order-free): DPP / swizzle / permlane steps into lane 0,
+// Wave maximum (order-free): DPP / permlane steps into lane 0,
 // then broadcast with readfirstlane (all lanes active).
 __device__ __forceinline__ double wave_max(double v) {
     const int lane = threadIdx.x & (MPQP_WAVE - 1);
@@ -416,7 +417,7 @@ __device__ __forceinline__ double tree_sum(double (&v)[MPQP_MAXS], int n, int la
 // lanes.  key < 0 marks "no candidate".
 __device__ __forceinline__ void lex_min(double &v, int &key, int &aux) {
     // order-free (a total order on (value, key) over valid keys): lane
-    // shifts into lane 0 (DPP / swizzle / permlane, no LDS round trip), then
+    // shifts into lane 0 (DPP / permlane, no LDS round trip), then
     // a broadcast
     const int lane = threadIdx.x & (MPQP_WAVE - 1);
 #define MPQP_LEX_STEP(I)                                                                         \

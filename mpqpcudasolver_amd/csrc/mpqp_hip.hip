@@ -41,6 +41,7 @@
 
 #include "../../include/mpqp_hip.h"
 #include "kernels.hpp"
+#include "opt_fn.hpp"
 #include "regions.hpp"
 
 static_assert(sizeof(DevRecord) == sizeof(MpqpRecord), "record layout");
@@ -58,6 +59,10 @@ static __device__ __align__(256) unsigned char scratch[MPQP_SCRATCH_BYTES];
 
 namespace {
 
+struct HipError {
+    std::string msg;
+};
+
 // Threads per feasibility LP when the autotuner does not choose: about 16
 // tableau entries per thread, one wave for a small LP, at most 512.
 int feas_threads_for(int M1, int K1) {
@@ -68,31 +73,24 @@ int feas_threads_for(int M1, int K1) {
 }
 constexpr int OPT_NT = 512;
 
-template <int NT, bool FP32, bool GT>
-const void *opt_fn_nt(int S) {
-#define MPQP_OPT_FN(s)                                                       \
-    (FP32 ? reinterpret_cast<const void *>(&opt_kernel32<NT, s, GT>)         \
-          : reinterpret_cast<const void *>(&opt_kernel64<NT, s, GT>))
-    switch (S) {
-    case 1: return MPQP_OPT_FN(1);
-    case 2: return MPQP_OPT_FN(2);
-    case 3: return MPQP_OPT_FN(3);
-    case 4: return MPQP_OPT_FN(4);
-    case 6: return MPQP_OPT_FN(6);
-    default: return MPQP_OPT_FN(8);
-    }
-#undef MPQP_OPT_FN
-}
-
 // The optimality kernel for a precision (FP32 pivots with certification, or
 // FP64), workgroup size, reduction slot count and tableau placement (LDS,
 // or split between LDS and global memory when it does not fit: 512 or 1024
 // threads).
 const void *opt_fn(bool fp32, int nt, int S, bool gt) {
-    if (gt && nt == 1024) return fp32 ? opt_fn_nt<1024, true, true>(S) : opt_fn_nt<1024, false, true>(S);
-    if (gt) return fp32 ? opt_fn_nt<512, true, true>(S) : opt_fn_nt<512, false, true>(S);
-    if (fp32) return nt == 256 ? opt_fn_nt<256, true, false>(S) : opt_fn_nt<512, true, false>(S);
-    return nt == 256 ? opt_fn_nt<256, false, false>(S) : opt_fn_nt<512, false, false>(S);
+#define MPQP_TRY(part, nt_, fp32_, gt_) \
+    if (nt == nt_ && fp32 == fp32_ && gt == gt_) return opt_fn_part##part(S);
+    MPQP_OPT_PARTS(MPQP_TRY)
+#undef MPQP_TRY
+    throw HipError{"no optimality kernel for this shape"};
+}
+
+// The register-tableau kernels, smallest first.
+const std::vector<RegConfig> &reg_configs() {
+#define MPQP_CFG(part, ...) reg_config_part##part(),
+    static const std::vector<RegConfig> c = {MPQP_REG_PARTS(MPQP_CFG)};
+#undef MPQP_CFG
+    return c;
 }
 
 // The feasibility kernel at a workgroup size the autotuner may choose.
@@ -125,10 +123,6 @@ __global__ void fill_i32(int *p, int n, int v) {
     if (i < n) p[i] = v;
 }
 
-struct HipError {
-    std::string msg;
-};
-
 // Rows of an optimality tableau too large for LDS that stay in LDS (even,
 // so that a state copy splits on a whole 16-byte vector), next to its cost
 // row, the bookkeeping and the deferred updates of the other rows (whose
@@ -158,7 +152,7 @@ struct BufView {
 // Names of the device buffers of a call: per call (level -1), or per level
 // of the depth-first traversal.
 enum Kind {
-    K_A1, K_XB1, K_A2, K_XB2, K_AMAT, K_GW, K_G, K_SPI, K_SPD, K_ROOTG, K_ROOT, K_ROOTI, K_CTR, K_GT64, K_GT32,
+    K_A1, K_XB1, K_A2, K_XB2, K_AMAT, K_GW, K_G, K_SPI, K_SPD, K_ROOTG, K_ROOT, K_ROOT32, K_ROOTI, K_CTR, K_GT64, K_GT32,
     K_SUM, K_COLQ,
     R_IN, R_SETS, R_OUT, R_INFO,
     L_SETS, L_PAR, L_P1PAR, L_REC, L_FLAG, L_POS, L_LIST, L_FBL, L_CNT, L_OFF, L_FS, L_OS, L_FB, L_B1, L_B2,
@@ -520,6 +514,8 @@ struct Run {
     int w32 = 2, w64 = 1;                // workgroups per CU a split tableau is sized for
     size_t gtab64_max = 0, gtab32_max = 0;  // global rows of the largest variant
     const void *fn64 = nullptr, *fn32 = nullptr;
+    const RegConfig *reg32 = nullptr;  // FP32 tableau in registers (null: LDS, or split)
+    int nt32 = OPT_NT, np32 = 1;       // threads of the FP32 kernel; its stage passes
     bool tune_pending = false;
     std::vector<int> tkey;
     double *G = nullptr;
@@ -675,9 +671,12 @@ struct Run {
         ra.root_nonb = ra.root_basis + M2;
         ra.root_ok = ra.root_nonb + K2;
         ra.root = droot.as<double>();
+        if (o.precision == MPQP_MIXED)
+            ra.root32 = A.get(K_ROOT32, -1, (size_t)opt_state_bytes<float>(M2, K2)).as<float>();
         hipLaunchKernelGGL(root_kernel<256>, dim3(1), dim3(256), (size_t)(M2 + 1) * 8 + (size_t)M2 * 4, st, ra);
         HIP_OK(hipGetLastError());
         P.root = ra.root;
+        P.root32 = ra.root32;
         P.root_basis = ra.root_basis;
         P.root_nonb = ra.root_nonb;
         P.root_ok = ra.root_ok;
@@ -723,6 +722,8 @@ struct Run {
         const long long budget = C.lds_limit - 512;
         gt64 = opt_lds_bytes_t<double>(M2, K2, N2, false, M2 + 1) > budget;
         gt32 = opt_lds_bytes_t<float>(M2, K2, N2, true, M2 + 1) > budget;
+        select_reg();
+        if (reg32) gt32 = false;
         S = red_slots(std::max(M2, N2 - in.n_eqs));
         feas_nt = feas_threads_for(M1, K1);
         // 1024 threads only where every optimality kernel of the call splits its tableau
@@ -764,6 +765,7 @@ struct Run {
     // tableau; for a split one also the LDS share of its rows
     std::vector<std::vector<int>> split_variants() const {
         const bool tuned_split = o.precision == MPQP_MIXED ? gt32 : gt64;
+        if (reg32) return {{512, w32, w64}};  // one shape; only the FP64 re-solve takes the size
         if (!tuned_split) {
             // an LDS tableau; the FP64 re-solve of a mixed run may split its own
             if (o.precision == MPQP_MIXED && gt64) return {{512, w32, w64}};
@@ -773,6 +775,32 @@ struct Run {
         return {{512, 2, 2}, {512, 1, 1}, {1024, 1, 1}};
     }
 
+    // The FP32 tableau in registers when a configuration holds it, except one
+    // of a single wave's rows, which has little to pivot in parallel: the LDS
+    // kernel took 0.39 ms for 1,249 LPs of 40 x 24 against 0.45, and 0.95
+    // against 0.82 for 12,464 LPs of 63 x 37.  A caller that names workgroup
+    // sizes gets the LDS and split kernels they are for.
+    void select_reg() {
+        reg32 = nullptr;
+        if (o.precision != MPQP_MIXED || o.opt_threads != 0 || o.split_wgs != 0) return;
+        if (in.M2 <= 44) return;
+        // its use counts share a word with a position
+        if (o.max_iter_phase1 >= 1 << 20 || o.max_iter_phase2 >= 1 << 20) return;
+        for (const RegConfig &c : reg_configs()) {
+            if (in.M2 > c.rows() || K2 > c.columns() || P.Nn > 64 * c.sn) continue;
+            // as few passes through the LDS stage as its share of a CU allows
+            for (int np = 1; np <= c.nw; np *= 2) {
+                const long long b = reg_lds_bytes(c.nw, c.rw, c.cs, in.M2, K2, in.N2, true, np);
+                if (b <= C.lds_limit / c.wgs() - 1024) {
+                    reg32 = &c;
+                    np32 = np;
+                    lds32 = b;
+                    return;
+                }
+            }
+        }
+    }
+
     void select_variant(int nt, int ws32, int ws64) {
         const int M2 = in.M2, N2 = in.N2;
         w32 = ws32;
@@ -780,7 +808,7 @@ struct Run {
         R64 = gt64 ? split_rows_for<double>(M2, K2, N2, false, C.lds_limit / w64 - 512) : M2;
         R32 = gt32 ? split_rows_for<float>(M2, K2, N2, true, C.lds_limit / w32 - 512) : M2;
         lds64 = opt_lds_bytes_t<double>(M2, K2, N2, false, gt64 ? R64 + 1 : M2 + 1);
-        lds32 = opt_lds_bytes_t<float>(M2, K2, N2, true, gt32 ? R32 + 1 : M2 + 1);
+        if (!reg32) lds32 = opt_lds_bytes_t<float>(M2, K2, N2, true, gt32 ? R32 + 1 : M2 + 1);
         select_opt(nt);
     }
 
@@ -799,14 +827,16 @@ struct Run {
         if (nt == 1024 && !all_split) nt = 512;
         opt_nt = nt;
         fn64 = opt_fn(false, opt_nt, S, gt64);
-        fn32 = opt_fn(true, opt_nt, S, gt32);
+        fn32 = !mx ? nullptr : (reg32 ? reg32->fn : opt_fn(true, opt_nt, S, gt32));
+        nt32 = reg32 ? reg32->threads() : opt_nt;
         cap64 = capacity(fn64, opt_nt, lds64);
-        cap32 = o.precision == MPQP_MIXED ? capacity(fn32, opt_nt, lds32) : 0;
+        cap32 = o.precision == MPQP_MIXED ? capacity(fn32, nt32, lds32) : 0;
     }
 
     void launch_opt(const void *fn, int grid, long long lds, OptArgs &oa) {
         void *args[] = {&oa};
-        HIP_OK(hipLaunchKernel(fn, dim3(grid), dim3(opt_nt), args, (size_t)lds, st));
+        oa.stage_passes = np32;
+        HIP_OK(hipLaunchKernel(fn, dim3(grid), dim3(fn == fn32 ? nt32 : opt_nt), args, (size_t)lds, st));
     }
 
     // device bytes a candidate of `level` needs in its chunk
@@ -1044,7 +1074,9 @@ struct Run {
                 // sample of the list (counters reset per trial)
                 float best = INFINITY;
                 std::vector<int> best_v{opt_nt, w32, w64};
-                for (const auto &v : split_variants()) {
+                const std::vector<std::vector<int>> variants = split_variants();
+                if (variants.size() == 1) best_v = variants[0];
+                else for (const auto &v : variants) {
                     select_variant(v[0], v[1], v[2]);
                     hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, dctr.as<int>(), 4, 0);
                     HIP_OK(hipGetLastError());

@@ -1,0 +1,60 @@
+// opt_fn.hip — one group of optimality kernels (see opt_fn.hpp).
+#include <hip/hip_runtime.h>
+
+#include "kernels.hpp"
+#include "opt_fn.hpp"
+
+#define MPQP_CAT_(a, b) a##b
+#define MPQP_CAT(a, b) MPQP_CAT_(a, b)
+
+#if MPQP_PART >= 8
+
+template <int P>
+struct Part;
+#define MPQP_PICK(part, nw_, rw_, cs_, ex_, sn_, eu_)                                                  \
+    template <>                                                                                        \
+    struct Part<part> {                                                                                \
+        static constexpr int nw = nw_, rw = rw_, cs = cs_, ex = ex_, sn = sn_, eu = eu_;               \
+    };
+MPQP_REG_PARTS(MPQP_PICK)
+
+RegConfig MPQP_CAT(reg_config_part, MPQP_PART)() {
+    typedef Part<MPQP_PART> P;
+    return RegConfig{P::nw, P::rw, P::cs, P::ex, P::sn, P::eu,
+                     reinterpret_cast<const void *>(&reg_kernel32<P::nw, P::rw, P::cs, P::ex, P::sn, P::eu>)};
+}
+
+#else
+
+template <int NT, bool FP32, bool GT>
+static const void *opt_fn_nt(int S) {
+#define MPQP_OPT_FN(s)                                                       \
+    (FP32 ? reinterpret_cast<const void *>(&opt_kernel32<NT, s, GT>)         \
+          : reinterpret_cast<const void *>(&opt_kernel64<NT, s, GT>))
+    switch (S) {
+    case 1: return MPQP_OPT_FN(1);
+    case 2: return MPQP_OPT_FN(2);
+    case 3: return MPQP_OPT_FN(3);
+    case 4: return MPQP_OPT_FN(4);
+    case 6: return MPQP_OPT_FN(6);
+    default: return MPQP_OPT_FN(8);
+    }
+#undef MPQP_OPT_FN
+}
+
+template <int P>
+struct Part;
+#define MPQP_PICK(part, nt, fp32, gt)                     \
+    template <>                                           \
+    struct Part<part> {                                   \
+        static constexpr int threads = nt;                \
+        static constexpr bool single = fp32, split = gt;  \
+    };
+MPQP_OPT_PARTS(MPQP_PICK)
+
+const void *MPQP_CAT(opt_fn_part, MPQP_PART)(int S) {
+    typedef Part<MPQP_PART> P;
+    return opt_fn_nt<P::threads, P::single, P::split>(S);
+}
+
+#endif

@@ -1,0 +1,46 @@
+// opt_fn.hpp — the optimality kernels by shape.  Their instantiations are most
+// of the build, so each group is a translation unit of its own (opt_fn.hip
+// compiled with MPQP_PART = its number), compiled side by side.
+#pragma once
+
+// Groups: threads per workgroup, FP32 pivots with certification or FP64, the
+// tableau in LDS or split between LDS and global memory; S the slots of a
+// reduction.
+#define MPQP_OPT_PARTS(X)          \
+    X(0, 256, true, false)         \
+    X(1, 512, true, false)         \
+    X(2, 512, true, true)          \
+    X(3, 1024, true, true)         \
+    X(4, 256, false, false)        \
+    X(5, 512, false, false)        \
+    X(6, 512, false, true)         \
+    X(7, 1024, false, true)
+
+#define MPQP_DECL(part, nt, fp32, gt) __attribute__((visibility("hidden"))) const void *opt_fn_part##part(int S);
+MPQP_OPT_PARTS(MPQP_DECL)
+#undef MPQP_DECL
+
+// Kernels with the FP32 tableau in registers (parts 8 ..): waves per
+// workgroup, rows per wave, column slots, extra columns, reduction slots over
+// the Nn variables, waves per SIMD of the register budget (512 / that many
+// registers a lane).
+#define MPQP_REG_PARTS(X)          \
+    X(8, 2, 44, 1, 4, 3, 4)        \
+    X(9, 2, 64, 1, 8, 4, 3)        \
+    X(10, 4, 44, 2, 0, 4, 3)       \
+    X(11, 4, 64, 2, 8, 6, 2)       \
+    X(12, 8, 44, 3, 4, 6, 2)       \
+    X(13, 8, 44, 4, 0, 6, 2)
+
+struct RegConfig {
+    int nw, rw, cs, ex, sn, eu;
+    const void *fn;
+    int rows() const { return nw * rw; }
+    int columns() const { return 64 * cs + ex; }
+    int threads() const { return nw * 64; }
+    int wgs() const { return eu * 4 / nw; }  // workgroups per CU of the budget
+};
+
+#define MPQP_DECL(part, ...) __attribute__((visibility("hidden"))) RegConfig reg_config_part##part();
+MPQP_REG_PARTS(MPQP_DECL)
+#undef MPQP_DECL

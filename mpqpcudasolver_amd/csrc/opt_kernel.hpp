@@ -132,9 +132,12 @@ struct OptLds {
     // SPLIT: deferred updates of the global rows (opt_lazy_pivot)
     Real *ep, *ef, *gx, *gp, *prow;
     int *gver, *eq;
+    int T_rhs, T_cost;  // the rhs column and the cost row
     // SPLIT: rows [R, M) of the tableau at gT (global memory), the rest in LDS
     __device__ void carve(unsigned char *smem, int M, int K, int N2, bool cert, Real *gT, int R) {
         ld = opt_ld<Real>(K);
+        T_rhs = K;
+        T_cost = M;
         Real *lo = reinterpret_cast<Real *>(smem);
         const int trows = SPLIT ? R + 1 : M + 1;
         T = TabRef<Real, SPLIT>{lo, gT, R, M, ld};
@@ -173,6 +176,9 @@ struct OptLds {
             eq = gver + G;
         }
     }
+    // rhs of a row, cost of a slot (certification)
+    __device__ __forceinline__ Real rhs_of(int i) const { return T.row(i)[T_rhs]; }
+    __device__ __forceinline__ Real cost_of(int k) const { return T.row(T_cost)[k]; }
     // rhs / perturbation entry of row i < M inside the phase-1 and phase-2
     // loops (the global rows' mirrors when the tableau is split)
     __device__ __forceinline__ const Real *rhs_at(int i, int RHS) const {
@@ -1373,13 +1379,53 @@ __device__ __forceinline__ double col_resid(const DevProb &P, const SBits &sb, i
     return acc;
 }
 
+// One correction of cert_primal: x += B32^-1 r; ends with a barrier.
+template <int NT, typename LT>
+__device__ __forceinline__ void cert_primal_corr(LT &L, const DevProb &P, int ne) {
+    const int M = P.M2, e0 = P.N2 - M;
+    double *x = L.cx, *r = L.cr;
+    for (int q = threadIdx.x; q < M * MPQP_GB; q += NT) {
+        // (B32^-1 r)_i: the unit term of a basic e at position i, then
+        // the nonbasic e-columns, rho ascending
+        const int i = q / MPQP_GB, g = q % MPQP_GB;
+        const float *Ti = L.T.row(i);
+        const int bv = L.basis[i];
+        double acc = (g == 0 && bv >= e0) ? r[bv - e0] : 0.0;
+        int k = g;
+        for (; k + (MPQP_CBL - 1) * MPQP_GB < ne; k += MPQP_CBL * MPQP_GB) {
+            int rk[MPQP_CBL], sk[MPQP_CBL];
+            double rv[MPQP_CBL], tv[MPQP_CBL];
+#pragma unroll
+            for (int u = 0; u < MPQP_CBL; ++u) {
+                rk[u] = L.elr[k + u * MPQP_GB];
+                sk[u] = L.els[k + u * MPQP_GB];
+            }
+#pragma unroll
+            for (int u = 0; u < MPQP_CBL; ++u) {
+                rv[u] = r[rk[u]];
+                tv[u] = (double)Ti[sk[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < MPQP_CBL; ++u) acc = fma(rv[u], tv[u], acc);
+        }
+        for (; k < ne; k += MPQP_GB) acc = fma(r[L.elr[k]], (double)Ti[L.els[k]], acc);
+        acc = team_add<MPQP_GB>(acc);
+        if (g == 0) {
+            const double xn = x[i] + acc;
+            x[i] = xn;
+            L.xv[bv] = xn == xn ? xn : INFINITY;
+        }
+    }
+    __syncthreads();
+}
+
 // x (LDS, by position; L.xv by variable, NaN when nonbasic, a NaN value of
 // a basic variable stored as +inf) := refined solution of B x = xb2; 1 once
 // max|xb2 - B x| <= cert_ptol.  *ne_out: the number of nonbasic e-variables.
-template <int NT, int S, typename LT>
+template <int NT, int S, typename LT, typename CorrF>
 __device__ __forceinline__ int cert_primal(LT &L, const DevProb &P, const unsigned *inS, double *red,
-                                           OptShared &sh, const int *Sset, int k, int *ne_out) {
-    const int M = P.M2, N2 = P.N2, RHS = P.K2, e0 = P.N2 - M;
+                                           OptShared &sh, const int *Sset, int k, int *ne_out, CorrF corr) {
+    const int M = P.M2, N2 = P.N2;
     double *x = L.cx, *r = L.cr;
     const int ne = elist_build<S>(L, P, sh);
     *ne_out = ne;
@@ -1389,7 +1435,7 @@ __device__ __forceinline__ int cert_primal(LT &L, const DevProb &P, const unsign
     const int xb0 = M - n_c - P.n_x, xb1 = M - n_c;
     for (int v = threadIdx.x; v < N2; v += NT) {
         const int w = L.where[v];
-        const double xw = w >= 0 ? (double)L.T.row(w)[RHS] : 0.0;
+        const double xw = w >= 0 ? (double)L.rhs_of(w) : 0.0;
         L.xv[v] = w >= 0 ? (xw == xw ? xw : INFINITY) : __builtin_nan("");
         if (w >= 0) x[w] = xw;
     }
@@ -1461,50 +1507,53 @@ __device__ __forceinline__ int cert_primal(LT &L, const DevProb &P, const unsign
         OPT_PROF(sh, 8);
         if (rmax <= P.cert_ptol) return 1;
         if (it == MPQP_CERT_STEPS) return 0;
-        for (int q = threadIdx.x; q < M * MPQP_GB; q += NT) {
-            // (B32^-1 r)_i: the unit term of a basic e at position i, then
-            // the nonbasic e-columns, rho ascending
-            const int i = q / MPQP_GB, g = q % MPQP_GB;
-            const float *Ti = L.T.row(i);
-            const int bv = L.basis[i];
-            double acc = (g == 0 && bv >= e0) ? r[bv - e0] : 0.0;
-            int k = g;
-            for (; k + (MPQP_CBL - 1) * MPQP_GB < ne; k += MPQP_CBL * MPQP_GB) {
-                int rk[MPQP_CBL], sk[MPQP_CBL];
-                double rv[MPQP_CBL], tv[MPQP_CBL];
-#pragma unroll
-                for (int u = 0; u < MPQP_CBL; ++u) {
-                    rk[u] = L.elr[k + u * MPQP_GB];
-                    sk[u] = L.els[k + u * MPQP_GB];
-                }
-#pragma unroll
-                for (int u = 0; u < MPQP_CBL; ++u) {
-                    rv[u] = r[rk[u]];
-                    tv[u] = (double)Ti[sk[u]];
-                }
-#pragma unroll
-                for (int u = 0; u < MPQP_CBL; ++u) acc = fma(rv[u], tv[u], acc);
-            }
-            for (; k < ne; k += MPQP_GB) acc = fma(r[L.elr[k]], (double)Ti[L.els[k]], acc);
-            acc = team_add<MPQP_GB>(acc);
-            if (g == 0) {
-                const double xn = x[i] + acc;
-                x[i] = xn;
-                L.xv[bv] = xn == xn ? xn : INFINITY;
-            }
-        }
-        __syncthreads();
+        corr(ne);
         OPT_PROF(sh, 9);
     }
+}
+
+// One correction of cert_dual: y += B32^-T r; ends with a barrier.
+template <int NT, typename LT>
+__device__ __forceinline__ void cert_dual_corr(const LT &L, const DevProb &P, int ne) {
+    const int M = P.M2, e0 = P.N2 - M;
+    double *y = L.cx, *r = L.cr;
+    for (int q = threadIdx.x; q < ne * MPQP_GT; q += NT) {
+        // (B32^-T r)_rho of a nonbasic e_rho: its tableau column,
+        // positions ascending
+        const int k = q / MPQP_GT, g = q % MPQP_GT;
+        const int rho = L.elr[k];
+        const int col = L.els[k];
+        double acc = 0.0;
+        int i = g;
+        for (; i + (MPQP_CBL - 1) * MPQP_GT < M; i += MPQP_CBL * MPQP_GT) {
+            double rv[MPQP_CBL], tv[MPQP_CBL];
+#pragma unroll
+            for (int u = 0; u < MPQP_CBL; ++u) {
+                rv[u] = r[i + u * MPQP_GT];
+                tv[u] = (double)L.T.row(i + u * MPQP_GT)[col];
+            }
+#pragma unroll
+            for (int u = 0; u < MPQP_CBL; ++u) acc = fma(rv[u], tv[u], acc);
+        }
+        for (; i < M; i += MPQP_GT) acc = fma(r[i], (double)L.T.row(i)[col], acc);
+        acc = team_add<MPQP_GT>(acc);
+        if (g == 0) y[rho] = y[rho] + acc;
+    }
+    for (int i = threadIdx.x; i < M; i += NT) {
+        // basic e_rho at position i: unit column
+        const int bv = L.basis[i];
+        if (bv >= e0) y[bv - e0] = y[bv - e0] + r[i];
+    }
+    __syncthreads();
 }
 
 // y (in L.cx) := refined solution of B^T y = c_B, c = cost(v), starting from
 // the FP32 cost row (y_rho = c(e_rho) - d(e_rho), d = 0 for a basic e: the
 // e-columns of A2 are the identity); 1 once max|c_B - B^T y| <= 2e-12.
 // ne: the e-list of cert_primal (same basis).
-template <int NT, int S, typename LT, typename CostF>
+template <int NT, int S, typename LT, typename CostF, typename CorrF>
 __device__ __forceinline__ int cert_dual(const LT &L, const DevProb &P, const unsigned *inS, double *red,
-                                         CostF cost, OptShared &sh, int ne) {
+                                         CostF cost, OptShared &sh, int ne, CorrF corr) {
     const int M = P.M2, e0 = P.N2 - M;
     double *y = L.cx, *r = L.cr;
     SBits sb;
@@ -1512,7 +1561,7 @@ __device__ __forceinline__ int cert_dual(const LT &L, const DevProb &P, const un
     for (int rho = threadIdx.x; rho < M; rho += NT) {
         const int w = L.where[e0 + rho];
         const double c = cost(e0 + rho);
-        y[rho] = w >= 0 ? c : c - (double)L.T.row(M)[-w - 1];
+        y[rho] = w >= 0 ? c : c - (double)L.cost_of(-w - 1);
     }
     int *ord = L.bcnt;  // positions, long columns first (bcnt is free after phase 1)
     order_flag_first<S>(ord, M, [&](int i) { return long_col(P, L.basis[i]); });
@@ -1531,34 +1580,7 @@ __device__ __forceinline__ int cert_dual(const LT &L, const DevProb &P, const un
         OPT_PROF(sh, 12);
         if (rmax <= 2e-12) return 1;
         if (it == MPQP_CERT_STEPS) return 0;
-        for (int q = threadIdx.x; q < ne * MPQP_GT; q += NT) {
-            // (B32^-T r)_rho of a nonbasic e_rho: its tableau column,
-            // positions ascending
-            const int k = q / MPQP_GT, g = q % MPQP_GT;
-            const int rho = L.elr[k];
-            const int col = L.els[k];
-            double acc = 0.0;
-            int i = g;
-            for (; i + (MPQP_CBL - 1) * MPQP_GT < M; i += MPQP_CBL * MPQP_GT) {
-                double rv[MPQP_CBL], tv[MPQP_CBL];
-#pragma unroll
-                for (int u = 0; u < MPQP_CBL; ++u) {
-                    rv[u] = r[i + u * MPQP_GT];
-                    tv[u] = (double)L.T.row(i + u * MPQP_GT)[col];
-                }
-#pragma unroll
-                for (int u = 0; u < MPQP_CBL; ++u) acc = fma(rv[u], tv[u], acc);
-            }
-            for (; i < M; i += MPQP_GT) acc = fma(r[i], (double)L.T.row(i)[col], acc);
-            acc = team_add<MPQP_GT>(acc);
-            if (g == 0) y[rho] = y[rho] + acc;
-        }
-        for (int i = threadIdx.x; i < M; i += NT) {
-            // basic e_rho at position i: unit column
-            const int bv = L.basis[i];
-            if (bv >= e0) y[bv - e0] = y[bv - e0] + r[i];
-        }
-        __syncthreads();
+        corr(ne);
         OPT_PROF(sh, 13);
     }
 }
@@ -1635,6 +1657,80 @@ __device__ __forceinline__ double cert_xmin(const LT &L, int M, double *red) {
     double mn = INFINITY;
     for (int i = threadIdx.x; i < M; i += NT) mn = fmin(mn, L.cx[i]);
     return -block_max<NT>(-mn, red);
+}
+
+// FP64 certification of phase 1 (1: certified, verdict and z1 set).  With an
+// artificial basic: the dual first (B^T y = c_B refined, nonnegative reduced
+// phase-1 costs); a dual objective xb2^T y >= dual_feas_tol bounds the
+// phase-1 optimum from below and certifies the infeasible verdict alone.
+// Otherwise (no artificial basic, or a smaller bound) also the primal:
+// x_B >= dual_stop_tol, z1 = the artificials' sum of the refined x.
+template <int NT, int S, typename LT, typename PF, typename DF>
+__device__ __forceinline__ int cert_phase1(LT &L, const DevProb &P, const DevOpts &O, const unsigned *inS, double *red,
+                                           OptShared &sh, const int *Sset, int k, P1Result &p1, PF pcorr, DF dcorr) {
+    const int M = P.M2, Nn = P.Nn;
+    auto cb1 = [Nn](int v) { return v >= Nn ? 1.0 : 0.0; };
+    int ok = p1.status == ST_OPTIMAL, ne = 0, done = 0;
+    if (ok) {
+        rows_where<S>(L.rows, M, sh, [&](int i) { return L.basis[i] >= Nn; });
+        if (sh.nrows > 0) {
+            ne = elist_build<S>(L, P, sh);
+            ok = cert_dual<NT, S>(L, P, inS, red, cb1, sh, ne, dcorr);
+            if (ok) ok = min_red_cost<NT, S>(L, P, inS, red, [](int) { return true; }, cb1) >= -O.certify_tol;
+            OPT_PROF(sh, 14);
+            if (ok) {
+                const double zd = cert_zdual<NT, S>(L, P, red);
+                if (zd >= O.dual_feas_tol) {
+                    p1.z1 = zd;
+                    p1.kkt = 0;
+                    done = 1;
+                }
+            }
+        }
+    }
+    if (ok && !done) {
+        ok = cert_primal<NT, S>(L, P, inS, red, sh, Sset, k, &ne, pcorr);
+        if (ok) ok = cert_xmin<NT>(L, M, red) >= O.dual_stop_tol;
+        if (ok) {
+            p1.z1 = cert_z<NT, S>(L, P, red, cb1);
+            p1.kkt = (p1.z1 > -O.dual_feas_tol && p1.z1 < O.dual_feas_tol) ? 1 : 0;
+        }
+        OPT_PROF(sh, 10);
+    }
+    return ok;
+}
+
+// FP64 certification of phase 2: x_B >= -certify_tol and nonnegative reduced
+// costs of the first N_ variables.
+template <int NT, int S, typename LT, typename PF, typename DF>
+__device__ __forceinline__ int cert_phase2(LT &L, const DevProb &P, const DevOpts &O, const unsigned *inS, double *red,
+                                           OptShared &sh, const int *Sset, int k, P2Result &p2, PF pcorr, DF dcorr) {
+    const int M = P.M2, EPS = P.n_x + P.n_t + P.n_c, Nn = P.Nn;
+    auto cb2 = [EPS](int v) { return v == EPS ? -1.0 : 0.0; };
+    int ok = p2.status == ST_OPTIMAL, ne = 0;
+    if (ok) ok = cert_primal<NT, S>(L, P, inS, red, sh, Sset, k, &ne, pcorr);
+    if (ok) ok = cert_xmin<NT>(L, M, red) >= -O.certify_tol;
+    if (ok) {
+        p2.z2 = cert_z<NT, S>(L, P, red, cb2);
+        p2.final_set = -p2.z2 > O.final_tol ? 1 : 0;
+        ok = cert_dual<NT, S>(L, P, inS, red, cb2, sh, ne, dcorr);
+    }
+    if (ok) ok = min_red_cost<NT, S>(L, P, inS, red, [Nn](int v) { return v < Nn; }, cb2) >= -O.certify_tol;
+    return ok;
+}
+
+// the optimality LP's part of a candidate's record (one thread)
+__device__ __forceinline__ void opt_record(DevRecord &R, const P1Result &p1, const P2Result &p2, int warm, int clean) {
+    R.p1_status = p1.status;
+    R.p1_iters = p1.iters;
+    R.kkt_feasible = p1.kkt;
+    R.p1_warm = warm;
+    R.z1 = p1.z1;
+    R.p1_clean = p1.kkt ? clean : 0;
+    R.p2_status = p2.status;
+    R.p2_iters = p2.iters;
+    R.z2 = p2.z2;
+    R.final_set = p2.final_set;
 }
 
 // ---------------------------------------------------------------------
@@ -1758,48 +1854,13 @@ __device__ __forceinline__ void opt_body(const OptArgs &a) {
             }
             fail = true;
         }
+        auto pcorr = [&](auto ne) { cert_primal_corr<NT>(L, P, ne); };
+        auto dcorr = [&](auto ne) { cert_dual_corr<NT>(L, P, ne); };
+        (void)pcorr;
+        (void)dcorr;
         if (!fail) {
             p1 = opt_phase1<Real, NT, S>(L, P, O, tl, sh);
-            if constexpr (MIXED) {
-                // FP64 certification of phase 1.  With an artificial basic:
-                // the dual first (B^T y = c_B refined, nonnegative reduced
-                // phase-1 costs); a dual objective xb2^T y >= dual_feas_tol
-                // bounds the phase-1 optimum from below and certifies the
-                // infeasible verdict alone.  Otherwise (no artificial basic,
-                // or a smaller bound) also the primal: x_B >= dual_stop_tol,
-                // z1 = the artificials' sum of the refined x.
-                const int Nn = P.Nn;
-                auto cb1 = [Nn](int v) { return v >= Nn ? 1.0 : 0.0; };
-                int ok = p1.status == ST_OPTIMAL, ne = 0, done = 0;
-                if (ok) {
-                    rows_where<S>(L.rows, M, sh, [&](int i) { return L.basis[i] >= Nn; });
-                    if (sh.nrows > 0) {
-                        ne = elist_build<S>(L, P, sh);
-                        ok = cert_dual<NT, S>(L, P, inS, red, cb1, sh, ne);
-                        if (ok)
-                            ok = min_red_cost<NT, S>(L, P, inS, red, [](int) { return true; }, cb1) >= -O.certify_tol;
-                        OPT_PROF(sh, 14);
-                        if (ok) {
-                            const double zd = cert_zdual<NT, S>(L, P, red);
-                            if (zd >= O.dual_feas_tol) {
-                                p1.z1 = zd;
-                                p1.kkt = 0;
-                                done = 1;
-                            }
-                        }
-                    }
-                }
-                if (ok && !done) {
-                    ok = cert_primal<NT, S>(L, P, inS, red, sh, Sset, k, &ne);
-                    if (ok) ok = cert_xmin<NT>(L, M, red) >= O.dual_stop_tol;
-                    if (ok) {
-                        p1.z1 = cert_z<NT, S>(L, P, red, cb1);
-                        p1.kkt = (p1.z1 > -O.dual_feas_tol && p1.z1 < O.dual_feas_tol) ? 1 : 0;
-                    }
-                    OPT_PROF(sh, 10);
-                }
-                fail = !ok;
-            }
+            if constexpr (MIXED) fail = !cert_phase1<NT, S>(L, P, O, inS, red, sh, Sset, k, p1, pcorr, dcorr);
             OPT_PROF(sh, 4);
         }
         if (!fail) {
@@ -1816,23 +1877,7 @@ __device__ __forceinline__ void opt_body(const OptArgs &a) {
                 OPT_PROF(sh, 5);
                 p2 = opt_phase2<Real, NT, S>(L, P, O, tl, sh);
                 OPT_PROF(sh, 6);
-                if constexpr (MIXED) {
-                    // FP64 certification of phase 2: x_B >= -certify_tol and
-                    // nonnegative reduced costs of the first N_ variables
-                    const int EPS = P.n_x + P.n_t + P.n_c, Nn = P.Nn;
-                    auto cb2 = [EPS](int v) { return v == EPS ? -1.0 : 0.0; };
-                    int ok = p2.status == ST_OPTIMAL, ne = 0;
-                    if (ok) ok = cert_primal<NT, S>(L, P, inS, red, sh, Sset, k, &ne);
-                    if (ok) ok = cert_xmin<NT>(L, M, red) >= -O.certify_tol;
-                    if (ok) {
-                        p2.z2 = cert_z<NT, S>(L, P, red, cb2);
-                        p2.final_set = -p2.z2 > O.final_tol ? 1 : 0;
-                        ok = cert_dual<NT, S>(L, P, inS, red, cb2, sh, ne);
-                    }
-                    if (ok)
-                        ok = min_red_cost<NT, S>(L, P, inS, red, [Nn](int v) { return v < Nn; }, cb2) >= -O.certify_tol;
-                    fail = !ok;
-                }
+                if constexpr (MIXED) fail = !cert_phase2<NT, S>(L, P, O, inS, red, sh, Sset, k, p2, pcorr, dcorr);
                 if (!fail && a.b2)
                     for (int i = tid; i < M; i += NT) a.b2[(long long)c * M + i] = L.basis[i];
             }
@@ -1847,18 +1892,7 @@ __device__ __forceinline__ void opt_body(const OptArgs &a) {
             }
             continue;
         }
-        if (tid == 0) {
-            R.p1_status = p1.status;
-            R.p1_iters = p1.iters;
-            R.kkt_feasible = p1.kkt;
-            R.p1_warm = warm;
-            R.z1 = p1.z1;
-            R.p1_clean = p1.kkt ? clean : 0;
-            R.p2_status = p2.status;
-            R.p2_iters = p2.iters;
-            R.z2 = p2.z2;
-            R.final_set = p2.final_set;
-        }
+        if (tid == 0) opt_record(R, p1, p2, warm, clean);
         OPT_PROF(sh, 7);
     }
 }

@@ -71,7 +71,7 @@ __host__ __device__ inline long long region_lds_bytes(int n_c, int n_t, int n_cp
 // over Kd in steps of 4 (operands outside the matrices read as 0).  Lane l
 // supplies A[i0 + l % 16][k + l / 16] and B[k + l / 16][j0 + l % 16] and
 // receives C[i0 + 4 r + l / 16][j0 + l % 16] in result register r.
-__global__ __launch_bounds__(64) void gemm_f64_mfma(const double *A, int lda, const double *B, int ldb, double *C,
+static __global__ __launch_bounds__(64) void gemm_f64_mfma(const double *A, int lda, const double *B, int ldb, double *C,
                                                     int ldc, int M, int N, int Kd) {
     typedef double v4d __attribute__((ext_vector_type(4)));
     const int tn = (N + 15) / 16;
