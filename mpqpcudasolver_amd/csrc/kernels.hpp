@@ -316,9 +316,21 @@ static __global__ void gather_rows_nx(const int *sets, const int *idx, int cnt, 
 // matrix cores.  licq_screen then factors G_SS (rows of S ascending) per
 // candidate.
 // ---------------------------------------------------------------------
+// The matrix is worked on in LDS when it fits there (in_lds; colq then
+// follows it): one workgroup's pivots wait on each access, and global memory
+// made them 9 us each at n_x = 60, ncols = 180 (0.55 ms; 0.12 ms in LDS).
 template <int NT>
-__global__ __launch_bounds__(NT) void gram_solve(double *W, int n_x, int ld, int ncols, double *colq) {
-    for (int i = 0; i < n_x; ++i) pivot_team<NT, double>(W, ld, n_x, ncols, i, i, colq);
+__global__ __launch_bounds__(NT) void gram_solve(double *W, int n_x, int ld, int ncols, double *colq, int in_lds) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    if (!in_lds) {
+        for (int i = 0; i < n_x; ++i) pivot_team<NT, double>(W, ld, n_x, ncols, i, i, colq);
+        return;
+    }
+    double *T = reinterpret_cast<double *>(smem);
+    for (int e = threadIdx.x; e < n_x * ld; e += NT) T[e] = W[e];
+    __syncthreads();
+    for (int i = 0; i < n_x; ++i) pivot_team<NT, double>(T, ld, n_x, ncols, i, i, T + n_x * ld);
+    for (int e = threadIdx.x; e < n_x * ld; e += NT) W[e] = T[e];
 }
 
 // G (n_c x n_c, row-major) = A (n_c x n_x, row-major) x Y (n_x x n_c, rows
@@ -484,7 +496,9 @@ struct P2Pred {  // min_idx_kernel_optimal, batched_simplex.cu:343-344
 struct RootArgs {
     DevProb P;
     DevOpts O;
-    double *G;        // M2 x (K2+2) scratch
+    double *G;        // M2 x (K2+2) scratch (root_w: by columns)
+    double *F, *p;    // n_x factor columns of M2, n_x pivots
+    int *prow, *pos;  // n_x pivot rows; the position of each row
     int *rowvar;      // M2
     int *slotvar;     // K2
     int *rowof;       // N2
@@ -495,6 +509,223 @@ struct RootArgs {
     int *root_nonb;   // K2
     int *root_ok;
 };
+
+// The root by columns.  The pivots are known in advance but for the rows of
+// the x pivots, so a column can go through all of them by itself, in one
+// wave's registers (lane = row), given each pivot's factor column:
+//   root_w  the n_c pivots (row of w_j, column w_j): their factor columns are
+//           the columns w_j of A2 as they stand, since no other w pivot's row
+//           has an entry there (the host has checked that this block of A2 is
+//           diagonal with usable entries);
+//   root_x  the n_x pivots on the columns x_i alone, one workgroup in LDS:
+//           the pivot rows and the factor columns;
+//   root_y  those pivots on every column, and the root's layout.
+// Every entry goes through pivot_team's operations (a row with a zero factor
+// keeps its entry, as there).  root_kernel below, one workgroup pivoting the
+// whole matrix in global memory, took 9.0 ms at n=60 m=120 p=12 (326 x 196)
+// and remains for a w block that is not diagonal; these three take 0.27 ms.
+#define MPQP_ROOT_R 8  // rows per lane: M2 <= 512
+
+// row r of a column held by lane (uniform r)
+__device__ __forceinline__ double root_row(const double (&col)[MPQP_ROOT_R], int r) {
+    double v = col[0];
+#pragma unroll
+    for (int s = 1; s < MPQP_ROOT_R; ++s) v = r / MPQP_WAVE == s ? col[s] : v;
+    return __shfl(v, r % MPQP_WAVE, MPQP_WAVE);
+}
+
+// One pivot (row r, entry p, factor column f) on a column; own: the pivot
+// column itself.
+__device__ __forceinline__ void root_pivot(double (&col)[MPQP_ROOT_R], int M, int r, double p, const double *f,
+                                           bool own) {
+    const int lane = threadIdx.x;
+    double fr[MPQP_ROOT_R];
+#pragma unroll
+    for (int s = 0; s < MPQP_ROOT_R; ++s) {
+        const int i = lane + MPQP_WAVE * s;
+        fr[s] = i < M ? f[i] : 0.0;
+    }
+    const double prj = (own ? 1.0 : root_row(col, r)) / p;
+#pragma unroll
+    for (int s = 0; s < MPQP_ROOT_R; ++s) {
+        const int i = lane + MPQP_WAVE * s;
+        const double t = own ? 0.0 : col[s];
+        const double u = prj != 0.0 ? fma(-fr[s], prj, t) : t;
+        col[s] = i == r ? prj : u;
+    }
+}
+
+// entry (r, v) of the optimality LP's first K columns without the S-only
+// entries of the w columns, the rhs (v = K) and the perturbation (K + 1)
+__device__ __forceinline__ double root_entry(const DevProb &P, double step, int r, int v) {
+    if (v == P.K2) return P.xb2[r];
+    if (v > P.K2) return (double)(r + 1) * step;
+    const int w = v - P.n_x - P.n_t;
+    if (w >= 0 && w < P.n_c && r >= P.M2 - P.n_c - P.n_x && r < P.M2 - P.n_c) return 0.0;
+    return P.A2[(long long)v * P.M2 + r];
+}
+
+static __global__ __launch_bounds__(64) void root_w(RootArgs a) {
+    const DevProb &P = a.P;
+    const int M = P.M2, v = blockIdx.x, lane = threadIdx.x;
+    const int w0 = P.n_x + P.n_t;
+    double col[MPQP_ROOT_R];
+#pragma unroll
+    for (int s = 0; s < MPQP_ROOT_R; ++s) {
+        const int i = lane + MPQP_WAVE * s;
+        col[s] = i < M ? root_entry(P, a.O.perturb_step, i, v) : 0.0;
+    }
+    // rows of w_j: no w pivot but its own changes them.  The factors of the
+    // next pivot are read while this one is applied.
+    auto factors = [&](double (&f)[MPQP_ROOT_R], int j) {
+#pragma unroll
+        for (int s = 0; s < MPQP_ROOT_R; ++s) {
+            const int i = lane + MPQP_WAVE * s;
+            f[s] = root_entry(P, 0.0, i < M ? i : 0, w0 + j);
+        }
+    };
+    double fn[MPQP_ROOT_R];
+    factors(fn, 0);
+    for (int j = 0; j < P.n_c; ++j) {
+        const int r = M - P.n_c + j;
+        const bool own = v == w0 + j;
+        double fr[MPQP_ROOT_R];
+#pragma unroll
+        for (int s = 0; s < MPQP_ROOT_R; ++s) fr[s] = fn[s];
+        factors(fn, j + 1 < P.n_c ? j + 1 : j);
+        const double t = root_row(col, r);
+        if (!own && t == 0.0) continue;
+        const double prj = (own ? 1.0 : t) / root_row(fr, r);
+#pragma unroll
+        for (int s = 0; s < MPQP_ROOT_R; ++s) {
+            const int i = lane + MPQP_WAVE * s;
+            col[s] = i == r ? prj : fma(-fr[s], prj, own ? 0.0 : col[s]);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < MPQP_ROOT_R; ++s) {
+        const int i = lane + MPQP_WAVE * s;
+        if (i < M) a.G[(long long)v * M + i] = col[s];
+    }
+}
+
+// a.F: the factor columns (n_x x M); a.p: the pivots; a.prow: their rows;
+// a.pos: the position of each row.  LDS: the x columns fit there.
+template <int NT, bool LDS>
+__global__ __launch_bounds__(NT) void root_x(RootArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __shared__ int sh_r;
+    __shared__ double sh_pr[512];  // the divided pivot row: n_x <= 512
+    __shared__ int sh_row[512];    // the pivot rows
+    const DevProb &P = a.P;
+    const int M = P.M2, n_x = P.n_x, n_c = P.n_c, n_t = P.n_t, r4 = M - n_c - n_x;
+    const int tid = threadIdx.x, lane = tid % MPQP_WAVE, wave = tid / MPQP_WAVE;
+    double *X;  // column i at X + i * M
+    if constexpr (LDS) X = reinterpret_cast<double *>(smem);
+    else X = a.G;
+    if constexpr (LDS)
+        for (int e = tid; e < n_x * M; e += NT) X[e] = a.G[e];
+    for (int r = tid; r < M; r += NT) a.pos[r] = r >= M - n_c ? n_x + (r - (M - n_c)) : (r < r4 ? n_x + n_c + r : -1);
+    unsigned used = 0u;  // wave 0: bit s of a lane: row r4 + lane + 64 s is taken
+    __syncthreads();
+    int ok = 1;
+    for (int i = 0; i < n_x; ++i) {
+        double *Xi = X + (long long)i * M;
+        if (wave == 0) {
+            // largest |entry| of the free rows, the lowest on ties
+            double v = 0.0;
+            int key = -1, aux = 0;
+            for (int t = lane, s = 0; t < n_x; t += MPQP_WAVE, ++s) {
+                const double av = fabs(Xi[r4 + t]);
+                if (!((used >> s) & 1u) && av == av && (key < 0 || -av < v)) {
+                    v = -av;
+                    key = t;
+                }
+            }
+            lex_min(v, key, aux);
+            if (key >= 0 && key % MPQP_WAVE == lane) used |= 1u << (key / MPQP_WAVE);
+            if (lane == 0) sh_r = key >= 0 && -v > a.O.licq_tol ? r4 + key : -1;
+        }
+        __syncthreads();
+        const int r = sh_r;
+        if (r < 0) {
+            ok = 0;
+            break;
+        }
+        const double p = Xi[r];
+        if (tid == 0) sh_row[i] = r;
+        for (int c = i + 1 + tid; c < n_x; c += NT) sh_pr[c] = X[(long long)c * M + r] / p;
+        __syncthreads();
+        for (int c = i + 1 + wave; c < n_x; c += NT / MPQP_WAVE) {
+            double *Xc = X + (long long)c * M;
+            const double prj = sh_pr[c];
+            double t[MPQP_ROOT_R], f[MPQP_ROOT_R];
+#pragma unroll
+            for (int s = 0; s < MPQP_ROOT_R; ++s) {
+                const int k = lane + MPQP_WAVE * s;
+                t[s] = Xc[k < M ? k : 0];
+                f[s] = Xi[k < M ? k : 0];
+            }
+#pragma unroll
+            for (int s = 0; s < MPQP_ROOT_R; ++s) {
+                const int k = lane + MPQP_WAVE * s;
+                if (k < M) Xc[k] = k == r ? prj : (prj != 0.0 ? fma(-f[s], prj, t[s]) : t[s]);
+            }
+        }
+        __syncthreads();
+    }
+    // column i is left as it was at its pivot: the factors (written once,
+    // since a barrier in the loop would wait for stores to global memory)
+    __syncthreads();
+    for (int e = tid; ok && e < n_x * M; e += NT) a.F[e] = X[e];
+    for (int i = tid; ok && i < n_x; i += NT) {
+        const int r = sh_row[i];
+        a.p[i] = X[(long long)i * M + r];
+        a.prow[i] = r;
+        a.pos[r] = i;
+    }
+    // basis and nonbasic: fixed but for the order of the e_r of the x rows
+    const int N2 = P.N2, K = P.K2;
+    for (int t = tid; t < M; t += NT)
+        a.root_basis[t] = t < n_x ? t : (t < n_x + n_c ? n_x + n_t + (t - n_x) : N2 - M + (t - n_x - n_c));
+    for (int t = tid; t < K; t += NT)
+        a.root_nonb[t] = t < n_t ? n_x + t : (t < n_t + 2 ? n_x + n_t + n_c + (t - n_t) : N2 - M + r4 + (t - n_t - 2));
+    if (a.root32) {
+        int *db = reinterpret_cast<int *>(a.root32 + (long long)opt_tw<float>(M, K));
+        __syncthreads();
+        for (int t = tid; t < M; t += NT) db[t] = a.root_basis[t];
+        for (int t = tid; t < K; t += NT) db[M + t] = a.root_nonb[t];
+    }
+    if (tid == 0) *a.root_ok = ok;
+}
+
+static __global__ __launch_bounds__(64) void root_y(RootArgs a) {
+    if (!*a.root_ok) return;
+    const DevProb &P = a.P;
+    const int M = P.M2, K = P.K2, n_x = P.n_x, n_t = P.n_t, n_c = P.n_c, r4 = M - n_c - n_x;
+    const int v = blockIdx.x, lane = threadIdx.x;
+    double col[MPQP_ROOT_R];
+#pragma unroll
+    for (int s = 0; s < MPQP_ROOT_R; ++s) {
+        const int i = lane + MPQP_WAVE * s;
+        col[s] = i < M && v >= n_x ? a.G[(long long)v * M + i] : 0.0;
+    }
+    // a column x_v begins with its own pivot
+    for (int i = v < n_x ? v : 0; i < n_x; ++i)
+        root_pivot(col, M, a.prow[i], a.p[i], a.F + (long long)i * M, i == v);
+    // its slot: theta', eps, u, then the e of the x rows and of the w rows
+    const int w0 = n_x + n_t;
+    const int kk = v < n_x ? n_t + 2 + a.prow[v] - r4
+                           : (v < w0 ? v - n_x : (v < w0 + n_c ? n_t + 2 + n_x + (v - w0) : (v < K ? n_t + (v - w0 - n_c) : v)));
+#pragma unroll
+    for (int s = 0; s < MPQP_ROOT_R; ++s) {
+        const int i = lane + MPQP_WAVE * s;
+        if (i < M) {
+            a.root[(long long)a.pos[i] * (K + 2) + kk] = col[s];
+            if (a.root32) a.root32[(long long)a.pos[i] * opt_ld<float>(K) + kk] = (float)col[s];
+        }
+    }
+}
 
 template <int NT>
 __global__ __launch_bounds__(NT) void root_kernel(RootArgs a) {

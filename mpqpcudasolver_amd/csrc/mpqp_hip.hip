@@ -653,27 +653,55 @@ struct Run {
         HIP_OK(hipStreamSynchronize(st));
     }
 
+    // The entries of A2 in the rows and columns of the w pivots form a
+    // diagonal block (the identity up to signs, main.py:112-116) with usable
+    // entries: what root_w assumes.
+    bool w_block_diagonal() const {
+        const int n_c = in.n_c, M2 = in.M2, w0 = in.n_x + in.n_t;
+        for (int j = 0; j < n_c; ++j) {
+            const double *col = in.A2 + (size_t)(w0 + j) * M2 + M2 - n_c;
+            for (int i = 0; i < n_c; ++i)
+                if (i != j && col[i] != 0.0) return false;
+            if (!(std::fabs(col[j]) > o.licq_tol)) return false;
+        }
+        return true;
+    }
+
     void build_root() {
         const int M2 = in.M2, N2 = in.N2;
-        BufView dG = A.get(K_ROOTG, -1, sizeof(double) * (size_t)M2 * (K2 + 2));
-        BufView droot = A.get(K_ROOT, -1, sizeof(double) * (size_t)M2 * (K2 + 2));
+        const size_t ng = (size_t)M2 * (K2 + 2), nf = (size_t)M2 * in.n_x;
+        BufView dG = A.get(K_ROOTG, -1, sizeof(double) * (ng + nf + in.n_x));
+        BufView droot = A.get(K_ROOT, -1, sizeof(double) * ng);
         BufView dint = A.get(K_ROOTI, -1, sizeof(int) * (size_t)(M2 + K2 + 2 * N2 + M2 + K2 + 1));
         int *ib = dint.as<int>();
         RootArgs ra{};
         ra.P = P;
         ra.O = dop;
         ra.G = dG.as<double>();
+        ra.F = ra.G + ng;
+        ra.p = ra.F + nf;
         ra.rowvar = ib;
         ra.slotvar = ib + M2;
         ra.rowof = ib + M2 + K2;
         ra.slotof = ib + M2 + K2 + N2;
+        ra.pos = ra.rowvar;    // M2 entries
+        ra.prow = ra.slotvar;  // n_x <= K2 entries
         ra.root_basis = ib + M2 + K2 + 2 * N2;
         ra.root_nonb = ra.root_basis + M2;
         ra.root_ok = ra.root_nonb + K2;
         ra.root = droot.as<double>();
         if (o.precision == MPQP_MIXED)
             ra.root32 = A.get(K_ROOT32, -1, (size_t)opt_state_bytes<float>(M2, K2)).as<float>();
-        hipLaunchKernelGGL(root_kernel<256>, dim3(1), dim3(256), (size_t)(M2 + 1) * 8 + (size_t)M2 * 4, st, ra);
+        if (w_block_diagonal()) {
+            hipLaunchKernelGGL(root_w, dim3((unsigned)(K2 + 2)), dim3(64), 0, st, ra);
+            const size_t xb = sizeof(double) * nf;
+            const bool in_lds = (long long)xb <= C.lds_limit - 6400;  // less its static LDS
+            if (in_lds) hipLaunchKernelGGL((root_x<1024, true>), dim3(1), dim3(1024), xb, st, ra);
+            else hipLaunchKernelGGL((root_x<1024, false>), dim3(1), dim3(1024), 0, st, ra);
+            hipLaunchKernelGGL(root_y, dim3((unsigned)(K2 + 2)), dim3(64), 0, st, ra);
+        } else {
+            hipLaunchKernelGGL(root_kernel<256>, dim3(1), dim3(256), (size_t)(M2 + 1) * 8 + (size_t)M2 * 4, st, ra);
+        }
         HIP_OK(hipGetLastError());
         P.root = ra.root;
         P.root32 = ra.root32;
@@ -704,8 +732,10 @@ struct Run {
         BufView dcq = A.get(K_COLQ, -1, sizeof(double) * (size_t)(n_x + 1));
         upload(dA.p, hA.data(), dA.n);
         upload(dW.p, hW.data(), dW.n);
-        hipLaunchKernelGGL(gram_solve<256>, dim3(1), dim3(256), 0, st, dW.as<double>(), n_x, ldw, ldw,
-                           dcq.as<double>());
+        const size_t wb = sizeof(double) * ((size_t)n_x * ldw + n_x + 1);
+        const bool in_lds = (long long)wb <= C.lds_limit - 64;
+        hipLaunchKernelGGL(gram_solve<1024>, dim3(1), dim3(1024), in_lds ? wb : 0, st, dW.as<double>(), n_x, ldw, ldw,
+                           dcq.as<double>(), in_lds ? 1 : 0);
         const int tiles = (n_c + 15) / 16;
         hipLaunchKernelGGL(gram_mfma, dim3((unsigned)(tiles * tiles)), dim3(64), 0, st, dA.as<const double>(),
                            dW.as<const double>() + n_x, n_c, n_x, ldw, dG.as<double>());

@@ -63,3 +63,35 @@ def test_register_loop_ends(libs, name, opts):
     g, o, _ = _pair(libs, lp, 3, **{"restart_pct": 100, **opts})
     assert compare_runs(g, o) == []
     assert np.array_equal(g.records["repivots"], o.records["repivots"])
+
+
+# ------------------------------------------------------------ the root tableau
+
+def _with_w_entry(lp):
+    """The LP with one off-diagonal entry in the block of the w pivots."""
+    lp.A2 = lp.A2.copy(order="F")
+    lp.A2[lp.M2 - lp.n_c + 3, lp.n_x + lp.n_t + 1] = 0.25
+    return lp
+
+
+ROOTS = [("columns", lambda lp: lp, {}), ("w_block_not_diagonal", _with_w_entry, {}),
+         ("w_pivots_unusable", lambda lp: lp, dict(licq_tol=2.0))]
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("name,change,opts", ROOTS, ids=[r[0] for r in ROOTS])
+def test_root_paths(libs, name, change, opts, precision):
+    """The root built column by column, and by the general elimination where
+    the w block is not diagonal (or has no usable pivot): records and bases
+    equal the oracle's."""
+    print(f"case: root tableau, {name}, precision {precision}", flush=True)
+    hip, orc = libs
+    lp = change(assemble_lps(synthetic_mpqp(7, 20, 3, 4)))
+    runs = []
+    for lib in (hip, orc):
+        lib.set_options(record=2, precision=precision, **opts)
+        runs.append(lib.run(lp, k_max=2, records=True, bases=True))
+        lib.set_options()
+    assert compare_runs(*runs) == []
+    if name == "w_pivots_unusable":
+        assert np.all(runs[0].records["p1_status"][runs[0].records["feasible"] == 1] == 5)
