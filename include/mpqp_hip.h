@@ -314,7 +314,7 @@ int mpqp_regions(const double *A, const double *b, const double *c, const double
  * is dropped (the second implies it) and the second is kept.  All-zero rows
  * with h >= 0 are dropped.
  * fixed (may be NULL): rows that are kept and never tested (equalities).
- * keep[i] = 1 for kept rows.  The LPs run on the device (one wave per LP).
+ * keep[i] = 1 for kept rows.  The LPs run on the device (one workgroup per LP).
  * Returns the number of kept rows; -1 on error, including an empty
  * polyhedron.  *n_lps (may be NULL) receives the number of LPs solved. */
 int mpqp_redundant_rows(const double *G, const double *h, int m, int nz, const int *fixed,

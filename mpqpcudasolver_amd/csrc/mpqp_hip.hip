@@ -103,6 +103,13 @@ void launch_feas(int nt, int grid, size_t lds, hipStream_t st, const FeasArgs &f
     }
 }
 
+// Threads of a redundancy LP's workgroup.  The LPs are few (one per row, and
+// one after the other in the sequential pass), so a pivot is spread as wide
+// as a workgroup goes: 120 rows in 16 dimensions took 5.71 / 2.37 / 1.79 /
+// 1.56 ms with 64 / 256 / 512 / 1024 threads, 12 rows in 4 the same with
+// any, 800 rows in 3 (four LPs a CU) 95 / 59 / 53 / 49 ms.
+constexpr int RED_NT = 1024;
+
 // The LICQ screen with a lane group of gs >= level lanes per candidate.
 void launch_licq(int gs, int n, hipStream_t st, const double *G, int n_c, const int *sets, int kw, int level,
                  double tol, int *fail) {
@@ -1773,10 +1780,10 @@ int run_redundant(const double *G, const double *h, int m, int nz, const int *fi
         HIP_OK(hipMemcpyAsync(dt.p, rows.data(), (size_t)n * 4, hipMemcpyHostToDevice, st));
         RedundArgs ra{m, nz, max_iter, dG, dh, dact, dt.as<int>(), dv.as<double>(), ds.as<int>(), ds.as<int>() + n};
         if (seq)
-            hipLaunchKernelGGL(redundancy_seq_kernel<64>, dim3(1), dim3(64), (size_t)(lds + (long long)m * 4), st, ra, n,
-                               dact);
+            hipLaunchKernelGGL(redundancy_seq_kernel<RED_NT>, dim3(1), dim3(RED_NT), (size_t)(lds + (long long)m * 4), st,
+                               ra, n, dact);
         else
-            hipLaunchKernelGGL(redundancy_kernel<64>, dim3((unsigned)n), dim3(64), (size_t)lds, st, ra);
+            hipLaunchKernelGGL(redundancy_kernel<RED_NT>, dim3((unsigned)n), dim3(RED_NT), (size_t)lds, st, ra);
         HIP_OK(hipGetLastError());
         std::vector<double> val(n);
         std::vector<int> sts(2 * (size_t)n);

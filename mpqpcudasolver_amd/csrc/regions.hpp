@@ -463,7 +463,7 @@ __global__ __launch_bounds__(NT) void region_kernel(RegionArgs a) {
 // P = {z : g_j z <= h_j, j active} (z = (x, theta), rows scaled to unit
 // norm).  Test t of row i: max g_i z over P with row i relaxed to
 // g_i z <= h_i + 1; row i is redundant iff the maximum stays <= h_i.  One
-// wave per test.  z = z+ - z-; an artificial w (-1 in every row) makes the
+// workgroup per test.  z = z+ - z-; an artificial w (-1 in every row) makes the
 // slack basis feasible when some h_j < 0 (phase 1: min w; P is empty if
 // w > 1e-9 at its optimum); phase 2 minimises -g_i z with w barred.
 // ---------------------------------------------------------------------
