@@ -245,53 +245,210 @@ __global__ __launch_bounds__(NT) void feas_kernel(FeasArgs a) {
 }
 
 // ---------------------------------------------------------------------
-// Level-wise enumeration on the device (persistent batching): the children
-// of the feasible parents, S + {j} for j above max S (in parent order, j
-// ascending, as the host enumeration), and the list of feasible candidates.
-// Counts are turned into offsets by an exclusive scan between the kernels.
+// Level-wise enumeration on the device: after the feasibility LPs the list
+// of the feasible candidates and their children's offsets (S + {j} for j
+// above max S, in parent order, j ascending), after the optimality LPs the
+// work sums and the final sets, in order.  Counts that the host needs go
+// into a host-visible mailbox, read once per chunk.  With scans, lists and
+// sums as launches of their own, and a copy and a wait for each count, small
+// calls spent their time there: n=10 m=20 p=2 |S|<=2 in FP64 890 -> 418 us,
+// n=20 m=40 p=4 |S|<=2 without allocation 1429 -> 909 us.  Each kernel here
+// takes 3 to 5 us, most of it the launch.
+//
+// LEVEL_TILE candidates per block.  With more than one block, level_count
+// writes each block's sums first and a block adds up those before it.
 // ---------------------------------------------------------------------
-static __global__ void child_count(const DevRecord *prec, const int *psets, int pn, int kw, int level, int n_c, int *cnt) {
-    const int pi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pi >= pn) return;
-    const int mx = level >= 2 ? psets[(long long)pi * kw + level - 2] : -1;
-    cnt[pi] = prec[pi].feasible ? n_c - 1 - mx : 0;
+#define LEVEL_NT 256
+#define LEVEL_TILE 1024
+#define LEVEL_MAIL_ROWS 16384
+
+struct LevelMail {
+    long long children;          // of the chunk's feasible candidates
+    int nf, final, fb, pad;      // feasible candidates, final sets, failed certifications
+    unsigned long long sums[6];  // see level_sums
+    int rows[LEVEL_MAIL_ROWS];   // the final sets (kw ints each), if they fit
+};
+
+struct LevelArgs {
+    const DevRecord *rec;
+    const int *sets;
+    int n, kw, level, n_c, emit;  // emit: collect the final sets
+    int2 *bsum;                   // per block: feasible and children, or final sets
+    int *list, *off;              // feasible candidates; first child of each candidate
+    int *ctr;                     // 4 counters of the optimality launches, [3]: length of the list
+    unsigned long long *sums;     // 6
+    int *rows;                    // final sets, kw ints each
+    LevelMail *mail;
+};
+
+// max S + 1 .. n_c - 1 extend a feasible candidate of this level
+__device__ __forceinline__ int child_first(const int *sets, int c, int kw, int level) {
+    return level > 0 ? sets[(long long)c * kw + level - 1] + 1 : 0;
 }
 
-// p1par[child] = parent whenever the parent's phase 1 ended optimal (its
-// phase-1 state warm-starts the child), else -1
-static __global__ void child_write(const DevRecord *prec, const int *psets, const int *off, const int *cnt, int pn, int kw,
-                            int level, int *sets, int *par, int *p1par) {
-    const int pi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pi >= pn) return;
-    const int c = cnt[pi];
-    if (c == 0) return;
-    const int *ps = psets + (long long)pi * kw;
-    const int mx = level >= 2 ? ps[level - 2] : -1;
-    const int warm = prec[pi].p1_status == ST_OPTIMAL ? pi : -1;
-    const int o = off[pi];
-    for (int t = 0; t < c; ++t) {
-        int *cs = sets + (long long)(o + t) * kw;
-        for (int u = 0; u < kw; ++u) cs[u] = u < level - 1 ? ps[u] : (u == level - 1 ? mx + 1 + t : -1);
-        par[o + t] = pi;
-        p1par[o + t] = warm;
+__device__ __forceinline__ int2 level_flags(const LevelArgs &a, int c, bool fin) {
+    if (c >= a.n) return make_int2(0, 0);
+    if (fin) return make_int2(a.emit && a.rec[c].final_set ? 1 : 0, 0);
+    const int f = a.rec[c].feasible ? 1 : 0;
+    return make_int2(f, f ? a.n_c - child_first(a.sets, c, a.kw, a.level) : 0);
+}
+
+// Work sums for the statistics: [0] feasibility pivots; [1] phase-1 / [2]
+// phase-2 pivots of the optimality LPs kept in the first precision; [3] / [4]
+// those of the LPs re-solved in FP64; [5] re-solves.
+__device__ __forceinline__ void level_sums(const LevelArgs &a, int c, unsigned long long (&s)[6]) {
+    if (c >= a.n) return;
+    const DevRecord &r = a.rec[c];
+    const bool rs = r.repivots != 0;
+    s[0] += (unsigned long long)r.feas_iters;
+    s[1] += (unsigned long long)(rs ? 0 : r.p1_iters);
+    s[2] += (unsigned long long)(rs ? 0 : r.p2_iters);
+    s[3] += (unsigned long long)(rs ? r.p1_iters : 0);
+    s[4] += (unsigned long long)(rs ? r.p2_iters : 0);
+    s[5] += (unsigned long long)r.repivots;
+}
+
+// the block's sums, added to out (LDS, cleared before)
+__device__ __forceinline__ void level_sums_add(unsigned long long (&v)[6], unsigned long long *out) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+#pragma unroll
+        for (int d = MPQP_WAVE / 2; d > 0; d >>= 1) v[i] += __shfl_xor(v[i], d, MPQP_WAVE);
+        if (threadIdx.x % MPQP_WAVE == 0 && v[i]) atomicAdd(&out[i], v[i]);
+    }
+    __syncthreads();
+}
+
+// Exclusive prefix of v over the block's threads, the block's total in tot.
+__device__ __forceinline__ int2 block_prefix(int2 v, int2 &tot) {
+    __shared__ int2 ws[LEVEL_NT / MPQP_WAVE];
+    const int lane = threadIdx.x % MPQP_WAVE, wave = threadIdx.x / MPQP_WAVE;
+    int2 x = v;
+#pragma unroll
+    for (int d = 1; d < MPQP_WAVE; d <<= 1) {
+        const int ox = __shfl_up(x.x, d, MPQP_WAVE), oy = __shfl_up(x.y, d, MPQP_WAVE);
+        if (lane >= d) {
+            x.x += ox;
+            x.y += oy;
+        }
+    }
+    __syncthreads();
+    if (lane == MPQP_WAVE - 1) ws[wave] = x;
+    __syncthreads();
+    int2 base = make_int2(0, 0);
+    tot = make_int2(0, 0);
+#pragma unroll
+    for (int w = 0; w < LEVEL_NT / MPQP_WAVE; ++w) {
+        if (w < wave) {
+            base.x += ws[w].x;
+            base.y += ws[w].y;
+        }
+        tot.x += ws[w].x;
+        tot.y += ws[w].y;
+    }
+    return make_int2(base.x + x.x - v.x, base.y + x.y - v.y);
+}
+
+// FIN: the final sets and the work sums, else the feasible candidates.
+template <bool FIN>
+__global__ __launch_bounds__(LEVEL_NT) void level_count(LevelArgs a) {
+    __shared__ unsigned long long s[6];
+    if (FIN && threadIdx.x < 6) s[threadIdx.x] = 0ull;
+    __syncthreads();
+    unsigned long long w[6] = {};
+    int2 v = make_int2(0, 0);
+    for (int u = threadIdx.x; u < LEVEL_TILE; u += LEVEL_NT) {
+        const int c = blockIdx.x * LEVEL_TILE + u;
+        const int2 f = level_flags(a, c, FIN);
+        v.x += f.x;
+        v.y += f.y;
+        if (FIN) level_sums(a, c, w);
+    }
+    int2 tot;
+    block_prefix(v, tot);
+    if (FIN) level_sums_add(w, s);
+    if (threadIdx.x == 0) a.bsum[blockIdx.x] = tot;
+    if (FIN && threadIdx.x < 6) atomicAdd(&a.sums[threadIdx.x], s[threadIdx.x]);
+}
+
+template <bool FIN>
+__global__ __launch_bounds__(LEVEL_NT) void level_write(LevelArgs a) {
+    __shared__ unsigned long long s[6];
+    __shared__ long long before[2];
+    const bool one = gridDim.x == 1;
+    if (threadIdx.x < 6) s[threadIdx.x] = 0ull;
+    if (threadIdx.x < 2) before[threadIdx.x] = 0;
+    __syncthreads();
+    long long px = 0, py = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += LEVEL_NT) {
+        px += a.bsum[b].x;
+        py += a.bsum[b].y;
+    }
+    if (px) atomicAdd((unsigned long long *)&before[0], (unsigned long long)px);
+    if (py) atomicAdd((unsigned long long *)&before[1], (unsigned long long)py);
+    __syncthreads();
+    px = before[0];
+    py = before[1];
+    unsigned long long w[6] = {};
+    for (int u = 0; u < LEVEL_TILE; u += LEVEL_NT) {
+        const int c = blockIdx.x * LEVEL_TILE + u + threadIdx.x;
+        if (blockIdx.x * LEVEL_TILE + u >= a.n) break;
+        const int2 f = level_flags(a, c, FIN);
+        if (FIN && one) level_sums(a, c, w);
+        int2 tot;
+        const int2 e = block_prefix(f, tot);
+        const int pos = (int)(px + e.x);
+        if constexpr (!FIN) {
+            if (c < a.n) a.off[c] = (int)(py + e.y);
+            if (f.x) a.list[pos] = c;
+        } else if (f.x) {
+            const int *S = a.sets + (long long)c * a.kw;
+            for (int t = 0; t < a.kw; ++t) {
+                const long long at = (long long)pos * a.kw + t;
+                a.rows[at] = S[t];
+                if (at < LEVEL_MAIL_ROWS) a.mail->rows[at] = S[t];
+            }
+        }
+        px += tot.x;
+        py += tot.y;
+    }
+    if (FIN && one) level_sums_add(w, s);
+    if (blockIdx.x != gridDim.x - 1) return;
+    if constexpr (!FIN) {
+        if (threadIdx.x < 6) a.sums[threadIdx.x] = 0ull;
+        if (threadIdx.x == 0) {
+            a.ctr[0] = a.ctr[1] = a.ctr[2] = 0;
+            a.ctr[3] = (int)px;
+            a.mail->nf = (int)px;
+            a.mail->children = py;
+        }
+    } else {
+        if (threadIdx.x < 6) a.mail->sums[threadIdx.x] = one ? s[threadIdx.x] : a.sums[threadIdx.x];
+        if (threadIdx.x == 0) {
+            a.mail->final = (int)px;
+            a.mail->fb = a.ctr[1];
+        }
     }
 }
 
-// child_write over parents [p0, p0 + pn) of a chunk: off[t] is parent
-// p0 + t's first child relative to the range; par holds chunk-wide parent
-// indices (their rows in the parent chunk's state stores)
-static __global__ void child_write_range(const DevRecord *prec, const int *psets, const int *off, int p0, int pn, int kw,
-                                  int level, int n_c, int *sets, int *par, int *p1par) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+// Children of parents [p0, p0 + pn) of a chunk: parent p0 + t's first child
+// is row off[t] of the range; par holds chunk-wide parent indices
+// (their rows in the parent chunk's state stores), p1par the parent whenever
+// its phase 1 ended optimal (its phase-1 state warm-starts the child), else
+// -1.  CHILD_LANES lanes per parent, a child each.
+#define CHILD_LANES 16
+static __global__ __launch_bounds__(256) void child_write(const DevRecord *prec, const int *psets, const int *off, int p0, int pn,
+                                                          int kw, int level, int n_c, int *sets, int *par, int *p1par) {
+    const int t = (blockIdx.x * 256 + threadIdx.x) / CHILD_LANES, g = threadIdx.x % CHILD_LANES;
     if (t >= pn) return;
     const int pi = p0 + t;
     if (!prec[pi].feasible) return;
     const int *ps = psets + (long long)pi * kw;
-    const int mx = level >= 2 ? ps[level - 2] : -1;
+    const int j0 = child_first(psets, pi, kw, level - 1);
     const int warm = prec[pi].p1_status == ST_OPTIMAL ? pi : -1;
     const int o = off[t];
-    for (int j = mx + 1; j < n_c; ++j) {
-        const int ch = o + (j - mx - 1);
+    for (int j = j0 + g; j < n_c; j += CHILD_LANES) {
+        const int ch = o + (j - j0);
         int *cs = sets + (long long)ch * kw;
         for (int u = 0; u < kw; ++u) cs[u] = u < level - 1 ? ps[u] : (u == level - 1 ? j : -1);
         par[ch] = pi;
@@ -299,13 +456,29 @@ static __global__ void child_write_range(const DevRecord *prec, const int *psets
     }
 }
 
-// rows[t] = sets[idx[t]] widened to nx entries, -1 padded (t < cnt)
-static __global__ void gather_rows_nx(const int *sets, const int *idx, int cnt, int kw, int nx, int *rows) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < cnt * nx) {
-        const int t = e / nx, u = e - t * nx;
-        rows[e] = u < kw ? sets[(long long)idx[t] * kw + u] : -1;
+// level 0: the empty set, without a parent
+static __global__ void level0_write(int *sets, int kw, int *par, int *p1par) {
+    for (int u = threadIdx.x; u < kw; u += blockDim.x) sets[u] = -1;
+    if (threadIdx.x == 0) *par = *p1par = -1;
+}
+
+// [Q | A^T] of gram_solve from A2 (its stationarity rows, columns x', each
+// row restored to the sign of its positive diagonal entry: main.py:108-116
+// negates the rows whose right-hand side is negative) and A (n_c x n_x).
+static __global__ __launch_bounds__(256) void gram_pack(const double *A2, int M2, int n_c, int n_x, const double *A,
+                                                        double *W) {
+    const int ld = n_x + n_c, r4 = M2 - n_c - n_x;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= n_x * ld) return;
+    const int i = e / ld, c = e - i * ld;
+    double v;
+    if (c < n_x) {
+        v = A2[(long long)c * M2 + r4 + i];
+        if (A2[(long long)i * M2 + r4 + i] < 0.0) v = -v;
+    } else {
+        v = A[(long long)(c - n_x) * n_x + i];
     }
+    W[e] = v;
 }
 
 // ---------------------------------------------------------------------
@@ -392,47 +565,6 @@ __global__ __launch_bounds__(64) void licq_screen(const double *G, int n_c, cons
         }
     }
     if (live && r == 0) fail[c] = bad ? 1 : 0;
-}
-
-static __global__ void feasible_flag(const DevRecord *rec, int n, int *flag) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n) flag[c] = rec[c].feasible ? 1 : 0;
-}
-
-// Record-free end of a call: per-level work sums for the statistics and
-// the final-set flags.  out[0] feasibility pivots; [1] phase-1 / [2] phase-2
-// pivots of the optimality LPs kept in the first precision; [3] / [4] those
-// of the LPs re-solved in FP64; [5] re-solves.  One atomic per block and sum.
-static __global__ void level_summary(const DevRecord *rec, int n, unsigned long long *out, int *flag) {
-    __shared__ unsigned long long s[6];
-    if (threadIdx.x < 6) s[threadIdx.x] = 0ull;
-    __syncthreads();
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n) {
-        const DevRecord &r = rec[c];
-        const int rs = r.repivots ? 1 : 0;
-        atomicAdd(&s[0], (unsigned long long)r.feas_iters);
-        atomicAdd(&s[rs ? 3 : 1], (unsigned long long)r.p1_iters);
-        atomicAdd(&s[rs ? 4 : 2], (unsigned long long)r.p2_iters);
-        if (rs) atomicAdd(&s[5], (unsigned long long)r.repivots);
-        flag[c] = r.final_set ? 1 : 0;
-    }
-    __syncthreads();
-    if (threadIdx.x < 6) atomicAdd(&out[threadIdx.x], s[threadIdx.x]);
-}
-
-// rows[t] = sets[idx[t]] (kw ints each) for t < cnt
-static __global__ void gather_rows(const int *sets, const int *idx, int cnt, int kw, int *rows) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < cnt * kw) {
-        const int t = e / kw, u = e - t * kw;
-        rows[e] = sets[(long long)idx[t] * kw + u];
-    }
-}
-
-static __global__ void list_write(const int *flag, const int *pos, int n, int *list) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n && flag[c]) list[pos[c]] = c;
 }
 
 // ---------------------------------------------------------------------

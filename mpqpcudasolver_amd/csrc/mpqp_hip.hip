@@ -37,8 +37,6 @@
 #include <thread>
 #include <vector>
 
-#include <hipcub/hipcub.hpp>
-
 #include "../../include/mpqp_hip.h"
 #include "kernels.hpp"
 #include "opt_fn.hpp"
@@ -162,8 +160,7 @@ enum Kind {
     K_A1, K_XB1, K_A2, K_XB2, K_AMAT, K_GW, K_G, K_SPI, K_SPD, K_ROOTG, K_ROOT, K_ROOT32, K_ROOTI, K_CTR, K_GT64, K_GT32,
     K_SUM, K_COLQ,
     R_IN, R_SETS, R_OUT, R_INFO,
-    L_SETS, L_PAR, L_P1PAR, L_REC, L_FLAG, L_POS, L_LIST, L_FBL, L_CNT, L_OFF, L_FS, L_OS, L_FB, L_B1, L_B2,
-    L_FIDX, L_FROWS, L_LICQ, L_SCAN,
+    L_SETS, L_PAR, L_P1PAR, L_REC, L_LIST, L_FBL, L_OFF, L_ROFF, L_FS, L_OS, L_FB, L_B1, L_B2, L_FROWS, L_LICQ, L_BSUM,
     K_N
 };
 
@@ -274,7 +271,8 @@ struct Ctx {
     bool ready = false;
     int device = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+    LevelMail *mail = nullptr;  // pinned host memory that the level kernels write
     MpqpOptions opt{};
     bool opt_set = false;
     std::string err;
@@ -291,6 +289,23 @@ struct Ctx {
     // its LDS share is sized for (FP32, FP64); the sizes of the last call
     std::map<std::vector<int>, std::vector<int>> tuned;
     int last_feas_nt = 0, last_opt_nt = 0;
+    // mailboxes of mpqp_many()'s workers, kept for later calls (at most
+    // MAX_MAIL; a call with more workers allocates the others for itself)
+    static constexpr size_t MAX_MAIL = 16;
+    std::vector<LevelMail *> many_mail;
+    LevelMail *worker_mail(size_t w) {
+        if (w < many_mail.size()) return many_mail[w];
+        LevelMail *m = nullptr;
+        HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&m), sizeof(LevelMail)));
+        many_mail.push_back(m);
+        return m;
+    }
+    void trim_mail() {
+        while (many_mail.size() > MAX_MAIL) {
+            hipHostFree(many_mail.back());
+            many_mail.pop_back();
+        }
+    }
     // the result of the last mpqp() call, freed by the next call unless the
     // caller freed it (the reference's host never frees its results)
     GPUResults *last_res = nullptr;
@@ -363,6 +378,7 @@ void ensure_ready() {
     HIP_OK(hipSetDevice(c.device));
     HIP_OK(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
     for (hipEvent_t &e : c.ev) HIP_OK(hipEventCreate(&e));
+    HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&c.mail), sizeof(LevelMail)));
     int lds = 0;
     HIP_OK(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, c.device));
     c.lds_limit = lds;
@@ -526,6 +542,7 @@ struct Run {
     bool tune_pending = false;
     std::vector<int> tkey;
     double *G = nullptr;
+    std::vector<double> hA;  // uploaded asynchronously: lives as long as the call
     std::vector<long long> cap_lvl;  // most candidates per chunk, by level
     // outputs, by level
     std::vector<std::vector<MpqpRecord>> rec_lvl;
@@ -567,7 +584,7 @@ struct Run {
             for (int rho = 0; rho < M2; ++rho) bmax = std::max(bmax, std::fabs(in.xb2[rho]));
             P.cert_ptol = 1e-12 * (1.0 + bmax);
         }
-        build_sparse();
+        if (o.precision == MPQP_MIXED) build_sparse();  // read by the certificate alone
         build_root();
         if (screen) build_gram();
     }
@@ -718,27 +735,21 @@ struct Run {
     }
 
     // G = A Q^-1 A^T for the LICQ screen.  A: the rows of AxT (or of A1 when
-    // AxT is null); Q: the stationarity rows of A2 (columns x'), each row
-    // restored to the sign of its positive diagonal entry (main.py:108-116
-    // negates the rows whose right-hand side is negative).
+    // AxT is null); Q: the stationarity rows of A2 (gram_pack).
     void build_gram() {
-        const int n_c = in.n_c, n_x = in.n_x, M2 = in.M2, M1 = in.M1;
-        const int r4 = M2 - n_c - n_x, ldw = n_x + n_c;
-        std::vector<double> hA((size_t)n_c * n_x), hW((size_t)n_x * ldw);
-        for (int j = 0; j < n_c; ++j)
-            for (int i = 0; i < n_x; ++i)
-                hA[(size_t)j * n_x + i] = in.AxT ? in.AxT[(size_t)j * n_x + i] : in.A1[(size_t)i * M1 + j];
-        for (int i = 0; i < n_x; ++i) {
-            const double sgn = in.A2[(size_t)i * M2 + r4 + i] < 0.0 ? -1.0 : 1.0;
-            for (int c = 0; c < n_x; ++c) hW[(size_t)i * ldw + c] = sgn * in.A2[(size_t)c * M2 + r4 + i];
-            for (int j = 0; j < n_c; ++j) hW[(size_t)i * ldw + n_x + j] = hA[(size_t)j * n_x + i];
+        const int n_c = in.n_c, n_x = in.n_x, M2 = in.M2, M1 = in.M1, ldw = n_x + n_c;
+        if (!in.AxT) {
+            hA.resize((size_t)n_c * n_x);
+            for (int j = 0; j < n_c; ++j)
+                for (int i = 0; i < n_x; ++i) hA[(size_t)j * n_x + i] = in.A1[(size_t)i * M1 + j];
         }
-        BufView dA = A.get(K_AMAT, -1, sizeof(double) * hA.size());
-        BufView dW = A.get(K_GW, -1, sizeof(double) * hW.size());
+        BufView dA = A.get(K_AMAT, -1, sizeof(double) * (size_t)n_c * n_x);
+        BufView dW = A.get(K_GW, -1, sizeof(double) * (size_t)n_x * ldw);
         BufView dG = A.get(K_G, -1, sizeof(double) * (size_t)n_c * n_c);
         BufView dcq = A.get(K_COLQ, -1, sizeof(double) * (size_t)(n_x + 1));
-        upload(dA.p, hA.data(), dA.n);
-        upload(dW.p, hW.data(), dW.n);
+        upload(dA.p, in.AxT ? in.AxT : hA.data(), dA.n);
+        hipLaunchKernelGGL(gram_pack, grid256((long long)n_x * ldw), dim3(256), 0, st, P.A2, M2, n_c, n_x,
+                           dA.as<const double>(), dW.as<double>());
         const size_t wb = sizeof(double) * ((size_t)n_x * ldw + n_x + 1);
         const bool in_lds = (long long)wb <= C.lds_limit - 64;
         hipLaunchKernelGGL(gram_solve<1024>, dim3(1), dim3(1024), in_lds ? wb : 0, st, dW.as<double>(), n_x, ldw, ldw,
@@ -747,7 +758,6 @@ struct Run {
         hipLaunchKernelGGL(gram_mfma, dim3((unsigned)(tiles * tiles)), dim3(64), 0, st, dA.as<const double>(),
                            dW.as<const double>() + n_x, n_c, n_x, ldw, dG.as<double>());
         HIP_OK(hipGetLastError());
-        HIP_OK(hipStreamSynchronize(st));
         G = dG.as<double>();
     }
 
@@ -879,8 +889,8 @@ struct Run {
     // device bytes a candidate of `level` needs in its chunk
     size_t cand_bytes(int level) const {
         const bool store = level < last_lvl;
-        // sets, rows of final sets (kw ints each), 12 ints of lists,
-        // counters and scan storage, the record
+        // sets, rows of final sets (kw ints each), 12 ints of lists, offsets
+        // and block sums, the record
         size_t b = sizeof(int) * (size_t)(2 * kw + 12) + sizeof(DevRecord);
         if (store) b += (size_t)fstride + (size_t)ostride;
         if (keep_bases) b += sizeof(int) * (size_t)(in.M1 + 2 * in.M2);
@@ -892,13 +902,13 @@ struct Run {
         if (gt64) A.get(K_GT64, -1, gtab64_max);
         if (gt32 && mixed) A.get(K_GT32, -1, gtab32_max);
         A.get(K_CTR, -1, sizeof(int) * 4);
-        A.get(K_SUM, -1, sizeof(unsigned long long) * 8 * (size_t)(last_lvl + 1));
+        A.get(K_SUM, -1, sizeof(unsigned long long) * 6);
         const size_t budget = A.budget((size_t)std::max(in.reserved_memory, 0) << 20);
         const int nl = last_lvl + 1;
         A.set_levels(nl);
         cap_lvl.assign(nl, 1);
         // per level: an equal share of the budget, less alignment and the
-        // scan's fixed storage
+        // block sums
         const size_t share = budget / (size_t)nl, slack = (size_t)1 << 20;
         for (int L = 0; L < nl; ++L) {
             long long c = (long long)((share > slack ? share - slack : 0) / cand_bytes(L));
@@ -910,20 +920,6 @@ struct Run {
         }
     }
 
-    // exclusive scan of nn ints (temporary storage of `level`)
-    void scan(const int *src, int *dst, int nn, int level) {
-        size_t tb = 0;
-        HIP_OK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, src, dst, nn, st));
-        const BufView tmp = A.get(L_SCAN, level, std::max<size_t>(tb, 16));
-        HIP_OK(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, src, dst, nn, st));
-    }
-    int scan_total(const int *src, const int *dst, int nn) {
-        int t[2] = {0, 0};
-        HIP_OK(hipMemcpyAsync(&t[0], dst + nn - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipMemcpyAsync(&t[1], src + nn - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIP_OK(hipStreamSynchronize(st));
-        return t[0] + t[1];
-    }
     static dim3 grid256(long long nn) { return dim3((unsigned)((nn + 255) / 256)); }
 
     // statistics of a chunk from its host records
@@ -957,7 +953,7 @@ struct Run {
         St.flops_feas += pf * flops(in.M1, K1);
     }
 
-    // statistics from the device sums of level_summary (the same totals:
+    // statistics from the device sums of level_sums (the same totals:
     // every term is an integer-valued double)
     void sum_stats(const unsigned long long *sm) {
         MpqpStats &St = C.stats;
@@ -992,7 +988,7 @@ struct Run {
         const bool store = level < last_lvl;
         const bool bases = keep_bases && !probe_only;
         const long long base = n_lvl[level];
-        hipEvent_t e0 = C.ev[0], e1 = C.ev[1], e2 = C.ev[2], e3 = C.ev[3];
+        hipEvent_t e0 = C.ev[0], e1 = C.ev[1], e2 = C.ev[2], e3 = C.ev[3], e4 = C.ev[4];
         BufView drec = lvl_buf(L_REC, level, sizeof(DevRecord) * (size_t)n);
         BufView fs, os;
         if (store) {
@@ -1060,36 +1056,45 @@ struct Run {
         HIP_OK(hipGetLastError());
         HIP_OK(hipEventRecord(e1, st));
 
-        // optimality LPs of the feasible candidates
-        const BufView flag = lvl_buf(L_FLAG, level, sizeof(int) * (size_t)n);
-        const BufView pos = lvl_buf(L_POS, level, sizeof(int) * (size_t)n);
-        hipLaunchKernelGGL(feasible_flag, grid256(n), dim3(256), 0, st, drec.as<const DevRecord>(), n, flag.as<int>());
-        HIP_OK(hipGetLastError());
-        scan(flag.as<const int>(), pos.as<int>(), n, level);
-        const int nf = scan_total(flag.as<const int>(), pos.as<const int>(), n);
-        BufView dlist;
-        if (nf > 0) {
-            dlist = lvl_buf(L_LIST, level, sizeof(int) * (size_t)n);
-            hipLaunchKernelGGL(list_write, grid256(n), dim3(256), 0, st, flag.as<const int>(), pos.as<const int>(), n,
-                               dlist.as<int>());
-            HIP_OK(hipGetLastError());
-        }
-        float ms = 0.f;
-        HIP_OK(hipEventSynchronize(e1));
-        HIP_OK(hipEventElapsedTime(&ms, e0, e1));
-        if (!probe_only) {
-            out.tf += ms * 1e-3;
-            C.stats.ms_feas += ms;
-        }
-        int n_fb = 0;
+        // the feasible candidates and their children's offsets
         BufView dctr = A.get(K_CTR, -1, sizeof(int) * 4);
+        const int nb = (n + LEVEL_TILE - 1) / LEVEL_TILE;
+        const BufView dlist = lvl_buf(L_LIST, level, sizeof(int) * (size_t)n);
+        const BufView doff = lvl_buf(L_OFF, level, sizeof(int) * (size_t)n);
+        LevelArgs la{};
+        la.rec = drec.as<const DevRecord>();
+        la.sets = dsets.as<const int>();
+        la.n = n;
+        la.kw = kw;
+        la.level = level;
+        la.n_c = in.n_c;
+        la.emit = !keep_rec && !probe_only && level >= in.k_min ? 1 : 0;
+        la.bsum = lvl_buf(L_BSUM, level, sizeof(int2) * (size_t)nb).as<int2>();
+        la.list = dlist.as<int>();
+        la.off = doff.as<int>();
+        la.ctr = dctr.as<int>();
+        la.sums = A.get(K_SUM, -1, sizeof(unsigned long long) * 6).as<unsigned long long>();
+        la.rows = la.emit ? lvl_buf(L_FROWS, level, sizeof(int) * (size_t)n * kw).as<int>() : nullptr;
+        la.mail = C.mail;
+        if (nb > 1) hipLaunchKernelGGL(level_count<false>, dim3(nb), dim3(LEVEL_NT), 0, st, la);
+        hipLaunchKernelGGL(level_write<false>, dim3(nb), dim3(LEVEL_NT), 0, st, la);
+        HIP_OK(hipGetLastError());
+        // optimality LPs of the feasible candidates: the kernels take their
+        // number from the device.  A plain launch has a workgroup for each
+        // candidate of a small chunk (those past the list end at once), and is
+        // sized by the list otherwise; the autotuner samples the list.
+        const bool plain = !mixed && o.batching != MPQP_PERSISTENT && !gt64;
+        int nf = n;
+        if (tune_here || (plain && n > 1024)) {
+            HIP_OK(hipStreamSynchronize(st));
+            nf = C.mail->nf;
+        }
         if (nf > 0) {
-            hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, dctr.as<int>(), 4, 0);
-            HIP_OK(hipGetLastError());
             OptArgs oa{};
             oa.P = P;
             oa.O = dop;
             oa.n = nf;
+            oa.n_dev = dctr.as<int>() + 3;
             oa.level = level;
             oa.kw = kw;
             oa.list = dlist.as<int>();
@@ -1103,7 +1108,7 @@ struct Run {
             oa.b1 = bases ? db1.as<int>() : nullptr;
             oa.b2 = bases ? db2.as<int>() : nullptr;
             BufView dfbl;
-            if (mixed) dfbl = lvl_buf(L_FBL, level, sizeof(int) * (size_t)nf);
+            if (mixed) dfbl = lvl_buf(L_FBL, level, sizeof(int) * (size_t)n);
             BufView gtab64 = gt64 ? A.get(K_GT64, -1, gtab64_max) : BufView{};
             BufView gtab32 = (gt32 && mixed) ? A.get(K_GT32, -1, gtab32_max) : BufView{};
             if (tune_here) {
@@ -1115,10 +1120,11 @@ struct Run {
                 if (variants.size() == 1) best_v = variants[0];
                 else for (const auto &v : variants) {
                     select_variant(v[0], v[1], v[2]);
-                    hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, dctr.as<int>(), 4, 0);
+                    hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, dctr.as<int>(), 3, 0);
                     HIP_OK(hipGetLastError());
                     OptArgs ot = oa;
                     ot.n = std::min(nf, 8192);
+                    ot.n_dev = nullptr;
                     ot.counter = dctr.as<int>();
                     if (mixed) {
                         ot.fb_list = dfbl.as<int>();
@@ -1143,12 +1149,12 @@ struct Run {
                     }
                 }
                 select_variant(best_v[0], best_v[1], best_v[2]);
-                hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, dctr.as<int>(), 4, 0);
+                hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, dctr.as<int>(), 3, 0);
                 HIP_OK(hipGetLastError());
                 C.tuned[tkey] = {feas_nt, opt_nt, w32, w64};
                 tune_pending = false;
             }
-            HIP_OK(hipEventRecord(e1, st));
+            HIP_OK(hipEventRecord(e4, st));
             if (mixed) {
                 oa.counter = dctr.as<int>();
                 oa.fb_list = dfbl.as<int>();
@@ -1181,9 +1187,23 @@ struct Run {
                 launch_opt(fn64, nf, lds64, oa);
             }
             HIP_OK(hipEventRecord(e2, st));
-            HIP_OK(hipEventSynchronize(e2));
-            HIP_OK(hipEventElapsedTime(&ms, e1, e2));
-            if (!probe_only) {
+        }
+        // work sums and final sets, then the one wait of a chunk
+        if (nb > 1) hipLaunchKernelGGL(level_count<true>, dim3(nb), dim3(LEVEL_NT), 0, st, la);
+        hipLaunchKernelGGL(level_write<true>, dim3(nb), dim3(LEVEL_NT), 0, st, la);
+        HIP_OK(hipGetLastError());
+        HIP_OK(hipStreamSynchronize(st));
+        const bool launched = nf > 0;
+        nf = C.mail->nf;
+        const long long n_children = C.mail->children;
+        const int n_final = C.mail->final, n_fb = C.mail->fb;
+        if (!probe_only) {
+            float ms = 0.f;
+            HIP_OK(hipEventElapsedTime(&ms, e0, e1));
+            out.tf += ms * 1e-3;
+            C.stats.ms_feas += ms;
+            if (launched && nf > 0) {
+                HIP_OK(hipEventElapsedTime(&ms, e4, e2));
                 out.to += ms * 1e-3;
                 C.stats.ms_opt += ms;
                 C.stats.launches_opt += mixed ? 2 : 1;
@@ -1192,11 +1212,6 @@ struct Run {
                     C.stats.ms_fallback += ms;
                     C.stats.launches_fallback += 1;
                 }
-            }
-            if (mixed && level <= 1) {
-                // the FP32 launch counted its certification failures
-                HIP_OK(hipMemcpyAsync(&n_fb, dctr.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost, st));
-                HIP_OK(hipStreamSynchronize(st));
             }
         }
         if (mixed && level <= 1) {
@@ -1250,29 +1265,15 @@ struct Run {
             }
         } else {
             // statistics summed and final sets compacted on the device
-            const BufView dsum = A.get(K_SUM, -1, sizeof(unsigned long long) * 8 * (size_t)(last_lvl + 1));
-            const BufView fflag = lvl_buf(L_FIDX, level, sizeof(int) * (size_t)n);
-            hipLaunchKernelGGL(level_summary, grid256(n), dim3(256), 0, st, drec.as<DevRecord>(), n,
-                               dsum.as<unsigned long long>() + 8 * level, fflag.as<int>());
-            HIP_OK(hipGetLastError());
-            if (level >= in.k_min) {
-                scan(fflag.as<int>(), pos.as<int>(), n, level);
-                const int cnt = scan_total(fflag.as<int>(), pos.as<int>(), n);
-                if (cnt > 0) {
-                    const BufView idx = lvl_buf(L_LIST, level, sizeof(int) * (size_t)n);
-                    hipLaunchKernelGGL(list_write, grid256(n), dim3(256), 0, st, fflag.as<int>(), pos.as<int>(), n,
-                                       idx.as<int>());
-                    const BufView rows = lvl_buf(L_FROWS, level, sizeof(int) * (size_t)cnt * kw);
-                    hipLaunchKernelGGL(gather_rows, grid256((long long)cnt * kw), dim3(256), 0, st, dsets.as<int>(),
-                                       idx.as<int>(), cnt, kw, rows.as<int>());
-                    HIP_OK(hipGetLastError());
-                    std::vector<int> &F = fin_lvl[level];
-                    const size_t f0 = F.size();
-                    F.resize(f0 + (size_t)cnt * kw);
-                    HIP_OK(hipMemcpyAsync(F.data() + f0, rows.p, sizeof(int) * (size_t)cnt * kw, hipMemcpyDeviceToHost,
-                                          st));
-                    HIP_OK(hipStreamSynchronize(st));
-                }
+            sum_stats(C.mail->sums);
+            std::vector<int> &F = fin_lvl[level];
+            const size_t f0 = F.size(), cnt = (size_t)n_final * kw;
+            F.resize(f0 + cnt);
+            if (cnt <= LEVEL_MAIL_ROWS) {
+                std::copy_n(C.mail->rows, cnt, F.begin() + f0);
+            } else {
+                HIP_OK(hipMemcpyAsync(F.data() + f0, la.rows, sizeof(int) * cnt, hipMemcpyDeviceToHost, st));
+                HIP_OK(hipStreamSynchronize(st));
             }
         }
 
@@ -1280,13 +1281,25 @@ struct Run {
         // chunks of at most cap_lvl[level + 1] and processed depth first
         if (!store) return true;
         const int nxt = level + 1;
-        const BufView dcnt = lvl_buf(L_CNT, level, sizeof(int) * (size_t)n);
-        hipLaunchKernelGGL(child_count, grid256(n), dim3(256), 0, st, drec.as<const DevRecord>(), dsets.as<const int>(),
-                           n, kw, nxt, in.n_c, dcnt.as<int>());
-        HIP_OK(hipGetLastError());
-        std::vector<int> hcnt(n);
-        HIP_OK(hipMemcpyAsync(hcnt.data(), dcnt.p, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, st));
+        auto descend = [&](int p0, int pn, long long tot, const int *off) {
+            A.begin_level(nxt);
+            const BufView csets = lvl_buf(L_SETS, nxt, sizeof(int) * (size_t)tot * kw);
+            const BufView cpar = lvl_buf(L_PAR, nxt, sizeof(int) * (size_t)tot);
+            const BufView cp1 = lvl_buf(L_P1PAR, nxt, sizeof(int) * (size_t)tot);
+            hipLaunchKernelGGL(child_write, grid256((long long)pn * CHILD_LANES), dim3(256), 0, st,
+                               drec.as<const DevRecord>(), dsets.as<const int>(), off, p0, pn, kw, nxt, in.n_c, csets.as<int>(), cpar.as<int>(),
+                               cp1.as<int>());
+            HIP_OK(hipGetLastError());
+            return process(nxt, (int)tot, csets, cpar, cp1, fs, os, base);
+        };
+        if (n_children == 0) return true;
+        if (n_children <= cap_lvl[nxt]) return descend(0, n, n_children, doff.as<const int>());
+        // several chunks: the children of ranges of parents
+        std::vector<int> hoff0(n), hcnt(n);
+        HIP_OK(hipMemcpyAsync(hoff0.data(), doff.p, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, st));
         HIP_OK(hipStreamSynchronize(st));
+        for (int t = 0; t < n; ++t)
+            hcnt[t] = (int)((unsigned)(t + 1 < n ? hoff0[t + 1] : (int)n_children) - (unsigned)hoff0[t]);
         const long long cap = cap_lvl[nxt];
         int p0 = 0;
         while (p0 < n) {
@@ -1304,18 +1317,10 @@ struct Run {
                     hoff[t - p0] = (int)acc;
                     acc += hcnt[t];
                 }
-                const BufView doff = lvl_buf(L_OFF, level, sizeof(int) * (size_t)(p1 - p0));
-                upload(doff.p, hoff.data(), doff.n);
-                A.begin_level(nxt);
-                const BufView csets = lvl_buf(L_SETS, nxt, sizeof(int) * (size_t)tot * kw);
-                const BufView cpar = lvl_buf(L_PAR, nxt, sizeof(int) * (size_t)tot);
-                const BufView cp1 = lvl_buf(L_P1PAR, nxt, sizeof(int) * (size_t)tot);
-                hipLaunchKernelGGL(child_write_range, grid256(p1 - p0), dim3(256), 0, st, drec.as<const DevRecord>(),
-                                   dsets.as<const int>(), doff.as<const int>(), p0, p1 - p0, kw, nxt, in.n_c,
-                                   csets.as<int>(), cpar.as<int>(), cp1.as<int>());
-                HIP_OK(hipGetLastError());
+                const BufView droff = lvl_buf(L_ROFF, level, sizeof(int) * (size_t)n);
+                upload(droff.p, hoff.data(), sizeof(int) * hoff.size());
                 HIP_OK(hipStreamSynchronize(st));  // hoff is read by the copy above
-                if (!process(nxt, (int)tot, csets, cpar, cp1, fs, os, base)) return false;
+                if (!descend(p0, p1 - p0, tot, droff.as<const int>())) return false;
             }
             p0 = p1;
         }
@@ -1348,31 +1353,15 @@ struct Run {
             fin_lvl.assign(nl, {});
             n_lvl.assign(nl, 0);
             probe_opt = probe_fb = 0;
-            if (!keep_rec) {
-                const BufView dsum = A.get(K_SUM, -1, sizeof(unsigned long long) * 8 * (size_t)nl);
-                hipLaunchKernelGGL(fill_i32, grid256(16LL * nl), dim3(256), 0, st, dsum.as<int>(), 16 * nl, 0);
-                HIP_OK(hipGetLastError());
-            }
             // level 0: the empty set
             A.begin_level(0);
-            std::vector<int> h(kw + 2, -1);
             const BufView s0 = lvl_buf(L_SETS, 0, sizeof(int) * kw);
             const BufView p0 = lvl_buf(L_PAR, 0, sizeof(int));
             const BufView q0 = lvl_buf(L_P1PAR, 0, sizeof(int));
-            upload(s0.p, h.data(), s0.n);
-            upload(p0.p, h.data(), sizeof(int));
-            upload(q0.p, h.data(), sizeof(int));
-            HIP_OK(hipStreamSynchronize(st));
+            hipLaunchKernelGGL(level0_write, dim3(1), dim3(64), 0, st, s0.as<int>(), kw, p0.as<int>(), q0.as<int>());
+            HIP_OK(hipGetLastError());
             if (process(0, 1, s0, p0, q0, BufView{}, BufView{}, 0)) break;
             mixed = false;  // too ill-conditioned for FP32 pivots: FP64 throughout
-        }
-        if (!keep_rec) {
-            const int nl = last_lvl + 1;
-            std::vector<unsigned long long> hs(8 * (size_t)nl);
-            const BufView dsum = A.get(K_SUM, -1, sizeof(unsigned long long) * 8 * (size_t)nl);
-            HIP_OK(hipMemcpyAsync(hs.data(), dsum.p, sizeof(unsigned long long) * hs.size(), hipMemcpyDeviceToHost, st));
-            HIP_OK(hipStreamSynchronize(st));
-            for (int L = 0; L <= std::min(k_max, last_lvl); ++L) sum_stats(&hs[8 * (size_t)L]);
         }
         C.stats.precision_used = mixed ? MPQP_MIXED : MPQP_FP64;
         C.stats.tableau_global = (gt64 ? 1 : 0) | (gt32 ? 2 : 0);
@@ -1437,7 +1426,13 @@ Output run_call_ctx(Ctx &C, const Input &in, Arena &A, bool noalloc, bool many =
     if (noalloc || many) o.record = 0;
     A.begin_call();
     Run r(C, o, A, in, noalloc);
-    r.run();
+    try {
+        r.run();
+    } catch (...) {
+        // the inputs, the host vectors and the mailbox outlive what is queued
+        hipStreamSynchronize(C.stream);
+        throw;
+    }
     return r.out;
 }
 
@@ -1511,6 +1506,7 @@ int run_many(const MpqpProblem *pr, int n, int reserved_memory, int workers, GPU
         c.device = M.device;
         HIP_OK(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
         for (hipEvent_t &e : c.ev) HIP_OK(hipEventCreate(&e));
+        c.mail = M.worker_mail(&c - wc.data());
         c.opt = o;
         c.opt_set = true;
         c.lds_limit = M.lds_limit;
@@ -1556,6 +1552,7 @@ int run_many(const MpqpProblem *pr, int n, int reserved_memory, int workers, GPU
         hipStreamDestroy(wc[w].stream);
         wc[w].stream = nullptr;
     }
+    M.trim_mail();
     M.stats = st;
     M.last_feas_nt = wc[0].last_feas_nt;
     M.last_opt_nt = wc[0].last_opt_nt;
