@@ -537,8 +537,8 @@ struct Run {
     int w32 = 2, w64 = 1;                // workgroups per CU a split tableau is sized for
     size_t gtab64_max = 0, gtab32_max = 0;  // global rows of the largest variant
     const void *fn64 = nullptr, *fn32 = nullptr;
-    const RegConfig *reg32 = nullptr;  // FP32 tableau in registers (null: LDS, or split)
-    int nt32 = OPT_NT, np32 = 1;       // threads of the FP32 kernel; its stage passes
+    const RegConfig *reg32 = nullptr, *reg64 = nullptr;  // tableau in registers (null: LDS, or split)
+    int nt32 = OPT_NT, nt64 = OPT_NT, np32 = 1;          // threads of the kernels; FP32 stage passes
     bool tune_pending = false;
     std::vector<int> tkey;
     double *G = nullptr;
@@ -771,6 +771,7 @@ struct Run {
         gt32 = opt_lds_bytes_t<float>(M2, K2, N2, true, M2 + 1) > budget;
         select_reg();
         if (reg32) gt32 = false;
+        if (reg64) gt64 = false;
         S = red_slots(std::max(M2, N2 - in.n_eqs));
         feas_nt = feas_threads_for(M1, K1);
         // 1024 threads only where every optimality kernel of the call splits its tableau
@@ -813,6 +814,7 @@ struct Run {
     std::vector<std::vector<int>> split_variants() const {
         const bool tuned_split = o.precision == MPQP_MIXED ? gt32 : gt64;
         if (reg32) return {{512, w32, w64}};  // one shape; only the FP64 re-solve takes the size
+        if (reg64 && o.precision != MPQP_MIXED) return {{512, w32, w64}};
         if (!tuned_split) {
             // an LDS tableau; the FP64 re-solve of a mixed run may split its own
             if (o.precision == MPQP_MIXED && gt64) return {{512, w32, w64}};
@@ -822,22 +824,34 @@ struct Run {
         return {{512, 2, 2}, {512, 1, 1}, {1024, 1, 1}};
     }
 
-    // The FP32 tableau in registers when a configuration holds it, except one
+    // The tableau in registers when a configuration holds it.  FP32 except one
     // of a single wave's rows, which has little to pivot in parallel: the LDS
     // kernel took 0.39 ms for 1,249 LPs of 40 x 24 against 0.45, and 0.95
-    // against 0.82 for 12,464 LPs of 63 x 37.  A caller that names workgroup
-    // sizes gets the LDS and split kernels they are for.
+    // against 0.82 for 12,464 LPs of 63 x 37.  FP64 at every size: 0.27 ms
+    // against the LDS kernel's 0.29 for those of 40 x 24, 0.61 against 0.83
+    // for 63 x 37, 8.5 against 17.0 for 39,774 of 171 x 102; 27.7 against the
+    // split kernel's 42.5 for 70,376 of 197 x 115, 31.8 against 71.7 for 7,261
+    // of 325 x 194.  A caller that names workgroup sizes gets the LDS and
+    // split kernels they are for.
     void select_reg() {
-        reg32 = nullptr;
-        if (o.precision != MPQP_MIXED || o.opt_threads != 0 || o.split_wgs != 0) return;
-        if (in.M2 <= 44) return;
+        reg32 = reg64 = nullptr;
+        if (o.opt_threads != 0 || o.split_wgs != 0) return;
+        for (const RegConfig &c : reg_configs()) {
+            if (c.fp32 || in.M2 > c.rows() || K2 > c.columns() || P.Nn > 64 * c.sn) continue;
+            const long long b = reg64_lds_bytes(c.nw, c.rw, c.cs, c.lw, in.M2, K2, in.N2);
+            if (b > C.lds_limit / c.wgs() - 1024) continue;
+            reg64 = &c;
+            lds64 = b;
+            break;
+        }
+        if (o.precision != MPQP_MIXED || in.M2 <= 44) return;
         // its use counts share a word with a position
         if (o.max_iter_phase1 >= 1 << 20 || o.max_iter_phase2 >= 1 << 20) return;
         for (const RegConfig &c : reg_configs()) {
-            if (in.M2 > c.rows() || K2 > c.columns() || P.Nn > 64 * c.sn) continue;
+            if (!c.fp32 || in.M2 > c.rows() || K2 > c.columns() || P.Nn > 64 * c.sn) continue;
             // as few passes through the LDS stage as its share of a CU allows
             for (int np = 1; np <= c.nw; np *= 2) {
-                const long long b = reg_lds_bytes(c.nw, c.rw, c.cs, in.M2, K2, in.N2, true, np);
+                const long long b = reg_lds_bytes(c.nw, c.rw, c.cs, in.M2, K2, in.N2, np);
                 if (b <= C.lds_limit / c.wgs() - 1024) {
                     reg32 = &c;
                     np32 = np;
@@ -854,7 +868,7 @@ struct Run {
         w64 = ws64;
         R64 = gt64 ? split_rows_for<double>(M2, K2, N2, false, C.lds_limit / w64 - 512) : M2;
         R32 = gt32 ? split_rows_for<float>(M2, K2, N2, true, C.lds_limit / w32 - 512) : M2;
-        lds64 = opt_lds_bytes_t<double>(M2, K2, N2, false, gt64 ? R64 + 1 : M2 + 1);
+        if (!reg64) lds64 = opt_lds_bytes_t<double>(M2, K2, N2, false, gt64 ? R64 + 1 : M2 + 1);
         if (!reg32) lds32 = opt_lds_bytes_t<float>(M2, K2, N2, true, gt32 ? R32 + 1 : M2 + 1);
         select_opt(nt);
     }
@@ -873,17 +887,18 @@ struct Run {
         if (nt == 256 && any_split) nt = 512;
         if (nt == 1024 && !all_split) nt = 512;
         opt_nt = nt;
-        fn64 = opt_fn(false, opt_nt, S, gt64);
+        fn64 = reg64 ? reg64->fn : opt_fn(false, opt_nt, S, gt64);
         fn32 = !mx ? nullptr : (reg32 ? reg32->fn : opt_fn(true, opt_nt, S, gt32));
         nt32 = reg32 ? reg32->threads() : opt_nt;
-        cap64 = capacity(fn64, opt_nt, lds64);
+        nt64 = reg64 ? reg64->threads() : opt_nt;
+        cap64 = capacity(fn64, nt64, lds64);
         cap32 = o.precision == MPQP_MIXED ? capacity(fn32, nt32, lds32) : 0;
     }
 
     void launch_opt(const void *fn, int grid, long long lds, OptArgs &oa) {
         void *args[] = {&oa};
         oa.stage_passes = np32;
-        HIP_OK(hipLaunchKernel(fn, dim3(grid), dim3(fn == fn32 ? nt32 : opt_nt), args, (size_t)lds, st));
+        HIP_OK(hipLaunchKernel(fn, dim3(grid), dim3(fn == fn32 ? nt32 : nt64), args, (size_t)lds, st));
     }
 
     // device bytes a candidate of `level` needs in its chunk

@@ -11,17 +11,25 @@
 
 template <int P>
 struct Part;
-#define MPQP_PICK(part, nw_, rw_, cs_, ex_, sn_, eu_)                                                  \
+#define MPQP_PICK(part, fp32_, nw_, rw_, lw_, cs_, ex_, sn_, eu_)                                      \
     template <>                                                                                        \
     struct Part<part> {                                                                                \
-        static constexpr int nw = nw_, rw = rw_, cs = cs_, ex = ex_, sn = sn_, eu = eu_;               \
+        static constexpr bool fp32 = fp32_;                                                            \
+        static constexpr int nw = nw_, rw = rw_, lw = lw_, cs = cs_, ex = ex_, sn = sn_, eu = eu_;     \
     };
 MPQP_REG_PARTS(MPQP_PICK)
 
+template <typename P>
+static const void *reg_fn() {
+    if constexpr (P::fp32)
+        return reinterpret_cast<const void *>(&reg_kernel32<P::nw, P::rw, P::cs, P::ex, P::sn, P::eu>);
+    else
+        return reinterpret_cast<const void *>(&reg_kernel64<P::nw, P::rw, P::cs, P::ex, P::lw, P::sn, P::eu>);
+}
+
 RegConfig MPQP_CAT(reg_config_part, MPQP_PART)() {
     typedef Part<MPQP_PART> P;
-    return RegConfig{P::nw, P::rw, P::cs, P::ex, P::sn, P::eu,
-                     reinterpret_cast<const void *>(&reg_kernel32<P::nw, P::rw, P::cs, P::ex, P::sn, P::eu>)};
+    return RegConfig{P::fp32, P::nw, P::rw, P::lw, P::cs, P::ex, P::sn, P::eu, reg_fn<P>()};
 }
 
 #else

@@ -20,20 +20,27 @@
 MPQP_OPT_PARTS(MPQP_DECL)
 #undef MPQP_DECL
 
-// Kernels with the FP32 tableau in registers (parts 8 ..): waves per
-// workgroup, rows per wave, column slots, extra columns, reduction slots over
-// the Nn variables, waves per SIMD of the register budget (512 / that many
-// registers a lane).
-#define MPQP_REG_PARTS(X)          \
-    X(8, 2, 44, 1, 4, 3, 4)        \
-    X(9, 2, 64, 1, 8, 4, 3)        \
-    X(10, 4, 44, 2, 0, 4, 3)       \
-    X(11, 4, 64, 2, 8, 6, 2)       \
-    X(12, 8, 44, 3, 4, 6, 2)       \
-    X(13, 8, 44, 4, 0, 6, 2)
+// Kernels with the tableau in registers (parts 8 ..): FP32 or FP64, waves per
+// workgroup, rows per wave, of these in LDS (FP64), column slots, extra
+// columns, reduction slots over the Nn variables, waves per SIMD of the
+// register budget (512 / that many registers a lane).
+#define MPQP_REG_PARTS(X)                  \
+    X(8, true, 2, 44, 0, 1, 4, 3, 4)       \
+    X(9, true, 2, 64, 0, 1, 8, 4, 3)       \
+    X(10, true, 4, 44, 0, 2, 0, 4, 3)      \
+    X(11, true, 4, 64, 0, 2, 8, 6, 2)      \
+    X(12, true, 8, 44, 0, 3, 4, 6, 2)      \
+    X(13, true, 8, 44, 0, 4, 0, 6, 2)      \
+    X(14, false, 2, 24, 0, 1, 0, 3, 4)     \
+    X(15, false, 2, 40, 0, 1, 0, 3, 3)     \
+    X(16, false, 4, 32, 0, 1, 8, 4, 3)     \
+    X(17, false, 4, 44, 0, 2, 0, 4, 2)     \
+    X(18, false, 8, 32, 0, 2, 8, 6, 2)     \
+    X(19, false, 8, 42, 11, 3, 4, 6, 2)
 
 struct RegConfig {
-    int nw, rw, cs, ex, sn, eu;
+    bool fp32;
+    int nw, rw, lw, cs, ex, sn, eu;
     const void *fn;
     int rows() const { return nw * rw; }
     int columns() const { return 64 * cs + ex; }

@@ -1,7 +1,7 @@
-// reg_kernel.hpp — the FP32 optimality LP (mixed precision) with its tableau
-// in registers, pivoted by the matrix cores.
+// reg_kernel.hpp — the optimality LP with its tableau in registers: FP32
+// (mixed precision) pivoted by the matrix cores, FP64 by the vector unit.
 //
-// One LP per workgroup of NW waves.  Wave w holds the rows w * RW ..
+// FP32.  One LP per workgroup of NW waves.  Wave w holds the rows w * RW ..
 // w * RW + RW - 1 of the condensed tableau, lane l of slot s the column
 // l + 64 s (CS slots): a block of four rows of a slot is the accumulator of
 // v_mfma_f32_4x4x1_16b_f32 with its A operand broadcast from one block (16
@@ -21,6 +21,22 @@
 // wave.  Each wave knows its smallest basic value after a pivot, so the
 // leaving row costs one exchange of NW values; the wave that holds it runs
 // the ratio test on its registers and publishes the divided row in LDS.
+//
+// FP64.  The same layout with a register pair per entry; of a wave's rows the
+// last LW may lie in its part of LDS, lane = column as well (336 x 196 doubles
+// are 512 KB: all of a CU's registers, or 3/4 of them and 132 KB of LDS).
+// The matrix unit has no FP64 form with a broadcast operand and no higher FP64
+// rate, so a pivot takes column q out of the pivot lane into scalar registers
+// (two lane reads a row) and is one v_fma_f64 per row and slot.
+//
+// What bounds both: with the tableau out of LDS and of global memory, the
+// chain of a pivot - leaving row, entering column, division, factors - at two
+// waves per SIMD, about 9,000 cycles in FP64 and 10,000 in FP32 at
+// n=60 m=120 p=12.  The LDS and split kernels (opt_kernel.hpp) spend the same
+// chain and a pass over the tableau: n=60 m=120 p=12 |S|<=3 mixed 822 -> 571 ms
+// with the FP32 tableau and -> 486 ms with the re-solves' FP64 too; FP64
+// |S|<=2 at that size 57 -> 25 ms of kernel time, n=30 m=62 p=8 |S|<=3 18.4
+// -> 8.5 ms, n=6 m=28 p=4 |S|<=6 6.4 -> 3.1 ms.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -68,23 +84,50 @@ __device__ __forceinline__ int opaque(int x) {
 __device__ __forceinline__ float lane_get(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
+__device__ __forceinline__ double lane_get(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+// v with lane l's value replaced by the uniform x (the compiler has no
+// builtin of the instruction's name: its intrinsic, by name)
+extern "C" __device__ __attribute__((const)) int mpqp_writelane(int x, int l, int v) __asm("llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ double lane_set(double v, int l, double x) {
+    return __hiloint2double(mpqp_writelane(__double2hiint(x), l, __double2hiint(v)),
+                            mpqp_writelane(__double2loint(x), l, __double2loint(v)));
+}
 
 // Minimum over the wave of values that are not NaN, known to every lane:
 // v_min with DPP row shifts, then the row broadcasts of lanes 15 and 31, into
 // lane 63 (six dependent instructions; lane shifts with compare and select
 // took four times as long).
 template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_min(float v) {
-    const int i = __float_as_int(v);
-    return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false)));
+__device__ __forceinline__ float dpp_get(float old, float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, ROWS, 0xf, false));
 }
-__device__ __forceinline__ float row8_min_f(float v) {  // into lane 7, of lanes 0 .. 7
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_get(double old, double v) {
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, ROWS, 0xf, false),
+        __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float min_r(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ float max_r(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ double min_r(double a, double b) { return fmin(a, b); }
+__device__ __forceinline__ double max_r(double a, double b) { return fmax(a, b); }
+template <int CTRL, int ROWS, typename Re>
+__device__ __forceinline__ Re dpp_min(Re v) {
+    return min_r(v, dpp_get<CTRL, ROWS>(v, v));
+}
+template <typename Re>
+__device__ __forceinline__ Re row8_min(Re v) {  // into lane 7, of lanes 0 .. 7
     v = dpp_min<0x111, 0xf>(v);
     v = dpp_min<0x112, 0xf>(v);
     return dpp_min<0x114, 0xf>(v);
 }
-__device__ __forceinline__ float wave_min_f(float v) {
-    v = row8_min_f(v);
+template <typename Re>
+__device__ __forceinline__ Re wave_min(Re v) {
+    v = row8_min(v);
     v = dpp_min<0x118, 0xf>(v);
     v = dpp_min<0x142, 0xa>(v);
     v = dpp_min<0x143, 0xc>(v);
@@ -93,21 +136,21 @@ __device__ __forceinline__ float wave_min_f(float v) {
 
 // The two smallest of the wave's values (not NaN; equal ones count twice),
 // known to every lane, in one pass.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ void dpp_min2(float &a, float &b) {
-    const int inf = 0x7f800000;
-    const float oa = __int_as_float(__builtin_amdgcn_update_dpp(inf, __float_as_int(a), CTRL, ROWS, 0xf, false));
-    const float ob = __int_as_float(__builtin_amdgcn_update_dpp(inf, __float_as_int(b), CTRL, ROWS, 0xf, false));
-    b = fminf(fminf(b, ob), fmaxf(a, oa));
-    a = fminf(a, oa);
+template <int CTRL, int ROWS, typename Re>
+__device__ __forceinline__ void dpp_min2(Re &a, Re &b) {
+    const Re oa = dpp_get<CTRL, ROWS>((Re)INFINITY, a), ob = dpp_get<CTRL, ROWS>((Re)INFINITY, b);
+    b = min_r(min_r(b, ob), max_r(a, oa));
+    a = min_r(a, oa);
 }
-__device__ __forceinline__ void row8_min2_f(float &a, float &b) {  // into lane 7, of lanes 0 .. 7
+template <typename Re>
+__device__ __forceinline__ void row8_min2(Re &a, Re &b) {  // into lane 7, of lanes 0 .. 7
     dpp_min2<0x111, 0xf>(a, b);
     dpp_min2<0x112, 0xf>(a, b);
     dpp_min2<0x114, 0xf>(a, b);
 }
-__device__ __forceinline__ void wave_min2_f(float &a, float &b) {
-    row8_min2_f(a, b);
+template <typename Re>
+__device__ __forceinline__ void wave_min2(Re &a, Re &b) {
+    row8_min2(a, b);
     dpp_min2<0x118, 0xf>(a, b);
     dpp_min2<0x142, 0xa>(a, b);
     dpp_min2<0x143, 0xc>(a, b);
@@ -151,6 +194,23 @@ __device__ __forceinline__ int tree32(float (&v)[S], int (&pk)[S], int n, int la
     return rfl(pk[0]);
 }
 
+// The reference tree over values of either type: id of the element it keeps
+// (ids below 1024, negative: no element), its value in v[0] of lane 0.
+template <int S, typename Pred>
+__device__ __forceinline__ int reg_tree(float (&v)[S], int (&id)[S], int (&cn)[S], int n, int lane, Pred pred) {
+    int pk[S];
+    reg_for<S>([&](auto s) MPQP_INL { pk[s] = id[s] < 0 ? -1 : cn[s] << 10 | id[s]; });
+    const int w = tree32<S>(v, pk, n, lane, [&](float vt, int pt, float vu, int pu) {
+        return pred((double)vt, pt, pt >> 10, (double)vu, pu, pu >> 10);
+    });
+    return w < 0 ? -1 : w & 1023;
+}
+template <int S, typename Pred>
+__device__ __forceinline__ int reg_tree(double (&v)[S], int (&id)[S], int (&cn)[S], int n, int lane, Pred pred) {
+    tree_argmin_s<S>(v, id, cn, n, lane, pred);
+    return rfl(id[0]);
+}
+
 // Of the elements (lane + 64 s, s < S) whose lanes are set in hit[s], the one
 // that a reference tree keeps when it replaces an element only by a strictly
 // smaller one and these are the minima: the combines run from the largest
@@ -183,27 +243,47 @@ __device__ __forceinline__ int tree_first(const unsigned long long (&hit)[S]) {
 // Rows past M repeat row M - 1, and the columns of a slot past K repeat
 // column 0: nothing reads them, and no entry depends on another row or column
 // than its own.
-template <int NW, int RW, int CS, int EX>
+//
+// FP64: the same, with the vector unit (T = fma(-f, pr, T) with the row's
+// factor in scalar registers) and, of a wave's RW rows, the last LW in its
+// part of LDS, lane = column as well.
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
 struct RegTab {
-    static_assert(RW % 4 == 0 && RW <= MPQP_WAVE, "blocks of four rows, one lane per row");
-    static constexpr int NB = RW / 4;
+    static_assert(RW <= MPQP_WAVE, "one lane per row");
+    static_assert(sizeof(Re) == 8 || (RW % 4 == 0 && LW == 0), "FP32: blocks of four rows");
+    static constexpr int RR = RW - LW;
     static constexpr int NS = CS + (EX > 0 ? 1 : 0);  // slots of a decision
-    v4f t[NB][CS];
-    float d[NS];       // cost row (the same in every wave)
-    float xs[EX + 2];  // by row (lanes < RW): the extra columns, the rhs, the perturbation
-    __device__ __forceinline__ float x() const { return xs[EX]; }
-    __device__ __forceinline__ float xp() const { return xs[EX + 1]; }
+    typedef std::conditional_t<sizeof(Re) == 4, v4f, Re> cell;
+    cell t[sizeof(Re) == 4 ? RW / 4 : RR][CS];
+    Re d[NS];       // cost row (the same in every wave)
+    Re xs[EX + 2];  // by row (lanes < RW): the extra columns, the rhs, the perturbation
+    Re *lt;         // this lane's column of the wave's LDS rows
+    __device__ __forceinline__ Re x() const { return xs[EX]; }
+    __device__ __forceinline__ Re xp() const { return xs[EX + 1]; }
+    template <int I, int S>
+    __device__ __forceinline__ Re get() const {
+        if constexpr (sizeof(Re) == 4) return t[I / 4][S][I % 4];
+        else if constexpr (I < RR) return t[I][S];
+        else return lt[((I - RR) * CS + S) * MPQP_WAVE];
+    }
+    template <int I, int S>
+    __device__ __forceinline__ void set(Re v) {
+        if constexpr (sizeof(Re) == 4) t[I / 4][S][I % 4] = v;
+        else if constexpr (I < RR) t[I][S] = v;
+        else lt[((I - RR) * CS + S) * MPQP_WAVE] = v;
+    }
 };
 
 // Per-wave results of the distributed decisions.
+template <typename Re>
 struct RegMin {
-    float m1, m2;  // smallest and second smallest x_B of the wave
-    int at, nan;   // row of the smallest; a NaN among them
+    Re m1, m2;    // smallest and second smallest x_B of the wave
+    int at, nan;  // row of the smallest; a NaN among them
 };
-template <int NW>
+template <typename Re, int NW>
 struct RegShared {
-    __attribute__((aligned(16))) RegMin min[NW];
-    float cmax[NW], rv[NW];
+    __attribute__((aligned(16))) RegMin<Re> min[NW];
+    Re cmax[NW], rv[NW];
     int rk[NW];
 };
 
@@ -213,35 +293,45 @@ struct RegShared {
 // nonbasic e-list; a stage of `rp` rows for the steps that read the tableau
 // against its layout (lambda swap, certification): np passes of NW / np
 // waves' rows each.
-__host__ __device__ inline long long reg_lds_bytes(int nw, int rw, int cs, int M, int K, int N2, bool cert, int np) {
+__host__ __device__ inline long long reg_lds_bytes(int nw, int rw, int cs, int M, int K, int N2, int np) {
     const long long mr = (long long)nw * rw, kc = 64LL * (cs + 1);
     long long b = (2 * kc + 3 * mr) * (long long)sizeof(float);
     b = (b + 15) & ~15LL;
     b += (3LL * N2 + 2 * M + K) * 4;
-    if (cert) b = ((b + 7) & ~7LL) + 2LL * M * 8 + 2LL * (M + 1) * 4;
+    b = ((b + 7) & ~7LL) + 2LL * M * 8 + 2LL * (M + 1) * 4;
     b = (b + 15) & ~15LL;
     b += mr / np * (K | 1) * (long long)sizeof(float);
     return (b + 15) & ~15LL;
 }
+// FP64: no certification and no stage; the LDS rows
+__host__ __device__ inline long long reg64_lds_bytes(int nw, int rw, int cs, int lw, int M, int K, int N2) {
+    const long long mr = (long long)nw * rw, kc = 64LL * (cs + 1);
+    long long b = ((long long)nw * lw * cs * 64 + 2 * kc + 3 * mr) * (long long)sizeof(double);
+    b += (3LL * N2 + 2 * M + K) * 4;
+    return (b + 15) & ~15LL;
+}
 
-template <int NW, int RW, int CS, int EX>
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
 struct RegLds {
     static constexpr int MR = NW * RW, KC = MPQP_WAVE * (CS + 1);
-    float *ep, *gx, *gp, *colx, *dl, *stage;
+    Re *ep, *gx, *gp, *colx, *dl, *rows_lds;
+    float *stage;
     int *basis, *nonb, *where, *bcnt, *nbcnt, *rows;
     double *cx, *cr, *xv;
     int *elr, *els;
     int sld, np, rp;
-    __device__ void carve(unsigned char *smem, int M, int K, int N2, bool cert, int np_) {
+    __device__ void carve(unsigned char *smem, int M, int K, int N2, int np_) {
+        constexpr size_t LT = (size_t)NW * LW * CS * MPQP_WAVE;
         np = np_;
-        rp = MR / np;
+        rp = sizeof(Re) == 4 ? MR / np : 0;
         sld = K | 1;
-        ep = reinterpret_cast<float *>(smem);
+        rows_lds = reinterpret_cast<Re *>(smem);
+        ep = rows_lds + LT;
         gx = ep + KC;
         gp = gx + MR;
         colx = gp + MR;
         dl = colx + MR;
-        size_t b = (size_t)(2 * KC + 3 * MR) * sizeof(float);
+        size_t b = (LT + 2 * KC + 3 * MR) * sizeof(Re);
         b = (b + 15) & ~(size_t)15;
         bcnt = reinterpret_cast<int *>(smem + b);
         nbcnt = bcnt + N2;
@@ -253,27 +343,28 @@ struct RegLds {
         cx = cr = nullptr;
         elr = els = nullptr;
         xv = reinterpret_cast<double *>(bcnt);
-        if (cert) {
+        stage = nullptr;
+        if constexpr (sizeof(Re) == 4) {
             b = (b + 7) & ~(size_t)7;
             cx = reinterpret_cast<double *>(smem + b);
             cr = cx + M;
             elr = reinterpret_cast<int *>(cr + M);
             els = elr + M + 1;
             b += (size_t)2 * M * 8 + (size_t)2 * (M + 1) * 4;
+            b = (b + 15) & ~(size_t)15;
+            stage = reinterpret_cast<float *>(smem + b);
         }
-        b = (b + 15) & ~(size_t)15;
-        stage = reinterpret_cast<float *>(smem + b);
     }
-    __device__ __forceinline__ float rhs_of(int i) const { return gx[i]; }
-    __device__ __forceinline__ float cost_of(int k) const { return dl[k]; }
+    __device__ __forceinline__ Re rhs_of(int i) const { return gx[i]; }
+    __device__ __forceinline__ Re cost_of(int k) const { return dl[k]; }
 };
 
 __device__ __forceinline__ int wave_id() { return rfl((int)(threadIdx.x / MPQP_WAVE)); }
 
 // The wave's rows into the stage, pass h (waves [h, h + 1) * NW / np); the
 // caller's barriers surround it.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_dump(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, int K, int h) {
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_dump(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int K, int h) {
     const int wave = wave_id(), lane = fresh_lane();
     const int w0 = h * (NW / L.np);
     if (wave >= w0 && wave < w0 + NW / L.np) {
@@ -283,7 +374,7 @@ __device__ __forceinline__ void reg_dump(const RegTab<NW, RW, CS, EX> &R, const 
             if (c < K) {
                 float *dc = dst + c;
                 reg_for<RW>([&](auto i) MPQP_INL {
-                    *dc = R.t[i / 4][s][i % 4];
+                    *dc = R.template get<decltype(i)::value, decltype(s)::value>();
                     dc += L.sld;
                 });
             }
@@ -297,7 +388,7 @@ __device__ __forceinline__ void reg_dump(const RegTab<NW, RW, CS, EX> &R, const 
 
 // T -= f (by row) x v (by column) in slot s, every block of rows
 template <int S, int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_rank1(RegTab<NW, RW, CS, EX> &R, float nf, float v) {
+__device__ __forceinline__ void reg_rank1(RegTab<float, NW, RW, CS, EX, 0> &R, float nf, float v) {
     reg_for<RW / 4>([&](auto b) MPQP_INL {
         R.t[b][S] = __builtin_amdgcn_mfma_f32_4x4x1f32(nf, v, R.t[b][S], 4, decltype(b)::value, 0);
     });
@@ -306,52 +397,74 @@ __device__ __forceinline__ void reg_rank1(RegTab<NW, RW, CS, EX> &R, float nf, f
 // Column q of the wave's rows by lane, through the wave's part of L.colx (a
 // wave's LDS operations stay in order).  CLEAR: the column is left zero
 // (T - f * 1 in its lane), if `on`.
-template <bool CLEAR, int NW, int RW, int CS, int EX, typename RT>
-__device__ __forceinline__ float reg_col_op(RT &R, const RegLds<NW, RW, CS, EX> &L, int q, bool on) {
+// FP64: lane by lane through scalar registers (CLEAR is left to reg_apply).
+template <bool CLEAR, typename Re, int NW, int RW, int CS, int EX, int LW, typename RT>
+__device__ __forceinline__ Re reg_col_op(RT &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int q, bool on) {
     const int lane = fresh_lane(), lq = q % MPQP_WAVE;
-    float *cx = L.colx + wave_id() * RW;
-    float v = 0.f;
-    reg_for<CS>([&](auto s) MPQP_INL {
-        if (q / MPQP_WAVE == s) {
-            if (lane == lq)
-                reg_for<RW / 4>([&](auto b) MPQP_INL { *reinterpret_cast<v4f *>(cx + 4 * b) = R.t[b][s]; });
-            __builtin_amdgcn_wave_barrier();
-            v = cx[lane < RW ? lane : 0];
-            if constexpr (CLEAR) reg_rank1<decltype(s)::value>(R, on ? -v : 0.f, lane == lq ? 1.f : 0.f);
-        }
-    });
-    reg_for<EX>([&](auto e) MPQP_INL {
-        const bool at = q == MPQP_WAVE * CS + e;
-        v = at ? R.xs[e] : v;
-        if constexpr (CLEAR) R.xs[e] = at && on ? 0.f : R.xs[e];
-    });
-    __builtin_amdgcn_wave_barrier();
-    return v;
+    Re v = 0;
+    if constexpr (sizeof(Re) == 8) {
+        reg_for<CS>([&](auto s) MPQP_INL {
+            if (q / MPQP_WAVE == s)
+                reg_for<RW>([&](auto i) MPQP_INL {
+                    v = lane_set(v, i, lane_get(R.template get<decltype(i)::value, decltype(s)::value>(), lq));
+                });
+        });
+        reg_for<EX>([&](auto e) MPQP_INL { v = q == MPQP_WAVE * CS + e ? R.xs[e] : v; });
+        return v;
+    } else {
+        float *cx = L.colx + wave_id() * RW;
+        reg_for<CS>([&](auto s) MPQP_INL {
+            if (q / MPQP_WAVE == s) {
+                if (lane == lq)
+                    reg_for<RW / 4>([&](auto b) MPQP_INL { *reinterpret_cast<v4f *>(cx + 4 * b) = R.t[b][s]; });
+                __builtin_amdgcn_wave_barrier();
+                v = cx[lane < RW ? lane : 0];
+                if constexpr (CLEAR) reg_rank1<decltype(s)::value>(R, on ? -v : 0.f, lane == lq ? 1.f : 0.f);
+            }
+        });
+        reg_for<EX>([&](auto e) MPQP_INL {
+            const bool at = q == MPQP_WAVE * CS + e;
+            v = at ? R.xs[e] : v;
+            if constexpr (CLEAR) R.xs[e] = at && on ? 0.f : R.xs[e];
+        });
+        __builtin_amdgcn_wave_barrier();
+        return v;
+    }
 }
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ float reg_col(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, int q) {
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ Re reg_col(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int q) {
     return reg_col_op<false>(R, L, q, false);
 }
 
 // Row `lr` of the wave; al[CS]: its extra columns, rhs and perturbation entry
 // in the first lanes.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_row(const RegTab<NW, RW, CS, EX> &R, int lr, float (&al)[CS + 1]) {
-    const int u = lr % 4;
-    reg_pick<0, RW / 4>(lr / 4, [&](auto b) MPQP_INL {
-        reg_for<CS>([&](auto s) MPQP_INL {
-            const v4f v = R.t[b][s];
-            al[s] = u < 2 ? (u == 0 ? v[0] : v[1]) : (u == 2 ? v[2] : v[3]);
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_row(const RegTab<Re, NW, RW, CS, EX, LW> &R, int lr, Re (&al)[CS + 1]) {
+    if constexpr (sizeof(Re) == 8) {
+        constexpr int RR = RW - LW;
+        if (LW > 0 && lr >= RR)
+            reg_for<CS>([&](auto s) MPQP_INL { al[s] = R.lt[((lr - RR) * CS + s) * MPQP_WAVE]; });
+        else
+            reg_pick<0, RR>(lr, [&](auto i) MPQP_INL {
+                reg_for<CS>([&](auto s) MPQP_INL { al[s] = R.t[i][s]; });
+            });
+    } else {
+        const int u = lr % 4;
+        reg_pick<0, RW / 4>(lr / 4, [&](auto b) MPQP_INL {
+            reg_for<CS>([&](auto s) MPQP_INL {
+                const v4f v = R.t[b][s];
+                al[s] = u < 2 ? (u == 0 ? v[0] : v[1]) : (u == 2 ? v[2] : v[3]);
+            });
         });
-    });
+    }
     const int lane = fresh_lane();
-    al[CS] = 0.f;
+    al[CS] = 0;
     reg_for<EX + 2>([&](auto e) MPQP_INL { al[CS] = lane == e ? lane_get(R.xs[e], lr) : al[CS]; });
 }
 
 // Row `lr` of the wave (its entries al) made zero: T - 1 * al.
 template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_clear_row(RegTab<NW, RW, CS, EX> &R, int lr, const float (&al)[CS + 1]) {
+__device__ __forceinline__ void reg_clear_row(RegTab<float, NW, RW, CS, EX, 0> &R, int lr, const float (&al)[CS + 1]) {
     const float a = fresh_lane() == lr ? -1.f : 0.f;
     // (one test after the other: the branches of a tree would meet with a
     // tableau changed in different places)
@@ -363,38 +476,84 @@ __device__ __forceinline__ void reg_clear_row(RegTab<NW, RW, CS, EX> &R, int lr,
     });
 }
 
+// FP64: row `lr` of the wave := al (blocks of rows for fewer tests)
+template <int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_set_row(RegTab<double, NW, RW, CS, EX, LW> &R, int lr, const double (&al)[CS + 1]) {
+    constexpr int RR = RW - LW, B = 4;
+    if (LW > 0 && lr >= RR)
+        reg_for<CS>([&](auto s) MPQP_INL { R.lt[((lr - RR) * CS + s) * MPQP_WAVE] = al[s]; });
+    reg_for<(RR + B - 1) / B>([&](auto b) MPQP_INL {
+        if (lr / B == b)
+            reg_for<B>([&](auto u) MPQP_INL {
+                constexpr int i = decltype(b)::value * B + decltype(u)::value;
+                if constexpr (i < RR) reg_for<CS>([&](auto s) MPQP_INL { R.t[i][s] = lr == i ? al[s] : R.t[i][s]; });
+            });
+    });
+}
+
 // The pivot row's wave: row lr (al) divided by p into L.ep (1 / p at column
 // q, if any), with its rhs and perturbation entries; the row itself is left
-// zero for reg_apply.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_divide(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, const float (&al)[CS + 1],
-                                           int lr, int q, float p) {
+// zero for reg_apply (FP32).
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_divide(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, const Re (&al)[CS + 1],
+                                           int lr, int q, Re p) {
     const int lane = fresh_lane();
     reg_for<CS + 1>([&](auto s) MPQP_INL {
         const int c = lane + MPQP_WAVE * s;
-        L.ep[c] = (c == q ? 1.f : al[s]) / p;
+        L.ep[c] = (c == q ? (Re)1 : al[s]) / p;
     });
-    reg_clear_row(R, lr, al);
+    if constexpr (sizeof(Re) == 4) reg_clear_row(R, lr, al);
 }
 
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_publish(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, const float (&al)[CS + 1],
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_publish(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, const Re (&al)[CS + 1],
                                             int lr, int q) {
-    float v = al[0];
-    reg_for<RegTab<NW, RW, CS, EX>::NS>([&](auto s) MPQP_INL { v = q / MPQP_WAVE == s ? al[s] : v; });
+    Re v = al[0];
+    reg_for<RegTab<Re, NW, RW, CS, EX, LW>::NS>([&](auto s) MPQP_INL { v = q / MPQP_WAVE == s ? al[s] : v; });
     reg_divide(R, L, al, lr, q, lane_get(v, q % MPQP_WAVE));
 }
 
 // The rank-1 update of the wave's rows by the divided pivot row pr (pr[CS]:
-// extra columns, rhs, perturbation) with the factors fv by lane.  The wave
-// that holds the pivot row r finds it zero: its factor -1 puts pr there.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_apply(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
-                                          const float (&pr)[CS + 1], float fv, int r) {
+// extra columns, rhs, perturbation) with the factors fv by lane.  FP32: the
+// wave that holds the pivot row r finds it zero: its factor -1 puts pr there.
+// FP64: a column whose entry of pr is zero keeps its entries, column q (any,
+// or -1) starts from zero, and the pivot row is put in place.
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_apply(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
+                                          const Re (&pr)[CS + 1], Re fv, int r, int q) {
     const int lane = fresh_lane(), wave = wave_id(), lr = r - wave * RW;
-    const float nf = lane == lr ? 1.f : -fv;
-    reg_for<CS>([&](auto s) MPQP_INL { reg_rank1<decltype(s)::value>(R, nf, pr[s]); });
-    reg_for<EX + 2>([&](auto e) MPQP_INL { R.xs[e] = fma(nf, lane_get(pr[CS], e), lane == lr ? 0.f : R.xs[e]); });
+    if constexpr (sizeof(Re) == 8) {
+        constexpr int CH = 16;  // rows whose factors are in scalar registers at a time
+        reg_for<(RW + CH - 1) / CH>([&](auto h) MPQP_INL {
+            constexpr int i0 = decltype(h)::value * CH, n = RW - i0 < CH ? RW - i0 : CH;
+            Re f[n];
+            reg_for<n>([&](auto i) MPQP_INL { f[i] = lane_get(fv, i0 + decltype(i)::value); });
+            reg_for<CS>([&](auto s) MPQP_INL {
+                constexpr int S = decltype(s)::value;
+                const bool at = lane + MPQP_WAVE * S == q;
+                if (pr[S] != (Re)0 && !at)
+                    reg_for<n>([&](auto i) MPQP_INL {
+                        constexpr int I = i0 + decltype(i)::value;
+                        R.template set<I, S>(fma(-f[i], pr[S], R.template get<I, S>()));
+                    });
+                if (at)
+                    reg_for<n>([&](auto i) MPQP_INL {
+                        constexpr int I = i0 + decltype(i)::value;
+                        R.template set<I, S>(fma(-f[i], pr[S], (Re)0));
+                    });
+            });
+        });
+        if ((unsigned)lr < (unsigned)RW) reg_set_row(R, lr, pr);
+        reg_for<EX + 2>([&](auto e) MPQP_INL {
+            const Re p = lane_get(pr[CS], e), x0 = q == MPQP_WAVE * CS + e && e < EX ? (Re)0 : R.xs[e];
+            const Re xn = p != (Re)0 ? fma(-fv, p, x0) : x0;
+            R.xs[e] = lane == lr ? p : xn;
+        });
+    } else {
+        const float nf = lane == lr ? 1.f : -fv;
+        reg_for<CS>([&](auto s) MPQP_INL { reg_rank1<decltype(s)::value>(R, nf, pr[s]); });
+        reg_for<EX + 2>([&](auto e) MPQP_INL { R.xs[e] = fma(nf, lane_get(pr[CS], e), lane == lr ? 0.f : R.xs[e]); });
+    }
     if (lane < RW) {
         L.gx[wave * RW + lane] = R.x();
         L.gp[wave * RW + lane] = R.xp();
@@ -405,38 +564,38 @@ __device__ __forceinline__ void reg_apply(RegTab<NW, RW, CS, EX> &R, const RegLd
 // included.  Barriers before (L.ep written) and after belong to the caller.
 // MAYBE: r < 0 leaves everything as it is (a branch around the update would
 // give the tableau's registers two states to be merged).
-template <bool MAYBE = false, int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_update(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, int r, int q) {
+template <bool MAYBE = false, typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_update(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int r, int q) {
     const int lane = fresh_lane();
     const bool off = MAYBE && r < 0;
-    float fv = reg_col_op<true>(R, L, q, !off);
-    float pr[CS + 1], dv = 0.f;
+    Re fv = reg_col_op<true>(R, L, q, !off);
+    Re pr[CS + 1], dv = 0;
     reg_for<CS + 1>([&](auto s) MPQP_INL {
         pr[s] = L.ep[lane + MPQP_WAVE * s];
-        if constexpr (MAYBE) pr[s] = off ? 0.f : pr[s];
+        if constexpr (MAYBE) pr[s] = off ? (Re)0 : pr[s];
     });
-    if constexpr (MAYBE) fv = off ? 0.f : fv;
-    constexpr int NS = RegTab<NW, RW, CS, EX>::NS;
+    if constexpr (MAYBE) fv = off ? (Re)0 : fv;
+    constexpr int NS = RegTab<Re, NW, RW, CS, EX, LW>::NS;
     reg_for<NS>([&](auto s) MPQP_INL { dv = q / MPQP_WAVE == s ? R.d[s] : dv; });
-    const float fd = lane_get(dv, q % MPQP_WAVE);
+    const Re fd = lane_get(dv, q % MPQP_WAVE);
     reg_for<NS>([&](auto s) MPQP_INL {
-        const float d0 = lane + MPQP_WAVE * s == q && !off ? 0.f : R.d[s];
-        R.d[s] = pr[s] != 0.f ? fma(-fd, pr[s], d0) : d0;
+        const Re d0 = lane + MPQP_WAVE * s == q && !off ? (Re)0 : R.d[s];
+        R.d[s] = pr[s] != (Re)0 ? fma(-fd, pr[s], d0) : d0;
     });
-    reg_apply(R, L, pr, fv, off ? -MPQP_WAVE * NW : r);
+    reg_apply(R, L, pr, fv, off ? -MPQP_WAVE * NW : r, off ? -1 : q);
 }
 
 // Cost row d = init(column) - c * (sum of the rows whose basic variable
 // satisfies sel), rows ascending: the waves that hold such rows continue the
 // chain one after the other through L.dl.
-template <int NW, int RW, int CS, int EX, typename SelF, typename InitF>
-__device__ __forceinline__ void reg_cost(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, int M, int K,
-                                         float c, SelF sel, InitF init) {
-    constexpr int NS = RegTab<NW, RW, CS, EX>::NS;
+template <typename Re, int NW, int RW, int CS, int EX, int LW, typename SelF, typename InitF>
+__device__ __forceinline__ void reg_cost(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int M, int K,
+                                         Re c, SelF sel, InitF init) {
+    constexpr int NS = RegTab<Re, NW, RW, CS, EX, LW>::NS;
     const int lane = fresh_lane(), wave = wave_id();
     reg_for<NS>([&](auto s) MPQP_INL {
         const int col = lane + MPQP_WAVE * s;
-        R.d[s] = col < K ? init(col) : 0.f;
+        R.d[s] = col < K ? (Re)init(col) : (Re)0;
     });
     bool started = false;
     for (int w = 0; w < NW; ++w) {
@@ -448,9 +607,9 @@ __device__ __forceinline__ void reg_cost(RegTab<NW, RW, CS, EX> &R, const RegLds
                 reg_for<NS>([&](auto s) MPQP_INL { R.d[s] = L.dl[lane + MPQP_WAVE * s]; });
             reg_for<RW>([&](auto i) MPQP_INL {
                 if ((m >> i) & 1ull) {
-                    reg_for<CS>([&](auto s) MPQP_INL { R.d[s] = fma(-c, R.t[i / 4][s][i % 4], R.d[s]); });
+                    reg_for<CS>([&](auto s) MPQP_INL { R.d[s] = fma(-c, R.template get<decltype(i)::value, decltype(s)::value>(), R.d[s]); });
                     if constexpr (EX > 0) {
-                        float v = 0.f;
+                        Re v = 0;
                         reg_for<EX>([&](auto e) MPQP_INL { v = lane == e ? lane_get(R.xs[e], i) : v; });
                         R.d[CS] = fma(-c, v, R.d[CS]);
                     }
@@ -468,56 +627,56 @@ __device__ __forceinline__ void reg_cost(RegTab<NW, RW, CS, EX> &R, const RegLds
 }
 
 // d into L.dl (wave 0)
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_cost_out(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L) {
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_cost_out(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L) {
     if (wave_id() == 0) {
         const int lane = fresh_lane();
-        reg_for<RegTab<NW, RW, CS, EX>::NS>([&](auto s) MPQP_INL { L.dl[lane + MPQP_WAVE * s] = R.d[s]; });
+        reg_for<RegTab<Re, NW, RW, CS, EX, LW>::NS>([&](auto s) MPQP_INL { L.dl[lane + MPQP_WAVE * s] = R.d[s]; });
     }
 }
 
 // The wave's two smallest basic values (perturbed: x + xp) for the choice of
 // the leaving row.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_min_out(const RegTab<NW, RW, CS, EX> &R, RegShared<NW> &ws, int M,
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_min_out(const RegTab<Re, NW, RW, CS, EX, LW> &R, RegShared<Re, NW> &ws, int M,
                                             bool pert) {
     const int lane = fresh_lane(), wave = wave_id();
     const bool valid = lane < RW && wave * RW + lane < M;
-    const float x = pert ? R.x() + R.xp() : R.x();
+    const Re x = pert ? R.x() + R.xp() : R.x();
     const bool nan = valid && x != x;
-    const float v = (valid && !nan) ? x : INFINITY;
-    float m1 = v, m2 = INFINITY;
-    wave_min2_f(m1, m2);
+    const Re v = (valid && !nan) ? x : (Re)INFINITY;
+    Re m1 = v, m2 = (Re)INFINITY;
+    wave_min2(m1, m2);
     const int f = __ffsll((long long)__ballot(v == m1)) - 1;
     const int an = __any(nan) ? 1 : 0;
     if (lane == 0) {
-        ws.min[wave] = RegMin{m1, m2, wave * RW + f, an};
+        ws.min[wave] = RegMin<Re>{m1, m2, wave * RW + f, an};
     }
 }
 
 // primal_ratio_wave over the register tableau, by the whole workgroup: every
 // wave returns the row.  Two barriers.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ int reg_ratio(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, RegShared<NW> &ws,
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ int reg_ratio(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, RegShared<Re, NW> &ws,
                                          int M, int q, const DevTol &tl) {
     const int lane = fresh_lane(), wave = wave_id();
     const bool valid = lane < RW && wave * RW + lane < M;
-    const float a = reg_col(R, L, q);
-    float lim = (float)tl.tol_plus;
+    const Re a = reg_col(R, L, q);
+    Re lim = (Re)tl.tol_plus;
     if (tl.pivot_rel > 0.0) {
-        const float fa = fabsf(a);
-        const float cw = -wave_min_f((valid && fa > 0.f) ? -fa : 0.f);
+        const Re fa = fabs(a);
+        const Re cw = -wave_min((valid && fa > (Re)0) ? -fa : (Re)0);
         if (lane == 0) ws.cmax[wave] = cw;
         __syncthreads();
-        const float cm = -lane_get(row8_min_f(-ws.cmax[lane % NW]), 7);
-        const float rl = (float)tl.pivot_rel * cm;
+        const Re cm = -lane_get(row8_min(-ws.cmax[lane % NW]), 7);
+        const Re rl = (Re)tl.pivot_rel * cm;
         lim = rl > lim ? rl : lim;
     }
     // the wave's smallest ratio, its lowest row
     const bool take = valid && a > lim;
-    const float rt = take ? R.x() / a : 0.f;
+    const Re rt = take ? R.x() / a : (Re)0;
     const bool num = take && rt == rt;
-    const float m = wave_min_f(num ? rt : INFINITY);
+    const Re m = wave_min(num ? rt : (Re)INFINITY);
     const unsigned long long hit = __ballot(num && rt == m), any = __ballot(take);
     const int f = __ffsll((long long)(hit ? hit : any)) - 1;
     if (lane == 0) {
@@ -526,8 +685,8 @@ __device__ __forceinline__ int reg_ratio(const RegTab<NW, RW, CS, EX> &R, const 
     }
     __syncthreads();
     const int k = ws.rk[lane % NW];
-    const float v = k >= 0 ? ws.rv[lane % NW] : INFINITY;
-    const float mm = lane_get(row8_min_f(v), 7);
+    const Re v = k >= 0 ? ws.rv[lane % NW] : (Re)INFINITY;
+    const Re mm = lane_get(row8_min(v), 7);
     const unsigned long long has = __ballot(lane < NW && k >= 0), best = __ballot(lane < NW && k >= 0 && v == mm);
     const int w = __ffsll((long long)(best ? best : has)) - 1;
     return w < 0 ? -1 : __builtin_amdgcn_readlane(k, w);
@@ -536,12 +695,12 @@ __device__ __forceinline__ int reg_ratio(const RegTab<NW, RW, CS, EX> &R, const 
 // A pivot on (r, q) that every wave knows: the row's wave divides and
 // publishes it, every wave updates; `between` is run by one thread while the
 // update runs (the basis bookkeeping).  Two barriers.
-template <int NW, int RW, int CS, int EX, typename F>
-__device__ __forceinline__ void reg_pivot(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, int r, int q,
+template <typename Re, int NW, int RW, int CS, int EX, int LW, typename F>
+__device__ __forceinline__ void reg_pivot(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int r, int q,
                                           F between) {
     const int wave = wave_id(), lr = r - wave * RW;
     if ((unsigned)lr < (unsigned)RW) {
-        float al[CS + 1];
+        Re al[CS + 1];
         reg_row(R, lr, al);
         reg_publish(R, L, al, lr, q);
     }
@@ -563,8 +722,8 @@ __device__ __forceinline__ void reg_swap(const LT &L, int r, int q) {
 // ---------------------------------------------------------------------
 // start
 // ---------------------------------------------------------------------
-template <int NW, int RW, int CS, int EX, typename Src>
-__device__ __forceinline__ void reg_load(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
+template <typename Re, int NW, int RW, int CS, int EX, int LW, typename Src>
+__device__ __forceinline__ void reg_load(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
                                          const DevProb &P, const Src *sT, int src_ld, const int *sb, const int *sn) {
     const int M = P.M2, K = P.K2;
     const int lane = fresh_lane(), wave = wave_id();
@@ -576,17 +735,17 @@ __device__ __forceinline__ void reg_load(RegTab<NW, RW, CS, EX> &R, const RegLds
     reg_for<RW>([&](auto i) MPQP_INL {
         const int row = min(wave * RW + i, M - 1);
         const Src *rp = sT + (long long)row * src_ld;
-        reg_for<CS>([&](auto s) MPQP_INL { R.t[i / 4][s][i % 4] = (float)rp[cc[s]]; });
+        reg_for<CS>([&](auto s) MPQP_INL { R.template set<decltype(i)::value, decltype(s)::value>((Re)rp[cc[s]]); });
     });
     const int row = wave * RW + lane;
     const bool valid = lane < RW && row < M;
     const Src *rr = sT + (long long)(valid ? row : 0) * src_ld;
     reg_for<EX>([&](auto e) MPQP_INL {
         const int c = MPQP_WAVE * CS + e;
-        R.xs[e] = (valid && c < K) ? (float)rr[c] : 0.f;
+        R.xs[e] = (valid && c < K) ? (Re)rr[c] : (Re)0;
     });
-    R.xs[EX] = valid ? (float)rr[K] : 0.f;
-    R.xs[EX + 1] = valid ? (float)rr[K + 1] : 0.f;
+    R.xs[EX] = valid ? (Re)rr[K] : (Re)0;
+    R.xs[EX + 1] = valid ? (Re)rr[K + 1] : (Re)0;
     for (int i = threadIdx.x; i < M; i += NW * MPQP_WAVE) {
         const int b = sb[i];
         L.basis[i] = b;
@@ -600,77 +759,103 @@ __device__ __forceinline__ void reg_load(RegTab<NW, RW, CS, EX> &R, const RegLds
     __syncthreads();
 }
 
-// opt_lambda: the lambda swaps of S[j0 .. j1); the rows are staged in LDS so
-// that a thread can walk its row's e-columns in the order of the terms.
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ int reg_lambda(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
-                                          const DevProb &P, const DevTol &tl, const int *Sset, int j0, int j1) {
+// opt_lambda: the lambda swaps of S[j0 .. j1), a row's terms in ascending t,
+// zeros skipped.  A thread walks its row's e-columns: in FP32 the rows are
+// staged in LDS; in FP64 the first swap reads them from the state that was
+// just loaded (sT, still as it was), and later ones, of a cold start, take
+// the columns out of the registers one after the other.
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ int reg_lambda(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
+                                          const DevProb &P, const DevTol &tl, const int *Sset, int j0, int j1,
+                                          const Re *sT, int src_ld) {
     const int M = P.M2, K = P.K2, N2 = P.N2;
     const int r4 = M - P.n_c - P.n_x, nt = P.n_x + 1;
     const int tid = threadIdx.x;
-    float *lam = L.ep;
+    Re *lam = L.ep;
     int *wl = L.bcnt;
+    auto walk = [&](const Re *Ti, int row) {
+        // loads of U terms in flight
+        constexpr int U = sizeof(Re) == 4 ? 4 : 8;
+        Re acc = 0;
+        for (int t0 = 0; t0 < nt; t0 += U) {
+            Re av[U], tv[U];
+            int w[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = t0 + u < nt ? t0 + u : nt - 1;
+                av[u] = t0 + u < nt ? lam[t] : (Re)0;
+                w[u] = wl[t];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) tv[u] = Ti[w[u] >= 0 ? 0 : -w[u] - 1];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const Re f1 = fma(av[u], (Re)1, acc);
+                const Re f2 = fma(av[u], tv[u], acc);
+                const Re na = w[u] >= 0 ? (row == w[u] ? f1 : acc) : f2;
+                acc = av[u] == (Re)0 ? acc : na;
+            }
+        }
+        L.colx[row] = acc;
+    };
     for (int jj = j0; jj < j1; ++jj) {
         const int j = Sset[jj];
         for (int t = tid; t < nt; t += NW * MPQP_WAVE) {
             const int rho = t == 0 ? j : r4 + t - 1;
-            lam[t] = (float)lam_entry(P, j, rho);
+            lam[t] = (Re)lam_entry(P, j, rho);
             wl[t] = L.where[N2 - M + rho];
         }
-        for (int h = 0; h < L.np; ++h) {
-            reg_dump(R, L, K, h);
+        if constexpr (sizeof(Re) == 4) {
+            for (int h = 0; h < L.np; ++h) {
+                reg_dump(R, L, K, h);
+                __syncthreads();
+                for (int i = tid; i < L.rp && h * L.rp + i < M; i += NW * MPQP_WAVE)
+                    walk(L.stage + i * L.sld, h * L.rp + i);
+                __syncthreads();
+            }
+        } else {
             __syncthreads();
-            for (int i = tid; i < L.rp && h * L.rp + i < M; i += NW * MPQP_WAVE) {
-                const int row = h * L.rp + i;
-                const float *Ti = L.stage + i * L.sld;
-                // terms in ascending t, zeros skipped; loads of 4 in flight
-                float acc = 0.f;
-                for (int t0 = 0; t0 < nt; t0 += 4) {
-                    float av[4], tv[4];
-                    int w[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int t = t0 + u < nt ? t0 + u : nt - 1;
-                        av[u] = t0 + u < nt ? lam[t] : 0.f;
-                        w[u] = wl[t];
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) tv[u] = Ti[w[u] >= 0 ? 0 : -w[u] - 1];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const float f1 = fma(av[u], 1.f, acc);
-                        const float f2 = fma(av[u], tv[u], acc);
-                        const float na = w[u] >= 0 ? (row == w[u] ? f1 : acc) : f2;
-                        acc = av[u] == 0.f ? acc : na;
-                    }
+            if (jj == j0) {
+                for (int i = tid; i < M; i += NW * MPQP_WAVE) walk(sT + (long long)i * src_ld, i);
+            } else {
+                const int lane = fresh_lane(), row = wave_id() * RW + lane;
+                Re acc = 0;
+                for (int t = 0; t < nt; ++t) {
+                    const Re av = lane_get(lam[t], 0);
+                    const int w = rfl(wl[t]);
+                    const Re tv = reg_col(R, L, w >= 0 ? 0 : -w - 1);
+                    const Re f1 = fma(av, (Re)1, acc);
+                    const Re f2 = fma(av, tv, acc);
+                    const Re na = w >= 0 ? (row == w ? f1 : acc) : f2;
+                    acc = av == (Re)0 ? acc : na;
                 }
-                L.colx[row] = acc;
+                if (lane < RW && row < M) L.colx[row] = acc;
             }
             __syncthreads();
         }
         const int p = rfl(L.where[P.n_x + P.n_t + j]);
         const int lane = fresh_lane(), wave = wave_id();
         const int row = wave * RW + lane;
-        const float fv = (lane < RW && row < M) ? L.colx[row] : 0.f;
+        const Re fv = (lane < RW && row < M) ? L.colx[row] : (Re)0;
         // w_j basic at position p: a pivot on row p with the column vcol held
         // outside the tableau; w_j nonbasic in column kk: the column
         // replaced (T - column * 1, then + vcol * 1, in its lane)
-        const float pv = lane_get(L.colx[p >= 0 ? p : 0], 0);
+        const Re pv = lane_get(L.colx[p >= 0 ? p : 0], 0);
         if (p >= 0 && !(fabs((double)pv) > tl.licq)) return 0;
         const int kk = p >= 0 ? -1 : -p - 1, lr = p - wave * RW;
         if (p >= 0 && (unsigned)lr < (unsigned)RW) {
-            float al[CS + 1];
+            Re al[CS + 1];
             reg_row(R, lr, al);
             reg_divide(R, L, al, lr, -1, pv);
         }
         __syncthreads();
-        reg_col_op<true>(R, L, kk < 0 ? 0 : kk, kk >= 0);
-        float pr[CS + 1];
+        if constexpr (sizeof(Re) == 4) reg_col_op<true>(R, L, kk < 0 ? 0 : kk, kk >= 0);
+        Re pr[CS + 1];
         reg_for<CS + 1>([&](auto s) MPQP_INL {
             const int col = lane + MPQP_WAVE * s;
-            pr[s] = kk < 0 ? L.ep[col] : (col == kk ? 1.f : 0.f);
+            pr[s] = kk < 0 ? L.ep[col] : (col == kk ? (Re)1 : (Re)0);
         });
-        reg_apply(R, L, pr, kk < 0 ? fv : -fv, kk < 0 ? p : -MPQP_WAVE * NW);
+        reg_apply(R, L, pr, kk < 0 ? fv : -fv, kk < 0 ? p : -MPQP_WAVE * NW, kk);
         __syncthreads();
     }
     return 1;
@@ -679,14 +864,14 @@ __device__ __forceinline__ int reg_lambda(RegTab<NW, RW, CS, EX> &R, const RegLd
 // ---------------------------------------------------------------------
 // phase 1 (opt_phase1's decisions)
 // ---------------------------------------------------------------------
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
                                                const DevProb &P, const DevOpts &O, const DevTol &tl, OptShared &sh,
-                                               RegShared<NW> &ws) {
-    constexpr int SM = (NW * RW + MPQP_WAVE - 1) / MPQP_WAVE, NS = RegTab<NW, RW, CS, EX>::NS;
+                                               RegShared<Re, NW> &ws) {
+    constexpr int SM = (NW * RW + MPQP_WAVE - 1) / MPQP_WAVE, NS = RegTab<Re, NW, RW, CS, EX, LW>::NS;
     const int M = P.M2, K = P.K2, N2 = P.N2, Nn = P.Nn;
     const int wave = wave_id();
-    reg_cost(R, L, M, K, 1.f, [&](int b) { return b >= Nn; },
+    reg_cost(R, L, M, K, (Re)1, [&](int b) { return b >= Nn; },
              [&](int col) { return L.nonb[col] >= Nn ? 1.f : 0.f; });
     for (int v = threadIdx.x; v < N2; v += NW * MPQP_WAVE) { L.bcnt[v] = 0; L.nbcnt[v] = 0; }
     {
@@ -717,9 +902,9 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
             // Leaving row, by every wave: a unique minimum (no NaN, no other
             // value within the tree's 1e-10 band, no counter preference) wins
             // every combine of the reference tree; anything else runs the tree.
-            const RegMin w = ws.min[lane % NW];
-            float m = lane < NW ? w.m1 : INFINITY, m2 = lane < NW ? w.m2 : INFINITY;
-            row8_min2_f(m, m2);
+            const RegMin<Re> w = ws.min[lane % NW];
+            Re m = lane < NW ? w.m1 : (Re)INFINITY, m2 = lane < NW ? w.m2 : (Re)INFINITY;
+            row8_min2(m, m2);
             m = lane_get(m, 7);
             m2 = lane_get(m2, 7);
             const int f = __ffsll((long long)__ballot(w.m1 == m)) - 1;
@@ -728,21 +913,40 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
             const bool go_on = (double)m < tl.dual_stop_tol;
             const int mode_b = (n_same % 20) >= 10 ? 1 : 0;
             if (rfl((mode_b || tie || __any(w.nan)) ? 1 : 0)) {
-                float v[SM];
-                int pk[SM];
+                Re v[SM];
+                int id[SM], cn[SM];
+                bool other = false;
+                unsigned long long hit[SM];
+                int c0 = -1;
 #pragma unroll
                 for (int s = 0; s < SM; ++s) {
                     const int i = lane + MPQP_WAVE * s;
                     const bool valid = i < M;
                     const int ic = valid ? i : 0;
-                    const float x0 = L.gx[ic], xp = L.gp[ic];
-                    v[s] = valid ? (pert ? x0 + xp : x0) : 0.f;
-                    pk[s] = L.bcnt[L.basis[ic]] << 10 | ic;
+                    const Re x0 = L.gx[ic], xp = L.gp[ic];
+                    v[s] = valid ? (pert ? x0 + xp : x0) : (Re)0;
+                    id[s] = ic;
+                    cn[s] = L.bcnt[L.basis[ic]];
                 }
-                const DminPred pred{mode_b, tl.dual_stop_tol};
-                r = tree32<SM>(v, pk, M, lane, [&](float vt, int pt, float vu, int pu) {
-                    return pred((double)vt, 0, pt >> 10, (double)vu, 0, pu >> 10);
-                }) & 1023;
+                // Several minima, or values within the band of the minimum:
+                // where their counts are all the same, the predicate keeps
+                // the smaller value, the first of the minima in its order
+                // (the values of a degenerate basis tie exactly).
+                reg_for<SM>([&](auto s) MPQP_INL {
+                    const bool valid = lane + MPQP_WAVE * s < M;
+                    hit[s] = __ballot(valid && v[s] == m);
+                    if (c0 < 0 && hit[s]) c0 = __builtin_amdgcn_readlane(cn[s], __ffsll((long long)hit[s]) - 1);
+                });
+                reg_for<SM>([&](auto s) MPQP_INL {
+                    const bool valid = lane + MPQP_WAVE * s < M;
+                    other |= valid && !((double)m <= (double)v[s] - 1e-10) && cn[s] != c0;
+                });
+                if (rfl((mode_b || __any(w.nan) || __any(other)) ? 1 : 0)) {
+                    r = reg_tree<SM>(v, id, cn, M, lane, DminPred{mode_b, tl.dual_stop_tol});
+                } else {
+                    r = tree_first<SM>(hit);
+                }
+                r = rfl(r);
             }
             if (rfl(go_on ? 1 : 0)) break;
             act = ACT_STOP;
@@ -773,22 +977,22 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
                     const int kk = lane + MPQP_WAVE * s;
                     cnt_of[s] = L.nbcnt[L.nonb[kk < K ? kk : 0]];
                 });
-                float al[CS + 1];
+                Re al[CS + 1];
                 reg_row(R, lr, al);
-                float dlim = (float)tl.tol_minus;
+                Re dlim = (Re)tl.tol_minus;
                 if (tl.pivot_rel > 0.0) {
-                    float am = 0.f;
+                    Re am = 0;
                     reg_for<NS>([&](auto s) MPQP_INL {
-                        const float a = lane + MPQP_WAVE * s < K ? fabsf(al[s]) : 0.f;
+                        const Re a = lane + MPQP_WAVE * s < K ? (Re)fabs(al[s]) : (Re)0;
                         am = a > am ? a : am;
                     });
-                    const float rl = -(float)tl.pivot_rel * -wave_min_f(-am);
+                    const Re rl = -(Re)tl.pivot_rel * -wave_min(-am);
                     dlim = rl < dlim ? rl : dlim;
                 }
                 const int mode = n_same < 10 ? 0 : (n_same < 100 ? 1 : 2);
-                float v[NS];
+                Re v[NS];
                 bool tk[NS];
-                float ml = INFINITY;
+                Re ml = (Re)INFINITY;
                 bool nn = false, any_t = false;
                 reg_for<NS>([&](auto s) MPQP_INL {
                     tk[s] = lane + MPQP_WAVE * s < K && al[s] < dlim;
@@ -808,7 +1012,7 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
                     // within 1e-12: if no other value lies within that band
                     // of the minimum, the minima are compared by their counts
                     // alone, and any of them beats everything else.
-                    const float m = wave_min_f(ml);
+                    const Re m = wave_min(ml);
                     unsigned long long hit[NS];
                     bool near = false;
                     int cnt = 0;
@@ -820,27 +1024,20 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
                     if (mode == 0 || (cnt == 1 && !__any(near))) {
                         qk = tree_first<NS>(hit);
                     } else if (!__any(near)) {
-                        int pk[NS];
-                        reg_for<NS>([&](auto s) MPQP_INL {
-                            const bool h = tk[s] && v[s] == m;
-                            pk[s] = h ? cnt_of[s] << 10 | (lane + MPQP_WAVE * s) : -1;
+                        int id[NS];
+                        reg_for<NS>([&](auto s) MPQP_INL { id[s] = tk[s] && v[s] == m ? lane + MPQP_WAVE * s : -1; });
+                        qk = reg_tree<NS>(v, id, cnt_of, K, lane, [](double, int it, int ct, double, int iu, int cu) {
+                            return (iu >= 0) & ((it < 0) | (ct > cu + 2));
                         });
-                        qk = tree32<NS>(v, pk, K, lane, [](float, int pt, float, int pu) {
-                            return (pu >= 0) & ((pt < 0) | ((pt >> 10) > (pu >> 10) + 2));
-                        }) & 1023;
                     }
                 }
                 if (qk == -2) {
-                    int pk[NS];
+                    int id[NS];
                     reg_for<NS>([&](auto s) MPQP_INL {
-                        pk[s] = tk[s] ? cnt_of[s] << 10 | (lane + MPQP_WAVE * s) : -1;
-                        v[s] = tk[s] ? v[s] : 100000.f;
+                        id[s] = tk[s] ? lane + MPQP_WAVE * s : -1;
+                        v[s] = tk[s] ? v[s] : (Re)100000;
                     });
-                    const DratioPred pred{mode};
-                    const int w = tree32<NS>(v, pk, K, lane, [&](float vt, int pt, float vu, int pu) {
-                        return pred((double)vt, pt, pt >> 10, (double)vu, pu, pu >> 10);
-                    });
-                    qk = w < 0 ? -1 : w & 1023;
+                    qk = reg_tree<NS>(v, id, cnt_of, K, lane, DratioPred{mode});
                 }
                 qk = rfl(qk);
                 if (qk >= 0) reg_publish(R, L, al, lr, qk);
@@ -849,16 +1046,16 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
             }
             if (wave == (wo + 1) % NW) {
                 // meanwhile: the sum of the negative x_B for the stall counter
-                float ps[SM];
+                Re ps[SM];
     #pragma unroll
                 for (int s = 0; s < SM; ++s) {
                     const int i = lane + MPQP_WAVE * s;
                     const int ic = i < M ? i : 0;
-                    const float x0 = L.gx[ic], xp = L.gp[ic];
-                    const float x = (pert && i < M) ? x0 + xp : x0;
-                    ps[s] = (i < M && x < 0.f) ? x : 0.f;
+                    const Re x0 = L.gx[ic], xp = L.gp[ic];
+                    const Re x = (pert && i < M) ? x0 + xp : x0;
+                    ps[s] = (i < M && x < (Re)0) ? x : (Re)0;
                 }
-                tree_sum_lane0<SM, float>(ps, M, lane);
+                tree_sum_lane0<SM, Re>(ps, M, lane);
                 if (lane == 0) sh.pinf = (double)ps[0];
             }
             __syncthreads();
@@ -909,14 +1106,14 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
             end = 3;
         } else {
             const int lane = fresh_lane();
-            float dl = INFINITY;
+            Re dl = (Re)INFINITY;
             bool nn = false;
             reg_for<NS>([&](auto s) MPQP_INL {
                 const bool in = lane + MPQP_WAVE * s < K;
                 nn |= in && R.d[s] != R.d[s];
                 dl = (in && R.d[s] < dl) ? R.d[s] : dl;
             });
-            const float dm = wave_min_f(dl);
+            const Re dm = wave_min(dl);
             double dv = (double)dm;
             int cnt = 0;
             reg_for<NS>([&](auto s) MPQP_INL {
@@ -953,13 +1150,13 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
     if (end != 1) return res;
     if (wave == 0) {
         const int lane = fresh_lane();
-        float zs[SM];
+        Re zs[SM];
 #pragma unroll
         for (int s = 0; s < SM; ++s) {
             const int i = lane + MPQP_WAVE * s;
-            zs[s] = (i < M) ? (L.basis[i] >= Nn ? 1.f : 0.f) * L.gx[i] : 0.f;
+            zs[s] = (i < M) ? (L.basis[i] >= Nn ? (Re)1 : (Re)0) * L.gx[i] : (Re)0;
         }
-        const double zz = (double)tree_sum_s<SM, float>(zs, M, lane);
+        const double zz = (double)tree_sum_s<SM, Re>(zs, M, lane);
         if (lane == 0) sh.z = zz;
     }
     reg_cost_out(R, L);
@@ -971,10 +1168,10 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<NW, RW, CS, EX> &R, const 
 }
 
 // opt_drive_out (on = 0: nothing to do)
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ int reg_drive_out(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, const DevProb &P,
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ int reg_drive_out(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, const DevProb &P,
                                              const DevTol &tl, OptShared &sh, int on) {
-    constexpr int SM = (NW * RW + MPQP_WAVE - 1) / MPQP_WAVE, NS = RegTab<NW, RW, CS, EX>::NS;
+    constexpr int SM = (NW * RW + MPQP_WAVE - 1) / MPQP_WAVE, NS = RegTab<Re, NW, RW, CS, EX, LW>::NS;
     const int M = P.M2, K = P.K2, Nn = P.Nn;
     rows_where<SM>(L.rows, M, sh, [&](int i) { return L.basis[i] >= Nn; });
     const int n = on ? rfl(sh.nrows) : 0, wave = wave_id();
@@ -983,7 +1180,7 @@ __device__ __forceinline__ int reg_drive_out(RegTab<NW, RW, CS, EX> &R, const Re
         const int i = rfl(L.rows[t]), lr = i - wave * RW;
         if ((unsigned)lr < (unsigned)RW) {
             const int lane = fresh_lane();
-            float al[CS + 1];
+            Re al[CS + 1];
             reg_row(R, lr, al);
             double v = 0.0;
             int key = -1, aux = 0;
@@ -1011,15 +1208,15 @@ __device__ __forceinline__ int reg_drive_out(RegTab<NW, RW, CS, EX> &R, const Re
 // ---------------------------------------------------------------------
 // phase 2 (opt_phase2's decisions); SN slots of 64 cover the Nn variables
 // ---------------------------------------------------------------------
-template <int SN, int NW, int RW, int CS, int EX>
-__device__ __forceinline__ P2Result reg_phase2(RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
+template <int SN, typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ P2Result reg_phase2(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
                                                const DevProb &P, const DevOpts &O, const DevTol &tl, OptShared &sh,
-                                               RegShared<NW> &ws) {
+                                               RegShared<Re, NW> &ws) {
     constexpr int SM = (NW * RW + MPQP_WAVE - 1) / MPQP_WAVE;
     const int M = P.M2, K = P.K2, N2 = P.N2, Nn = P.Nn;
     const int EPS = P.n_x + P.n_t + P.n_c;
     const int wave = wave_id();
-    reg_cost(R, L, M, K, -1.f, [&](int b) { return b == EPS; },
+    reg_cost(R, L, M, K, (Re)-1, [&](int b) { return b == EPS; },
              [&](int col) { return L.nonb[col] == EPS ? -1.f : 0.f; });
     for (int v = threadIdx.x; v < N2; v += NW * MPQP_WAVE) L.bcnt[v] = 0;
     reg_cost_out(R, L);
@@ -1030,20 +1227,21 @@ __device__ __forceinline__ P2Result reg_phase2(RegTab<NW, RW, CS, EX> &R, const 
         if (it < O.max_iter_p2) {
             if (wave == 0) { MPQP_PRIO_HI();
                 const int lane = fresh_lane();
-                float v[SN];
-                int pk[SN];
-                float ml = INFINITY;
+                Re v[SN];
+                int id[SN], cn[SN];
+                Re ml = (Re)INFINITY;
                 bool tree = false;
 #pragma unroll
                 for (int s = 0; s < SN; ++s) {
                     const int var = lane + MPQP_WAVE * s;
-                    v[s] = 0.f;
-                    pk[s] = var;
+                    v[s] = 0;
+                    id[s] = var;
+                    cn[s] = 0;
                     if (var < Nn) {
-                        const int w = L.where[var], cn = L.bcnt[var];
-                        v[s] = w >= 0 ? 100000.f : L.dl[-w - 1];
-                        pk[s] = cn << 10 | var;
-                        tree |= v[s] != v[s] || (cn != 0 && (double)v[s] < -1e-10);
+                        const int w = L.where[var];
+                        cn[s] = L.bcnt[var];
+                        v[s] = w >= 0 ? (Re)100000 : L.dl[-w - 1];
+                        tree |= v[s] != v[s] || (cn[s] != 0 && (double)v[s] < -1e-10);
                         ml = v[s] < ml ? v[s] : ml;
                     }
                 }
@@ -1051,17 +1249,15 @@ __device__ __forceinline__ P2Result reg_phase2(RegTab<NW, RW, CS, EX> &R, const 
                 // differ among the improving variables: with none of them
                 // chosen before, the first of the minima in its order.
                 int wv;
-                float dm;
+                Re dm;
                 if (!__any(tree)) {
-                    dm = wave_min_f(ml);
+                    dm = wave_min(ml);
                     unsigned long long hit[SN];
 #pragma unroll
                     for (int s = 0; s < SN; ++s) hit[s] = __ballot(lane + MPQP_WAVE * s < Nn && v[s] == dm);
                     wv = tree_first<SN>(hit);
                 } else {
-                    wv = tree32<SN>(v, pk, Nn, lane, [](float vt, int pt, float vu, int pu) {
-                        return P2Pred{}((double)vt, 0, pt >> 10, (double)vu, 0, pu >> 10);
-                    }) & 1023;
+                    wv = reg_tree<SN>(v, id, cn, Nn, lane, P2Pred{});
                     dm = lane_get(v[0], 0);
                 }
                 const double dmin = (double)dm;
@@ -1069,13 +1265,13 @@ __device__ __forceinline__ P2Result reg_phase2(RegTab<NW, RW, CS, EX> &R, const 
                 int q = -1;
                 double zz = 0.0;
                 if (dmin > tl.tol_minus_opt) {
-                    float zs[SM];
+                    Re zs[SM];
     #pragma unroll
                     for (int s = 0; s < SM; ++s) {
                         const int i = lane + MPQP_WAVE * s;
-                        zs[s] = (i < M) ? (L.basis[i] == EPS ? -1.f : 0.f) * L.gx[i] : 0.f;
+                        zs[s] = (i < M) ? (L.basis[i] == EPS ? (Re)-1 : (Re)0) * L.gx[i] : (Re)0;
                     }
-                    zz = (double)tree_sum_s<SM, float>(zs, M, lane);
+                    zz = (double)tree_sum_s<SM, Re>(zs, M, lane);
                 } else {
                     q = -L.where[wv] - 1;
                 }
@@ -1113,8 +1309,8 @@ __device__ __forceinline__ P2Result reg_phase2(RegTab<NW, RW, CS, EX> &R, const 
 // the certificate's corrections over the staged rows
 // ---------------------------------------------------------------------
 // x += B32^-1 r (see cert_primal): the team of row i over its e-columns
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_primal_corr(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_primal_corr(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
                                                 const DevProb &P, int ne) {
     const int M = P.M2, K = P.K2, e0 = P.N2 - M;
     double *x = L.cx, *r = L.cr;
@@ -1158,8 +1354,8 @@ __device__ __forceinline__ void reg_primal_corr(const RegTab<NW, RW, CS, EX> &R,
 
 // y += B32^-T r (see cert_dual): the team of an e-column down the positions,
 // its partial sums kept across the passes
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_dual_corr(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L,
+template <typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_dual_corr(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
                                               const DevProb &P, int ne) {
     constexpr int NT = NW * MPQP_WAVE;
     constexpr int NI = ((MPQP_WAVE * CS + EX) * MPQP_GT + NT - 1) / NT;
@@ -1214,40 +1410,41 @@ __device__ __forceinline__ void reg_dual_corr(const RegTab<NW, RW, CS, EX> &R, c
 }
 
 // The phase-1 state into the store of the next level (rows of opt_ld).
-template <int NW, int RW, int CS, int EX>
-__device__ __forceinline__ void reg_store(const RegTab<NW, RW, CS, EX> &R, const RegLds<NW, RW, CS, EX> &L, int M, int K,
+template <typename Dst, typename Re, int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ void reg_store(const RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int M, int K,
                                           unsigned char *dst) {
-    const int ld = opt_ld<float>(K), wave = wave_id(), lane = fresh_lane();
-    float *dT = reinterpret_cast<float *>(dst);
+    const int ld = opt_ld<Dst>(K), wave = wave_id(), lane = fresh_lane();
+    Dst *dT = reinterpret_cast<Dst *>(dst);
     reg_for<CS>([&](auto s) MPQP_INL {
         const unsigned c = lane + MPQP_WAVE * s;
         if (c < (unsigned)K)
             reg_for<RW>([&](auto i) MPQP_INL {
                 const int row = wave * RW + i;
-                if (row < M) (dT + (long long)row * ld)[c] = R.t[i / 4][s][i % 4];
+                if (row < M) (dT + (long long)row * ld)[c] = (Dst)R.template get<decltype(i)::value, decltype(s)::value>();
             });
     });
     if (lane < RW && wave * RW + lane < M) {
-        float *dr = dT + (long long)(wave * RW + lane) * ld;
+        Dst *dr = dT + (long long)(wave * RW + lane) * ld;
         reg_for<EX>([&](auto e) MPQP_INL {
-            if (MPQP_WAVE * CS + e < K) dr[MPQP_WAVE * CS + e] = R.xs[e];
+            if (MPQP_WAVE * CS + e < K) dr[MPQP_WAVE * CS + e] = (Dst)R.xs[e];
         });
-        dr[K] = R.x();
-        dr[K + 1] = R.xp();
+        dr[K] = (Dst)R.x();
+        dr[K + 1] = (Dst)R.xp();
     }
-    int *db = reinterpret_cast<int *>(dT + (long long)opt_tw<float>(M, K));
+    int *db = reinterpret_cast<int *>(dT + (long long)opt_tw<Dst>(M, K));
     for (int i = threadIdx.x; i < M; i += NW * MPQP_WAVE) db[i] = L.basis[i];
     for (int kk = threadIdx.x; kk < K; kk += NW * MPQP_WAVE) db[M + kk] = L.nonb[kk];
 }
 
-// The FP32 opt_body over a register tableau.
-template <int NW, int RW, int CS, int EX, int SN>
+// opt_body over a register tableau.
+template <typename Re, int NW, int RW, int CS, int EX, int LW, int SN>
 __device__ __forceinline__ void reg_body(const OptArgs &a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __shared__ OptShared sh;
-    __shared__ RegShared<NW> ws;
+    __shared__ RegShared<Re, NW> ws;
     __shared__ unsigned inS[8];
     __shared__ double red[NW];
+    constexpr bool MIXED = sizeof(Re) == 4;
     constexpr int NT = NW * MPQP_WAVE, SM = (NW * RW + MPQP_WAVE - 1) / MPQP_WAVE;
     const DevProb &P = a.P;
     const DevOpts &O = a.O;
@@ -1255,10 +1452,11 @@ __device__ __forceinline__ void reg_body(const OptArgs &a) {
     const int tid = threadIdx.x;
     const int k = a.level;
     const int n = a.n_dev ? *a.n_dev : a.n;
-    RegTab<NW, RW, CS, EX> R;
-    RegLds<NW, RW, CS, EX> L;
-    L.carve(smem, M, K, N2, true, a.stage_passes);
-    const DevTol tl = dev_tol32(O);
+    RegTab<Re, NW, RW, CS, EX, LW> R;
+    RegLds<Re, NW, RW, CS, EX, LW> L;
+    L.carve(smem, M, K, N2, a.stage_passes);
+    R.lt = L.rows_lds + wave_id() * (LW * CS * MPQP_WAVE) + fresh_lane();
+    const DevTol tl = MIXED ? dev_tol32(O) : dev_tol64(O);
     if (a.counter) {
         if (tid == 0) sh.item = atomicAdd(a.counter, 1);
     }
@@ -1295,17 +1493,33 @@ __device__ __forceinline__ void reg_body(const OptArgs &a) {
         P1Result p1{ST_NOT_RUN, 0, 0, 0.0};
         P2Result p2{ST_NOT_RUN, 0, 0, 0.0};
         int clean = 0, warm = par >= 0 ? 1 : 0;
-        auto pcorr = [&](int ne) { reg_primal_corr(R, L, P, ne); };
-        auto dcorr = [&](int ne) { reg_dual_corr(R, L, P, ne); };
+        auto pcorr = [&](int ne) {
+            if constexpr (MIXED) reg_primal_corr(R, L, P, ne);
+        };
+        auto dcorr = [&](int ne) {
+            if constexpr (MIXED) reg_dual_corr(R, L, P, ne);
+        };
+        (void)pcorr;
+        (void)dcorr;
         auto solve = [&]() MPQP_INL -> bool {
             // start: the parent's state + the lambda swap of S[k-1]; else
             // (or if that basis is singular) the root's + those of all of S
             for (;;) {
-                const float *sT = warm ? reinterpret_cast<const float *>(a.ostore_prev + (long long)par * a.ostride)
-                                       : P.root32;
-                const int *sb = reinterpret_cast<const int *>(sT + (long long)opt_tw<float>(M, K));
-                reg_load(R, L, P, sT, opt_ld<float>(K), sb, sb + M);
-                const int ok = reg_lambda(R, L, P, tl, Sset, warm ? k - 1 : 0, k);
+                const Re *sT;
+                const int *sb, *sn;
+                int sld = opt_ld<Re>(K);
+                if constexpr (MIXED) {
+                    sT = warm ? reinterpret_cast<const Re *>(a.ostore_prev + (long long)par * a.ostride) : P.root32;
+                    sb = reinterpret_cast<const int *>(sT + (long long)opt_tw<Re>(M, K));
+                    sn = sb + M;
+                } else {
+                    sT = warm ? reinterpret_cast<const Re *>(a.ostore_prev + (long long)par * a.ostride) : P.root;
+                    sb = warm ? reinterpret_cast<const int *>(sT + (long long)opt_tw<Re>(M, K)) : P.root_basis;
+                    sn = warm ? sb + M : P.root_nonb;
+                    sld = warm ? sld : K + 2;
+                }
+                reg_load(R, L, P, sT, sld, sb, sn);
+                const int ok = reg_lambda(R, L, P, tl, Sset, warm ? k - 1 : 0, k, sT, sld);
                 __syncthreads();
                 if (ok) break;
                 if (!warm) return false;
@@ -1314,19 +1528,27 @@ __device__ __forceinline__ void reg_body(const OptArgs &a) {
             OPT_PROF(sh, 0);
             p1 = reg_phase1(R, L, P, O, tl, sh, ws);
             OPT_PROF(sh, 3);
-            if (!cert_phase1<NT, SM>(L, P, O, inS, red, sh, Sset, k, p1, pcorr, dcorr)) return false;
+            if constexpr (MIXED) {
+                if (!cert_phase1<NT, SM>(L, P, O, inS, red, sh, Sset, k, p1, pcorr, dcorr)) return false;
+            }
             OPT_PROF(sh, 4);
             p1.kkt = rfl(p1.kkt);
             clean = reg_drive_out(R, L, P, tl, sh, p1.kkt);
             if (a.b1)
                 for (int i = tid; i < M; i += NT) a.b1[(long long)c * M + i] = L.basis[i];
-            if (a.store) reg_store(R, L, M, K, a.ostore_cur + (long long)c * a.ostride);
+            if (a.store && (MIXED || p1.status == ST_OPTIMAL)) {
+                unsigned char *dst = a.ostore_cur + (long long)c * a.ostride;
+                if (MIXED || a.store32) reg_store<float>(R, L, M, K, dst);
+                else reg_store<Re>(R, L, M, K, dst);
+            }
             if (p1.kkt) {
                 __syncthreads();
                 OPT_PROF(sh, 5);
                 p2 = reg_phase2<SN>(R, L, P, O, tl, sh, ws);
                 OPT_PROF(sh, 6);
-                if (!cert_phase2<NT, SM>(L, P, O, inS, red, sh, Sset, k, p2, pcorr, dcorr)) return false;
+                if constexpr (MIXED) {
+                    if (!cert_phase2<NT, SM>(L, P, O, inS, red, sh, Sset, k, p2, pcorr, dcorr)) return false;
+                }
                 if (a.b2)
                     for (int i = tid; i < M; i += NT) a.b2[(long long)c * M + i] = L.basis[i];
             }
@@ -1334,11 +1556,16 @@ __device__ __forceinline__ void reg_body(const OptArgs &a) {
         };
         const bool fail = !solve();
         if (fail) {
-            if (a.b1)
-                for (int i = tid; i < M; i += NT) a.b1[(long long)c * M + i] = -1;
-            if (tid == 0) {
-                Rc.repivots = 1;
-                a.fb_list[atomicAdd(a.fb_count, 1)] = c;
+            if constexpr (MIXED) {
+                // handed to the FP64 re-solve
+                if (a.b1)
+                    for (int i = tid; i < M; i += NT) a.b1[(long long)c * M + i] = -1;
+                if (tid == 0) {
+                    Rc.repivots = 1;
+                    a.fb_list[atomicAdd(a.fb_count, 1)] = c;
+                }
+            } else {
+                if (tid == 0) Rc.p1_status = ST_SINGULAR;
             }
             continue;
         }
@@ -1350,5 +1577,9 @@ __device__ __forceinline__ void reg_body(const OptArgs &a) {
 // EU: waves per SIMD the register budget is for (512 / EU vector registers)
 template <int NW, int RW, int CS, int EX, int SN, int EU>
 __global__ __launch_bounds__(NW *MPQP_WAVE) __attribute__((amdgpu_waves_per_eu(EU, EU))) void reg_kernel32(OptArgs a) {
-    reg_body<NW, RW, CS, EX, SN>(a);
+    reg_body<float, NW, RW, CS, EX, 0, SN>(a);
+}
+template <int NW, int RW, int CS, int EX, int LW, int SN, int EU>
+__global__ __launch_bounds__(NW *MPQP_WAVE) __attribute__((amdgpu_waves_per_eu(EU, EU))) void reg_kernel64(OptArgs a) {
+    reg_body<double, NW, RW, CS, EX, LW, SN>(a);
 }
