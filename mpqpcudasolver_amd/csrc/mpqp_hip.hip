@@ -32,6 +32,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <condition_variable>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -179,6 +180,142 @@ struct Arena {
     virtual void begin_level(int level) { (void)level; }
 };
 
+// Pinned host memory for copies to and from the caller's arrays, SLOTS blocks
+// allocated when first used and kept (32 MiB in all), with an event each.
+struct Staging {
+    static constexpr size_t SLOT = (size_t)4 << 20;
+    static constexpr int SLOTS = 8;
+    unsigned char *p[SLOTS] = {};
+    hipEvent_t ev[SLOTS] = {};
+    unsigned char *slot(int i) {
+        if (!p[i]) {
+            HIP_OK(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming));
+            HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&p[i]), SLOT));
+        }
+        return p[i];
+    }
+};
+
+// Copies from device memory into the caller's arrays through the staging
+// blocks.  A direct copy into pageable memory moves 16 GB/s into pages in use
+// and far less into new ones, which it faults in one by one: the 82 MB of
+// 3,000 regions at n=60 m=120 p=12 took 7 of the call's 8.4 ms, now 3 of 4.5.  Here the
+// device writes pinned blocks (54 GB/s) while up to four threads empty the
+// earlier ones, faults included; a call of less than two blocks' bytes is
+// emptied by the caller's thread.
+class CopyBack {
+  public:
+    struct Seg {
+        size_t off, bytes;  // in the device buffer
+        void *dst;
+    };
+    CopyBack(Staging &s, hipStream_t stream, int device, size_t total) : S(s), st(stream) {
+        if (total < 2 * Staging::SLOT) return;
+        try {
+            for (int t = 0; t < 4; ++t)
+                th.emplace_back([this, device] {
+                    if (hipSetDevice(device) != hipSuccess) return;  // the caller empties what is left
+                    while (drain_one(true)) {}
+                });
+        } catch (const std::exception &) {
+            // fewer threads, or none
+        }
+    }
+    ~CopyBack() { stop(); }
+    // segs (ascending) of the buffer at dev, read in stream order
+    void copy(const unsigned char *dev, const std::vector<Seg> &segs) {
+        size_t i = 0;
+        while (i < segs.size()) {
+            // a run of adjacent segments
+            size_t j = i, end = segs[i].off + segs[i].bytes;
+            while (j + 1 < segs.size() && segs[j + 1].off == end) end += segs[++j].bytes;
+            for (size_t a = segs[i].off; a < end; a += Staging::SLOT)
+                issue(dev, a, std::min(Staging::SLOT, end - a), segs, i, j);
+            i = j + 1;
+        }
+    }
+    // every copy is in its array
+    void finish() {
+        while (drain_one(false)) {}
+        std::unique_lock<std::mutex> lk(m);
+        cv.wait(lk, [this] { return drained == issued; });
+        if (err != hipSuccess) throw HipError{std::string("copy to the host failed: ") + hipGetErrorString(err)};
+    }
+
+  private:
+    struct Part {
+        size_t src, bytes;
+        unsigned char *dst;
+    };
+    Staging &S;
+    hipStream_t st;
+    std::vector<std::thread> th;
+    std::mutex m;
+    std::condition_variable cv;
+    std::vector<Part> parts[Staging::SLOTS];
+    bool busy[Staging::SLOTS] = {};
+    long long issued = 0, taken = 0, drained = 0;
+    bool ended = false;
+    hipError_t err = hipSuccess;
+
+    void issue(const unsigned char *dev, size_t a, size_t bytes, const std::vector<Seg> &segs, size_t i, size_t j) {
+        const int b = (int)(issued % Staging::SLOTS);
+        for (;;) {
+            {
+                std::unique_lock<std::mutex> lk(m);
+                if (!busy[b]) break;
+                if (taken == issued) {  // a thread is at it
+                    cv.wait(lk);
+                    continue;
+                }
+            }
+            drain_one(false);
+        }
+        unsigned char *p = S.slot(b);
+        std::vector<Part> ps;
+        for (size_t k = i; k <= j; ++k) {
+            const size_t lo = std::max(a, segs[k].off), hi = std::min(a + bytes, segs[k].off + segs[k].bytes);
+            if (lo < hi)
+                ps.push_back(Part{lo - a, hi - lo, static_cast<unsigned char *>(segs[k].dst) + (lo - segs[k].off)});
+        }
+        HIP_OK(hipMemcpyAsync(p, dev + a, bytes, hipMemcpyDeviceToHost, st));
+        HIP_OK(hipEventRecord(S.ev[b], st));
+        std::lock_guard<std::mutex> lk(m);
+        parts[b].swap(ps);
+        busy[b] = true;
+        ++issued;
+        cv.notify_all();
+    }
+    // Empties the oldest block not yet taken; wait: until there is one or the
+    // copies have ended.  False: none left.
+    bool drain_one(bool wait) {
+        int b;
+        {
+            std::unique_lock<std::mutex> lk(m);
+            if (wait) cv.wait(lk, [this] { return taken < issued || ended; });
+            if (taken == issued) return false;
+            b = (int)(taken++ % Staging::SLOTS);
+        }
+        const hipError_t e = hipEventSynchronize(S.ev[b]);
+        if (e == hipSuccess)
+            for (const Part &q : parts[b]) std::memcpy(q.dst, S.p[b] + q.src, q.bytes);
+        std::lock_guard<std::mutex> lk(m);
+        if (e != hipSuccess) err = e;
+        busy[b] = false;
+        ++drained;
+        cv.notify_all();
+        return true;
+    }
+    void stop() {
+        {
+            std::lock_guard<std::mutex> lk(m);
+            ended = true;
+            cv.notify_all();
+        }
+        for (std::thread &t : th) t.join();
+    }
+};
+
 // Grow-only hipMalloc'd buffers kept across calls (mpqp()).
 struct PoolArena : Arena {
     struct Buf {
@@ -273,6 +410,7 @@ struct Ctx {
     hipStream_t stream = nullptr;
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     LevelMail *mail = nullptr;  // pinned host memory that the level kernels write
+    Staging staging;            // copies of mpqp_regions()
     MpqpOptions opt{};
     bool opt_set = false;
     std::string err;
@@ -1636,28 +1774,48 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     hipStream_t st = C.stream;
     MpqpRegionStats rs{};
     const int m0 = n_c + n_cp, ldy = n_c + p + 1;
-    // inputs: A, inv_Q, W = [A^T | H | c], Y, GX, b, F, CRA, CRb
-    std::vector<double> W((size_t)n_x * ldy);
-    for (int i = 0; i < n_x; ++i) {
-        for (int j = 0; j < n_c; ++j) W[(size_t)i * ldy + j] = in.A[(size_t)j * n_x + i];
-        for (int t = 0; t < p; ++t) W[(size_t)i * ldy + n_c + t] = in.H[(size_t)i * p + t];
-        W[(size_t)i * ldy + n_c + p] = in.c[i];
-    }
+    // inputs, in one copy: A, inv_Q, W = [A^T | H | c], b, F, CRA, CRb, the
+    // sets; on the device followed by Y, GX
     const size_t nA = (size_t)n_c * n_x, nQ = (size_t)n_x * n_x, nW = (size_t)n_x * ldy, nGX = (size_t)n_c * ldy,
                  nF = (size_t)n_c * p, nCA = (size_t)n_cp * p;
-    const size_t in_doubles = nA + nQ + 2 * nW + nGX + n_c + nF + nCA + n_cp;
-    BufView din = C.pools.get(R_IN, -1, in_doubles * 8);
-    double *dA = din.as<double>(), *dQ = dA + nA, *dW = dQ + nQ, *dY = dW + nW, *dGX = dY + nW, *db = dGX + nGX,
-           *dF = db + n_c, *dCA = dF + nF, *dCb = dCA + nCA;
-    HIP_OK(hipMemcpyAsync(dA, in.A, nA * 8, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(dQ, in.iQ, nQ * 8, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(dW, W.data(), nW * 8, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(db, in.b, (size_t)n_c * 8, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(dF, in.F, nF * 8, hipMemcpyHostToDevice, st));
-    if (n_cp) {
-        HIP_OK(hipMemcpyAsync(dCA, in.CRA, nCA * 8, hipMemcpyHostToDevice, st));
-        HIP_OK(hipMemcpyAsync(dCb, in.CRb, (size_t)n_cp * 8, hipMemcpyHostToDevice, st));
+    const size_t up = (nA + nQ + nW + n_c + nF + nCA + n_cp) * 8, nS = (size_t)in.n_sets * width * 4;
+    BufView din = C.pools.get(R_IN, -1, up + (nW + nGX) * 8);
+    BufView dsets = C.pools.get(R_SETS, -1, nS);
+    double *dA = din.as<double>(), *dQ = dA + nA, *dW = dQ + nQ, *db = dW + nW, *dF = db + n_c, *dCA = dF + nF,
+           *dCb = dCA + nCA, *dY = dCb + n_cp, *dGX = dY + nW;
+    std::vector<double> big;
+    const bool fits = up + nS <= Staging::SLOT;
+    if (!fits) big.resize(up / 8);
+    double *hp = fits ? reinterpret_cast<double *>(C.staging.slot(0)) : big.data();
+    auto put = [&](double *&h, const double *src, size_t cnt) {
+        if (cnt) std::memcpy(h, src, cnt * 8);
+        h += cnt;
+    };
+    {
+        double *h = hp;
+        put(h, in.A, nA);
+        put(h, in.iQ, nQ);
+        for (int i = 0; i < n_x; ++i, h += ldy) {
+            for (int j = 0; j < n_c; ++j) h[j] = in.A[(size_t)j * n_x + i];
+            for (int t = 0; t < p; ++t) h[n_c + t] = in.H[(size_t)i * p + t];
+            h[n_c + p] = in.c[i];
+        }
+        put(h, in.b, n_c);
+        put(h, in.F, nF);
+        put(h, in.CRA, nCA);
+        put(h, in.CRb, n_cp);
+        if (fits && nS) std::memcpy(h, in.sets, nS);
     }
+    // (declared after `big`, destroyed before it: whatever ends the call, the
+    // host memory of the copies stays until the stream is done with it)
+    struct StreamEnd {
+        hipStream_t st;
+        ~StreamEnd() { (void)hipStreamSynchronize(st); }
+    } stream_end{st};
+    HIP_OK(hipMemcpyAsync(din.p, hp, up, hipMemcpyHostToDevice, st));
+    if (nS)
+        HIP_OK(hipMemcpyAsync(dsets.p, fits ? static_cast<const void *>(hp + up / 8) : in.sets, nS,
+                              hipMemcpyHostToDevice, st));
     HIP_OK(hipEventRecord(C.ev[0], st));
     const unsigned ty = (unsigned)(((n_x + 15) / 16) * ((ldy + 15) / 16));
     hipLaunchKernelGGL(gemm_f64_mfma, dim3(ty), dim3(64), 0, st, dQ, n_x, dW, ldy, dY, ldy, n_x, ldy, n_x);
@@ -1665,23 +1823,25 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     hipLaunchKernelGGL(gemm_f64_mfma, dim3(tg), dim3(64), 0, st, dA, n_x, dY, ldy, dGX, ldy, n_c, ldy, n_x);
     HIP_OK(hipGetLastError());
     HIP_OK(hipEventRecord(C.ev[1], st));
-    HIP_OK(hipEventSynchronize(C.ev[1]));
-    float ms = 0.f;
-    HIP_OK(hipEventElapsedTime(&ms, C.ev[0], C.ev[1]));
-    rs.ms_prep = ms;
-    // outputs per set, in one buffer: par_A, par_b, lam_A, lam_b, cr_A, cr_b, center
+    // outputs per set, in one buffer: par_A, par_b, lam_A, lam_b, cr_A, cr_b,
+    // center, the info
     const size_t o_pa = (size_t)n_x * p, o_pb = n_x, o_la = (size_t)width * p, o_lb = width, o_ca = (size_t)m0 * p,
                  o_cb = m0, o_ce = p;
     const size_t per_set = o_pa + o_pb + o_la + o_lb + o_ca + o_cb + o_ce;
+    // (smaller chunks, whose copies would run under the next one's kernel,
+    // lost more to the kernel's last waves: 3,000 sets at n=60 m=120 p=12 took
+    // 5.7 ms in chunks of 16 MiB, 4.3 ms in one)
     const long long chunk_cap = std::max<long long>(1, std::min<long long>(1 << 16, ((long long)256 << 20) /
                                                                                        (long long)(per_set * 8 + 64)));
     const int max_iter = 20 * (m0 + 2 * p + 2) + 1000;
+    std::vector<DevRegion> info((size_t)in.n_sets);
+    const bool any_out = out.par_A || out.par_b || out.lam_A || out.lam_b || out.cr_A || out.cr_b || out.center;
+    CopyBack back(C.staging, st, C.device,
+                  (size_t)in.n_sets * (sizeof(DevRegion) + (any_out ? per_set * 8 : (size_t)0)));
+    float ms = 0.f;
     for (long long s0 = 0; s0 < in.n_sets; s0 += chunk_cap) {
         const int n = (int)std::min<long long>(chunk_cap, in.n_sets - s0);
-        BufView dsets = C.pools.get(R_SETS, -1, (size_t)n * width * 4);
-        BufView dout = C.pools.get(R_OUT, -1, (size_t)n * per_set * 8);
-        BufView dinfo = C.pools.get(R_INFO, -1, (size_t)n * sizeof(DevRegion));
-        HIP_OK(hipMemcpyAsync(dsets.p, in.sets + s0 * width, (size_t)n * width * 4, hipMemcpyHostToDevice, st));
+        BufView dout = C.pools.get(R_OUT, -1, (size_t)n * (per_set * 8 + sizeof(DevRegion)));
         RegionArgs ra{};
         ra.n_c = n_c;
         ra.n_x = n_x;
@@ -1696,43 +1856,43 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
         ra.Y = dY;
         ra.ldy = ldy;
         ra.GX = dGX;
-        ra.sets = dsets.as<const int>();
+        ra.sets = dsets.as<const int>() + (size_t)s0 * width;
         ra.width = width;
-        double *o = dout.as<double>();
-        ra.par_A = o;
-        ra.par_b = ra.par_A + (size_t)n * o_pa;
-        ra.lam_A = ra.par_b + (size_t)n * o_pb;
-        ra.lam_b = ra.lam_A + (size_t)n * o_la;
-        ra.cr_A = ra.lam_b + (size_t)n * o_lb;
-        ra.cr_b = ra.cr_A + (size_t)n * o_ca;
-        ra.center = ra.cr_b + (size_t)n * o_cb;
-        ra.info = dinfo.as<DevRegion>();
+        std::vector<CopyBack::Seg> segs;
+        size_t off = 0;
+        auto part = [&](double *&dev, double *dst, size_t per) {
+            dev = dout.as<double>() + off / 8;
+            if (dst) segs.push_back({off, (size_t)n * per * 8, dst + (size_t)s0 * per});
+            off += (size_t)n * per * 8;
+        };
+        part(ra.par_A, out.par_A, o_pa);
+        part(ra.par_b, out.par_b, o_pb);
+        part(ra.lam_A, out.lam_A, o_la);
+        part(ra.lam_b, out.lam_b, o_lb);
+        part(ra.cr_A, out.cr_A, o_ca);
+        part(ra.cr_b, out.cr_b, o_cb);
+        part(ra.center, out.center, o_ce);
+        ra.info = reinterpret_cast<DevRegion *>(dout.as<unsigned char>() + off);
+        segs.push_back({off, (size_t)n * sizeof(DevRegion), info.data() + s0});
         HIP_OK(hipEventRecord(C.ev[2], st));
         hipLaunchKernelGGL(region_kernel<256>, dim3((unsigned)n), dim3(256), (size_t)lds, st, ra);
         HIP_OK(hipGetLastError());
         HIP_OK(hipEventRecord(C.ev[3], st));
-        std::vector<DevRegion> info(n);
-        HIP_OK(hipMemcpyAsync(info.data(), ra.info, (size_t)n * sizeof(DevRegion), hipMemcpyDeviceToHost, st));
-        auto back = [&](double *dst, const double *src, size_t per) {
-            if (dst) HIP_OK(hipMemcpyAsync(dst + (size_t)s0 * per, src, (size_t)n * per * 8, hipMemcpyDeviceToHost, st));
-        };
-        back(out.par_A, ra.par_A, o_pa);
-        back(out.par_b, ra.par_b, o_pb);
-        back(out.lam_A, ra.lam_A, o_la);
-        back(out.lam_b, ra.lam_b, o_lb);
-        back(out.cr_A, ra.cr_A, o_ca);
-        back(out.cr_b, ra.cr_b, o_cb);
-        back(out.center, ra.center, o_ce);
-        HIP_OK(hipStreamSynchronize(st));
+        back.copy(dout.as<unsigned char>(), segs);
+        HIP_OK(hipEventSynchronize(C.ev[3]));
         HIP_OK(hipEventElapsedTime(&ms, C.ev[2], C.ev[3]));
         rs.ms_sets += ms;
         rs.launches += 1;
-        for (int i = 0; i < n; ++i) {
-            rs.found += info[i].status == MPQP_REGION_FOUND;
-            rs.pivots += info[i].iters;
-        }
-        if (out.info) std::memcpy(out.info + s0, info.data(), (size_t)n * sizeof(DevRegion));
     }
+    back.finish();
+    HIP_OK(hipEventSynchronize(C.ev[1]));
+    HIP_OK(hipEventElapsedTime(&ms, C.ev[0], C.ev[1]));
+    rs.ms_prep = ms;
+    for (const DevRegion &r : info) {
+        rs.found += r.status == MPQP_REGION_FOUND;
+        rs.pivots += r.iters;
+    }
+    if (out.info && !info.empty()) std::memcpy(out.info, info.data(), info.size() * sizeof(DevRegion));
     rs.sets = in.n_sets;
     C.rstats = rs;
     return (int)rs.found;
