@@ -115,6 +115,12 @@ __device__ __forceinline__ float min_r(float a, float b) { return fminf(a, b); }
 __device__ __forceinline__ float max_r(float a, float b) { return fmaxf(a, b); }
 __device__ __forceinline__ double min_r(double a, double b) { return fmin(a, b); }
 __device__ __forceinline__ double max_r(double a, double b) { return fmax(a, b); }
+__device__ __forceinline__ unsigned min_r(unsigned a, unsigned b) { return a < b ? a : b; }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned dpp_get(unsigned old, unsigned v) {
+    return (unsigned)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ unsigned lane_get(unsigned v, int l) { return (unsigned)__builtin_amdgcn_readlane((int)v, l); }
 template <int CTRL, int ROWS, typename Re>
 __device__ __forceinline__ Re dpp_min(Re v) {
     return min_r(v, dpp_get<CTRL, ROWS>(v, v));
@@ -132,30 +138,6 @@ __device__ __forceinline__ Re wave_min(Re v) {
     v = dpp_min<0x142, 0xa>(v);
     v = dpp_min<0x143, 0xc>(v);
     return lane_get(v, 63);
-}
-
-// The two smallest of the wave's values (not NaN; equal ones count twice),
-// known to every lane, in one pass.
-template <int CTRL, int ROWS, typename Re>
-__device__ __forceinline__ void dpp_min2(Re &a, Re &b) {
-    const Re oa = dpp_get<CTRL, ROWS>((Re)INFINITY, a), ob = dpp_get<CTRL, ROWS>((Re)INFINITY, b);
-    b = min_r(min_r(b, ob), max_r(a, oa));
-    a = min_r(a, oa);
-}
-template <typename Re>
-__device__ __forceinline__ void row8_min2(Re &a, Re &b) {  // into lane 7, of lanes 0 .. 7
-    dpp_min2<0x111, 0xf>(a, b);
-    dpp_min2<0x112, 0xf>(a, b);
-    dpp_min2<0x114, 0xf>(a, b);
-}
-template <typename Re>
-__device__ __forceinline__ void wave_min2(Re &a, Re &b) {
-    row8_min2(a, b);
-    dpp_min2<0x118, 0xf>(a, b);
-    dpp_min2<0x142, 0xa>(a, b);
-    dpp_min2<0x143, 0xc>(a, b);
-    a = lane_get(a, 63);
-    b = lane_get(b, 63);
 }
 
 // The reference tree (tree_argmin_s) over float values with an id below 1024
@@ -255,6 +237,7 @@ struct RegTab {
     static constexpr int NS = CS + (EX > 0 ? 1 : 0);  // slots of a decision
     typedef std::conditional_t<sizeof(Re) == 4, v4f, Re> cell;
     cell t[sizeof(Re) == 4 ? RW / 4 : RR][CS];
+    int cb;         // by row: use count of the basic variable (phase 1)
     Re d[NS];       // cost row (the same in every wave)
     Re xs[EX + 2];  // by row (lanes < RW): the extra columns, the rhs, the perturbation
     Re *lt;         // this lane's column of the wave's LDS rows
@@ -277,8 +260,11 @@ struct RegTab {
 // Per-wave results of the distributed decisions.
 template <typename Re>
 struct RegMin {
-    Re m1, m2;    // smallest and second smallest x_B of the wave
-    int at, nan;  // row of the smallest; a NaN among them
+    Re m1;     // smallest x_B of the wave
+    int at;    // its row: of several, the one that the reference tree keeps
+    int cnt;   // use count of the values within the tree's band of m1, if
+    int flag;  // it is the same; 1: it is not, 2: a NaN among the values,
+               // 4: no row
 };
 template <typename Re, int NW>
 struct RegShared {
@@ -394,6 +380,15 @@ __device__ __forceinline__ void reg_rank1(RegTab<float, NW, RW, CS, EX, 0> &R, f
     });
 }
 
+// The LDS rows' entries of column q < 64 CS by lane (lane = row; 0 elsewhere)
+template <int NW, int RW, int CS, int EX, int LW>
+__device__ __forceinline__ double reg_lds_col(const RegTab<double, NW, RW, CS, EX, LW> &R, int q) {
+    const int lane = fresh_lane(), g = lane - (RW - LW);
+    const bool in = (unsigned)g < (unsigned)LW && q < MPQP_WAVE * CS;
+    const double v = R.lt[(in ? (g * CS + q / MPQP_WAVE) * MPQP_WAVE + q % MPQP_WAVE : 0) - lane];
+    return in ? v : 0.0;
+}
+
 // Column q of the wave's rows by lane, through the wave's part of L.colx (a
 // wave's LDS operations stay in order).  CLEAR: the column is left zero
 // (T - f * 1 in its lane), if `on`.
@@ -403,11 +398,10 @@ __device__ __forceinline__ Re reg_col_op(RT &R, const RegLds<Re, NW, RW, CS, EX,
     const int lane = fresh_lane(), lq = q % MPQP_WAVE;
     Re v = 0;
     if constexpr (sizeof(Re) == 8) {
+        if constexpr (LW > 0) v = reg_lds_col(R, q);
         reg_for<CS>([&](auto s) MPQP_INL {
             if (q / MPQP_WAVE == s)
-                reg_for<RW>([&](auto i) MPQP_INL {
-                    v = lane_set(v, i, lane_get(R.template get<decltype(i)::value, decltype(s)::value>(), lq));
-                });
+                reg_for<RW - LW>([&](auto i) MPQP_INL { v = lane_set(v, i, lane_get(R.t[i][s], lq)); });
         });
         reg_for<EX>([&](auto e) MPQP_INL { v = q == MPQP_WAVE * CS + e ? R.xs[e] : v; });
         return v;
@@ -518,29 +512,64 @@ __device__ __forceinline__ void reg_publish(RegTab<Re, NW, RW, CS, EX, LW> &R, c
 // wave that holds the pivot row r finds it zero: its factor -1 puts pr there.
 // FP64: a column whose entry of pr is zero keeps its entries, column q (any,
 // or -1) starts from zero, and the pivot row is put in place.
-template <typename Re, int NW, int RW, int CS, int EX, int LW>
+template <bool COL = false, typename Re, int NW, int RW, int CS, int EX, int LW>
 __device__ __forceinline__ void reg_apply(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L,
                                           const Re (&pr)[CS + 1], Re fv, int r, int q) {
     const int lane = fresh_lane(), wave = wave_id(), lr = r - wave * RW;
     if constexpr (sizeof(Re) == 8) {
         constexpr int CH = 16;  // rows whose factors are in scalar registers at a time
-        reg_for<(RW + CH - 1) / CH>([&](auto h) MPQP_INL {
-            constexpr int i0 = decltype(h)::value * CH, n = RW - i0 < CH ? RW - i0 : CH;
+        const int lq = q % MPQP_WAVE;
+        // (COL: the factors are column q, taken a chunk at a time: its lane's
+        // entries of one slot, or the extra column that fv already is)
+        constexpr int RR = RW - LW;
+        if constexpr (LW > 0) {
+            if (COL && q < MPQP_WAVE * CS) fv = reg_lds_col(R, q < 0 ? 0 : q);
+        }
+        reg_for<(RR + CH - 1) / CH>([&](auto h) MPQP_INL {
+            constexpr int i0 = decltype(h)::value * CH, n = RR - i0 < CH ? RR - i0 : CH;
             Re f[n];
-            reg_for<n>([&](auto i) MPQP_INL { f[i] = lane_get(fv, i0 + decltype(i)::value); });
+            if (!COL || (EX > 0 && q >= MPQP_WAVE * CS)) {
+                reg_for<n>([&](auto i) MPQP_INL { f[i] = lane_get(fv, i0 + decltype(i)::value); });
+            }
+            if constexpr (COL)
+                reg_for<CS>([&](auto s) MPQP_INL {
+                    if (q / MPQP_WAVE == s)
+                        reg_for<n>([&](auto i) MPQP_INL {
+                            constexpr int I = i0 + decltype(i)::value;
+                            f[i] = lane_get(R.t[I][s], lq);
+                            fv = lane_set(fv, I, f[i]);
+                        });
+                });
             reg_for<CS>([&](auto s) MPQP_INL {
                 constexpr int S = decltype(s)::value;
                 const bool at = lane + MPQP_WAVE * S == q;
                 if (pr[S] != (Re)0 && !at)
                     reg_for<n>([&](auto i) MPQP_INL {
                         constexpr int I = i0 + decltype(i)::value;
-                        R.template set<I, S>(fma(-f[i], pr[S], R.template get<I, S>()));
+                        R.t[I][S] = fma(-f[i], pr[S], R.t[I][S]);
                     });
                 if (at)
                     reg_for<n>([&](auto i) MPQP_INL {
                         constexpr int I = i0 + decltype(i)::value;
-                        R.template set<I, S>(fma(-f[i], pr[S], (Re)0));
+                        R.t[I][S] = fma(-f[i], pr[S], (Re)0);
                     });
+            });
+        });
+        // the LDS rows, G of them in flight
+        constexpr int G = 4;
+        reg_for<(LW + G - 1) / G>([&](auto h) MPQP_INL {
+            constexpr int g0 = decltype(h)::value * G, n = LW - g0 < G ? LW - g0 : G;
+            Re f[n];
+            reg_for<n>([&](auto i) MPQP_INL { f[i] = lane_get(fv, RR + g0 + i); });
+            reg_for<CS>([&](auto s) MPQP_INL {
+                Re x[n];
+                reg_for<n>([&](auto i) MPQP_INL { x[i] = R.lt[((g0 + i) * CS + s) * MPQP_WAVE]; });
+                const bool at = lane + MPQP_WAVE * s == q;
+                reg_for<n>([&](auto i) MPQP_INL {
+                    x[i] = fma(-f[i], pr[s], at ? (Re)0 : x[i]);
+                });
+                if (pr[s] != (Re)0)
+                    reg_for<n>([&](auto i) MPQP_INL { R.lt[((g0 + i) * CS + s) * MPQP_WAVE] = x[i]; });
             });
         });
         if ((unsigned)lr < (unsigned)RW) reg_set_row(R, lr, pr);
@@ -568,7 +597,9 @@ template <bool MAYBE = false, typename Re, int NW, int RW, int CS, int EX, int L
 __device__ __forceinline__ void reg_update(RegTab<Re, NW, RW, CS, EX, LW> &R, const RegLds<Re, NW, RW, CS, EX, LW> &L, int r, int q) {
     const int lane = fresh_lane();
     const bool off = MAYBE && r < 0;
-    Re fv = reg_col_op<true>(R, L, q, !off);
+    Re fv = 0;
+    if constexpr (sizeof(Re) == 4) fv = reg_col_op<true>(R, L, q, !off);
+    else reg_for<EX>([&](auto e) MPQP_INL { fv = q == MPQP_WAVE * CS + e ? R.xs[e] : fv; });
     Re pr[CS + 1], dv = 0;
     reg_for<CS + 1>([&](auto s) MPQP_INL {
         pr[s] = L.ep[lane + MPQP_WAVE * s];
@@ -582,7 +613,7 @@ __device__ __forceinline__ void reg_update(RegTab<Re, NW, RW, CS, EX, LW> &R, co
         const Re d0 = lane + MPQP_WAVE * s == q && !off ? (Re)0 : R.d[s];
         R.d[s] = pr[s] != (Re)0 ? fma(-fd, pr[s], d0) : d0;
     });
-    reg_apply(R, L, pr, fv, off ? -MPQP_WAVE * NW : r, off ? -1 : q);
+    reg_apply<true>(R, L, pr, fv, off ? -MPQP_WAVE * NW : r, off ? -1 : q);
 }
 
 // Cost row d = init(column) - c * (sum of the rows whose basic variable
@@ -635,22 +666,32 @@ __device__ __forceinline__ void reg_cost_out(const RegTab<Re, NW, RW, CS, EX, LW
     }
 }
 
-// The wave's two smallest basic values (perturbed: x + xp) for the choice of
-// the leaving row.
+// The wave's smallest basic value (perturbed: x + xp) for the choice of the
+// leaving row.  The reference tree keeps, of equal values with equal counts,
+// the index whose lowest bits are clear first (see tree_first): the smallest
+// index with its bits reversed.
 template <typename Re, int NW, int RW, int CS, int EX, int LW>
 __device__ __forceinline__ void reg_min_out(const RegTab<Re, NW, RW, CS, EX, LW> &R, RegShared<Re, NW> &ws, int M,
                                             bool pert) {
-    const int lane = fresh_lane(), wave = wave_id();
-    const bool valid = lane < RW && wave * RW + lane < M;
+    const int lane = fresh_lane(), wave = wave_id(), row = wave * RW + lane;
+    const bool valid = lane < RW && row < M;
     const Re x = pert ? R.x() + R.xp() : R.x();
     const bool nan = valid && x != x;
     const Re v = (valid && !nan) ? x : (Re)INFINITY;
-    Re m1 = v, m2 = (Re)INFINITY;
-    wave_min2(m1, m2);
-    const int f = __ffsll((long long)__ballot(v == m1)) - 1;
-    const int an = __any(nan) ? 1 : 0;
+    const Re m1 = wave_min(v);
+    const unsigned long long hit = __ballot(v == m1 && valid);
+    const unsigned long long near = hit | __ballot(valid && !((double)m1 <= (double)v - 1e-10));
+    int f = __ffsll((long long)hit) - 1, flag = 0;
+    const int cnt = __builtin_amdgcn_readlane(R.cb, f < 0 ? 0 : f);
+    if ((near & (near - 1)) != 0ull) {
+        flag = (near & ~__ballot(R.cb == cnt)) != 0ull ? 1 : 0;
+        const unsigned k = wave_min((hit >> lane) & 1ull ? __brev((unsigned)row) : ~0u);
+        f = hit ? (int)__brev(k) - wave * RW : f;
+    }
+    if (__any(nan)) flag |= 2;
+    if (hit == 0ull) flag |= 4;
     if (lane == 0) {
-        ws.min[wave] = RegMin<Re>{m1, m2, wave * RW + f, an};
+        ws.min[wave] = RegMin<Re>{m1, wave * RW + f, cnt, flag};
     }
 }
 
@@ -886,6 +927,7 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
     double best_p = -INFINITY;
     int it = 0;
     bool stopped = false;  // uniform, as every condition around the pivots must be
+    R.cb = 0;
     reg_min_out(R, ws, M, n_same >= O.stall_perturb);
     __syncthreads();
     // One exit and one way back, so that the tableau has one place: what
@@ -899,25 +941,29 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
             if (it >= O.max_iter_p1) { act = ACT_STOP; break; }
             pert = !no_pert && n_same >= O.stall_perturb;
             const int lane = fresh_lane();
-            // Leaving row, by every wave: a unique minimum (no NaN, no other
-            // value within the tree's 1e-10 band, no counter preference) wins
-            // every combine of the reference tree; anything else runs the tree.
+            // Leaving row, by every wave.  Without counter preference the
+            // predicate lets a value give way to a smaller one, and within
+            // its 1e-10 band to one of a smaller count: where the counts of
+            // the values within that band of the minimum are all the same
+            // (and none is NaN), the minima win every combine, and of them
+            // the first in the tree's order remains (FP64 values of a
+            // degenerate basis tie exactly, three decisions of four).
+            // Anything else runs the tree.
             const RegMin<Re> w = ws.min[lane % NW];
-            Re m = lane < NW ? w.m1 : (Re)INFINITY, m2 = lane < NW ? w.m2 : (Re)INFINITY;
-            row8_min2(m, m2);
-            m = lane_get(m, 7);
-            m2 = lane_get(m2, 7);
-            const int f = __ffsll((long long)__ballot(w.m1 == m)) - 1;
-            r = __builtin_amdgcn_readlane(w.at, f);
-            const bool tie = m2 == m || (double)m > (double)m2 - 1e-10;
+            const Re m = lane_get(row8_min(lane < NW ? w.m1 : (Re)INFINITY), 7);
             const bool go_on = (double)m < tl.dual_stop_tol;
             const int mode_b = (n_same % 20) >= 10 ? 1 : 0;
-            if (rfl((mode_b || tie || __any(w.nan)) ? 1 : 0)) {
+            const unsigned long long wh = __ballot(lane < NW && w.m1 == m && !(w.flag & 4));
+            const bool wn = lane < NW && !((double)m <= (double)w.m1 - 1e-10);
+            const int f = __ffsll((long long)wh) - 1;
+            r = __builtin_amdgcn_readlane(w.at, f < 0 ? 0 : f);
+            const int c0 = __builtin_amdgcn_readlane(w.cnt, f < 0 ? 0 : f);
+            const bool mixed_counts = wn && ((w.flag & 1) || w.cnt != c0);
+            if ((wh & (wh - 1)) != 0ull)
+                r = (int)__brev(lane_get(row8_min((wh >> lane) & 1ull ? __brev((unsigned)w.at) : ~0u), 7));
+            if (rfl((mode_b || f < 0 || __any(mixed_counts || (lane < NW && (w.flag & 2)))) ? 1 : 0)) {
                 Re v[SM];
                 int id[SM], cn[SM];
-                bool other = false;
-                unsigned long long hit[SM];
-                int c0 = -1;
 #pragma unroll
                 for (int s = 0; s < SM; ++s) {
                     const int i = lane + MPQP_WAVE * s;
@@ -928,26 +974,9 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
                     id[s] = ic;
                     cn[s] = L.bcnt[L.basis[ic]];
                 }
-                // Several minima, or values within the band of the minimum:
-                // where their counts are all the same, the predicate keeps
-                // the smaller value, the first of the minima in its order
-                // (the values of a degenerate basis tie exactly).
-                reg_for<SM>([&](auto s) MPQP_INL {
-                    const bool valid = lane + MPQP_WAVE * s < M;
-                    hit[s] = __ballot(valid && v[s] == m);
-                    if (c0 < 0 && hit[s]) c0 = __builtin_amdgcn_readlane(cn[s], __ffsll((long long)hit[s]) - 1);
-                });
-                reg_for<SM>([&](auto s) MPQP_INL {
-                    const bool valid = lane + MPQP_WAVE * s < M;
-                    other |= valid && !((double)m <= (double)v[s] - 1e-10) && cn[s] != c0;
-                });
-                if (rfl((mode_b || __any(w.nan) || __any(other)) ? 1 : 0)) {
-                    r = reg_tree<SM>(v, id, cn, M, lane, DminPred{mode_b, tl.dual_stop_tol});
-                } else {
-                    r = tree_first<SM>(hit);
-                }
-                r = rfl(r);
+                r = reg_tree<SM>(v, id, cn, M, lane, DminPred{mode_b, tl.dual_stop_tol});
             }
+            r = rfl(r);
             if (rfl(go_on ? 1 : 0)) break;
             act = ACT_STOP;
             if (pert) {
@@ -962,6 +991,7 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
             best_p = -INFINITY;
             __syncthreads();
             if (threadIdx.x == 0) L.bcnt[L.basis[r]] += 1;
+            R.cb += lane == r - wave * RW ? 1 : 0;
             reg_min_out(R, ws, M, false);
             __syncthreads();
             ++it;
@@ -1073,14 +1103,9 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
         }
         stall = n_same > O.stall_exit;
         // the bookkeeping's reads pass while the tableau is updated
-        int bv = 0, nv = 0, bc = 0, nc = 0;
-        if (wave == NW - 1) {
-            bv = L.basis[r];
-            nv = L.nonb[q];
-            bc = L.bcnt[bv];
-            nc = L.nbcnt[nv];
-        }
+        const int bv = L.basis[r], nv = L.nonb[q], bc = L.bcnt[bv], nc = L.nbcnt[nv], ec = L.bcnt[nv];
         reg_update(R, L, r, q);
+        R.cb = fresh_lane() == r - wave * RW ? ec : R.cb;
         if (threadIdx.x == (NW - 1) * MPQP_WAVE) {
             L.bcnt[bv] = bc + 1;
             L.nbcnt[nv] = nc + 1;
