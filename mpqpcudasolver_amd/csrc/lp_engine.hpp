@@ -81,13 +81,16 @@ struct DevProb {
     // Rows in slots ordered longest first (csr_row: slot -> row), ELL layout
     // interleaved for the row teams (GR lanes): entry t of slot sl at
     // ((t / GR) * M2 + sl) * GR + t % GR; csr_n: the slot's step count.
-    // Columns contiguous from csc_ptr[v] (a multiple of the column team
-    // size GC): csc_n entries (rows ascending; for a w column those outside
-    // the stationarity rows), padded to whole steps, then for a w column its
-    // csc_x stationarity-row entries.
+    // Columns contiguous in steps of the column team's size GC: the entries
+    // (rows ascending; for a w column those outside the stationarity rows),
+    // padded to whole steps, then for a w column its stationarity-row
+    // entries.  csc_col[v]: first step (17 bits), steps of the first segment
+    // (7), of the second (7), 1 in the last bit for an e-column that is the
+    // unit vector of its row.
     const int *csr_n, *csr_row, *csr_var;
     const double *csr_val;
-    const int *csc_n, *csc_x, *csc_ptr, *csc_row;
+    const int *csc_row;
+    const unsigned *csc_col;
     const double *csc_val;
 };
 

@@ -734,9 +734,10 @@ struct Run {
     // interleaved for teams of GR lanes (entry t of slot sl at ((t / GR) *
     // M2 + sl) * GR + t % GR), csr_n[sl] = the step count of the slot's wave
     // slice rounded up to whole batches of MPQP_CB.  Columns: contiguous
-    // from csc_ptr[v] (a multiple of GC), the first segment (rows
-    // ascending) padded to whole steps, then the second.  Padding entries:
-    // index -1, value 0.
+    // from a multiple of GC, the first segment (rows ascending) padded to
+    // whole steps, then the second; csc_col[v] packs their places and step
+    // counts, and marks the unit columns, which are not read at all (a third
+    // of the columns that phase 1 prices).  Padding entries: index -1, value 0.
     void build_sparse() {
         const int n_c = in.n_c, n_x = in.n_x, n_t = in.n_t, M2 = in.M2, N2 = in.N2;
         const double *A2 = in.A2;
@@ -789,24 +790,30 @@ struct Run {
                 rval[er] = a;
             }
         }
-        BufView dsp_i = A.get(K_SPI, -1, sizeof(int) * (2 * M2 + 3 * N2 + rvar.size() + crow.size()));
+        // 17 + 7 + 7 bits hold any LP of at most 512 rows (csc_col)
+        std::vector<unsigned> ccol(N2);
+        for (int v = 0; v < N2; ++v) {
+            const unsigned at = (unsigned)cptr[v] / GC, n1 = (unsigned)(cn[v] + GC - 1) / GC, n2 = (unsigned)(cx[v] + GC - 1) / GC;
+            if (at >= 1u << 17 || n1 > 127u || n2 > 127u)
+                throw HipError{"mpqp: A2 has too many entries for mixed precision"};
+            const int rho = v - (N2 - M2);
+            const bool unit = rho >= 0 && cn[v] == 1 && cx[v] == 0 && crow[cptr[v]] == rho && cval[cptr[v]] == 1.0;
+            ccol[v] = at | n1 << 17 | n2 << 24 | (unit ? 1u << 31 : 0u);
+        }
+        BufView dsp_i = A.get(K_SPI, -1, sizeof(int) * (2 * M2 + N2 + rvar.size() + crow.size()));
         BufView dsp_d = A.get(K_SPD, -1, sizeof(double) * (rval.size() + cval.size()));
         int *ib0 = dsp_i.as<int>();
         double *db0 = dsp_d.as<double>();
         P.csr_n = ib0;
         P.csr_row = ib0 + M2;
-        P.csc_n = ib0 + 2 * M2;
-        P.csc_x = P.csc_n + N2;
-        P.csc_ptr = P.csc_x + N2;
-        P.csr_var = P.csc_ptr + N2;
+        P.csc_col = reinterpret_cast<unsigned *>(ib0 + 2 * M2);
+        P.csr_var = ib0 + 2 * M2 + N2;
         P.csc_row = P.csr_var + rvar.size();
         P.csr_val = db0;
         P.csc_val = db0 + rval.size();
         upload(const_cast<int *>(P.csr_n), ssteps.data(), sizeof(int) * M2);
         upload(const_cast<int *>(P.csr_row), slot_row.data(), sizeof(int) * M2);
-        upload(const_cast<int *>(P.csc_n), cn.data(), sizeof(int) * N2);
-        upload(const_cast<int *>(P.csc_x), cx.data(), sizeof(int) * N2);
-        upload(const_cast<int *>(P.csc_ptr), cptr.data(), sizeof(int) * N2);
+        upload(const_cast<unsigned *>(P.csc_col), ccol.data(), sizeof(int) * N2);
         upload(const_cast<int *>(P.csr_var), rvar.data(), sizeof(int) * rvar.size());
         upload(const_cast<int *>(P.csc_row), crow.data(), sizeof(int) * crow.size());
         upload(const_cast<double *>(P.csr_val), rval.data(), sizeof(double) * rval.size());

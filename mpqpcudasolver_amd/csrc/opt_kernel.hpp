@@ -178,6 +178,7 @@ struct OptLds {
     }
     // rhs of a row, cost of a slot (certification)
     __device__ __forceinline__ Real rhs_of(int i) const { return T.row(i)[T_rhs]; }
+    __device__ __forceinline__ unsigned col(const DevProb &P, int v) const { return P.csc_col[v]; }
     __device__ __forceinline__ Real cost_of(int k) const { return T.row(T_cost)[k]; }
     // rhs / perturbation entry of row i < M inside the phase-1 and phase-2
     // loops (the global rows' mirrors when the tableau is split)
@@ -1200,7 +1201,7 @@ __device__ __forceinline__ double block_max(double v, double *red) {
 // team sum) and form a second segment of a w column's list, walked only
 // for j in S; the one masked entry left is (row of w_j, w_j), j in S.
 #define MPQP_CB 4   // A2 entries in flight per lane
-#define MPQP_CBL 4  // tableau entries in flight per lane
+#define MPQP_CBL 8  // tableau entries in flight per lane
 #define MPQP_GR 4
 #define MPQP_GC 8
 #define MPQP_GB 2
@@ -1298,29 +1299,29 @@ __device__ __forceinline__ int elist_build(LT &L, const DevProb &P, OptShared &s
     return ne;
 }
 
-// ord[0, n) := 0 .. n-1 with the indexes whose flag holds first, each group
-// ascending (wave 0 builds it, then the workgroup synchronizes).  The column
-// walks below take their teams in this order so that the long columns share
-// the first round of teams instead of stretching every round.
-// n <= 64 S; the flags are evaluated once, all S of a lane together.
+// ord[0, n) := 0 .. n-1 by class (0, 1, 2), each class ascending (wave 0
+// builds it, then the workgroup synchronizes).  The column walks below take
+// their teams in this order so that the long columns share the first rounds
+// of teams instead of stretching every round, and the unit columns the last.
+// n <= 64 S; the classes are evaluated once, all S of a lane together.
 template <int S, typename F>
-__device__ __forceinline__ void order_flag_first(int *ord, int n, F f) {
+__device__ __forceinline__ void order_by_class(int *ord, int n, F f) {
     const int lane = threadIdx.x & (MPQP_WAVE - 1);
     if (threadIdx.x < MPQP_WAVE) {
         const unsigned long long lt = (1ull << lane) - 1ull;
-        bool fl[S];
+        int cl[S];
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             const int i = lane + MPQP_WAVE * s;
-            fl[s] = f(i < n ? i : 0);
+            cl[s] = f(i < n ? i : 0);
         }
         int base = 0;
 #pragma unroll
-        for (int pass = 0; pass < 2; ++pass)
+        for (int pass = 0; pass < 3; ++pass)
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const int i = lane + MPQP_WAVE * s;
-                const bool take = i < n && (fl[s] == (pass == 0));
+                const bool take = i < n && cl[s] == pass;
                 const unsigned long long m = __ballot(take);
                 if (take) ord[base + __popcll(m & lt)] = i;
                 base += __popcll(m);
@@ -1329,13 +1330,22 @@ __device__ __forceinline__ void order_flag_first(int *ord, int n, F f) {
     __syncthreads();
 }
 
-// a column of more than 4 team steps (both segments counted)
-__device__ __forceinline__ bool long_col(const DevProb &P, int v) {
-    return P.csc_n[v] + P.csc_x[v] > 4 * MPQP_GC;
+// a column's place and steps (csc_col)
+__device__ __forceinline__ unsigned col_n1(unsigned m) { return (m >> 17) & 127u; }
+__device__ __forceinline__ unsigned col_n2(unsigned m) { return (m >> 24) & 127u; }
+__device__ __forceinline__ bool col_unit(unsigned m) { return (m >> 31) != 0u; }
+
+// Order of the column walks: columns of more than 4 team steps, the others,
+// unit columns (nothing to read).
+__device__ __forceinline__ int col_class(unsigned m) {
+    return col_unit(m) ? 2 : (col_n1(m) + col_n2(m) > 4u ? 0 : 1);
 }
 
 // One segment of a column walk: steps s < ns of lane g's entries from
 // base (entry base + s * MPQP_GC), row rmask skipped (the masked entry).
+// (The walks are bound by their loads: the next batch loaded ahead, or the
+// steps past a whole batch as one batch with repeats, were 3 to 10% slower
+// for the whole kernel.)
 __device__ __forceinline__ double col_walk(const DevProb &P, unsigned base, unsigned ns, int rmask, const double *y,
                                            double acc) {
     unsigned s = 0;
@@ -1368,14 +1378,15 @@ __device__ __forceinline__ double col_walk(const DevProb &P, unsigned base, unsi
 // Lane g's partial of c - sum over column v of A2 of a * y[row] (c on lane
 // 0): the first segment (rows ascending; for a w column, the rows outside
 // the stationarity block), then for w_j with j in S its stationarity rows.
-__device__ __forceinline__ double col_resid(const DevProb &P, const SBits &sb, int v, int g, double c,
+__device__ __forceinline__ double col_resid(const DevProb &P, const SBits &sb, unsigned m, int v, int g, double c,
                                             const double *y) {
+    if (col_unit(m)) return g == 0 ? fma(-1.0, y[v - (P.N2 - P.M2)], c) : 0.0;
     const int j = v - (P.n_x + P.n_t);
     const bool in = (unsigned)j < (unsigned)P.n_c && sb.has(j);
-    const unsigned base = (unsigned)P.csc_ptr[v] + (unsigned)g;
-    const unsigned ns1 = ((unsigned)P.csc_n[v] + MPQP_GC - 1) / MPQP_GC;
+    const unsigned base = (m & 0x1ffffu) * MPQP_GC + (unsigned)g;
+    const unsigned ns1 = col_n1(m);
     double acc = col_walk(P, base, ns1, in ? P.M2 - P.n_c + j : -2, y, g == 0 ? c : 0.0);
-    if (in) acc = col_walk(P, base + ns1 * MPQP_GC, ((unsigned)P.csc_x[v] + MPQP_GC - 1) / MPQP_GC, -2, y, acc);
+    if (in) acc = col_walk(P, base + ns1 * MPQP_GC, col_n2(m), -2, y, acc);
     return acc;
 }
 
@@ -1563,15 +1574,15 @@ __device__ __forceinline__ int cert_dual(const LT &L, const DevProb &P, const un
         const double c = cost(e0 + rho);
         y[rho] = w >= 0 ? c : c - (double)L.cost_of(-w - 1);
     }
-    int *ord = L.bcnt;  // positions, long columns first (bcnt is free after phase 1)
-    order_flag_first<S>(ord, M, [&](int i) { return long_col(P, L.basis[i]); });
+    int *ord = L.bcnt;  // positions in the order of the walks (bcnt is free after phase 1)
+    order_by_class<S>(ord, M, [&](int i) { return col_class(L.col(P, L.basis[i])); });
     OPT_PROF(sh, 11);
     for (int it = 0;; ++it) {
         double rn = 0.0;
         for (int q = threadIdx.x; q < M * MPQP_GC; q += NT) {
             const int i = ord[q / MPQP_GC], g = q % MPQP_GC;
             const int bv = L.basis[i];
-            double acc = col_resid(P, sb, bv, g, cost(bv), y);
+            double acc = col_resid(P, sb, L.col(P, bv), bv, g, cost(bv), y);
             acc = team_add<MPQP_GC>(acc);
             if (g == 0) r[i] = acc;
             rn = fmax(rn, res_mag(acc));
@@ -1592,17 +1603,17 @@ __device__ __forceinline__ double min_red_cost(LT &L, const DevProb &P, const un
                                                double *red, Sel sel, CostF cost) {
     SBits sb;
     sb.load(inS);
-    // nonbasic slots, long columns first (over the e-list, free again;
+    // nonbasic slots in the order of the walks (over the e-list, free again;
     // identity order if K2 exceeds its M2 + 1 entries)
     int *ord = L.elr;
     const bool use_ord = P.K2 <= P.M2 + 1 && P.K2 <= MPQP_WAVE * S;
-    if (use_ord) order_flag_first<S>(ord, P.K2, [&](int kk) { return long_col(P, L.nonb[kk]); });
+    if (use_ord) order_by_class<S>(ord, P.K2, [&](int kk) { return col_class(L.col(P, L.nonb[kk])); });
     double mn = INFINITY;
     for (int q = threadIdx.x; q < P.K2 * MPQP_GC; q += NT) {
         const int kk = use_ord ? ord[q / MPQP_GC] : q / MPQP_GC, g = q % MPQP_GC;
         const int v = L.nonb[kk];
         if (sel(v)) {
-            const double d = team_add<MPQP_GC>(col_resid(P, sb, v, g, cost(v), L.cx));
+            const double d = team_add<MPQP_GC>(col_resid(P, sb, L.col(P, v), v, g, cost(v), L.cx));
             mn = fmin(mn, d == d ? d : -INFINITY);
         }
     }

@@ -342,6 +342,7 @@ struct RegLds {
         }
     }
     __device__ __forceinline__ Re rhs_of(int i) const { return gx[i]; }
+    __device__ __forceinline__ unsigned col(const DevProb &P, int v) const { return P.csc_col[v]; }
     __device__ __forceinline__ Re cost_of(int k) const { return dl[k]; }
 };
 
