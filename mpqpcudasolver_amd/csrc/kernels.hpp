@@ -97,6 +97,29 @@ __host__ __device__ inline long long feas_lds_bytes(int M, int K, int n_c) {
     return (b + 15) & ~15LL;
 }
 
+// the feasibility LP's part of a candidate's record, the rest cleared (one
+// thread)
+__device__ __forceinline__ void feas_record(DevRecord &R, int level, int status, int iters, int feasible, double z) {
+    R.level = level;
+    R.feas_status = status;
+    R.feas_iters = iters;
+    R.feasible = feasible;
+    R.z_feas = z;
+    R.p1_status = R.p1_iters = R.kkt_feasible = R.p1_warm = 0;
+    R.p2_status = R.p2_iters = R.final_set = 0;
+    R.z1 = R.z2 = 0.0;
+    R.repivots = 0;
+    R.p1_clean = 0;
+}
+
+// rows of S linearly dependent (LICQ screen): no LP, no children
+template <int NT>
+__device__ __forceinline__ void feas_dependent(const FeasArgs &a, int c) {
+    if (threadIdx.x == 0) feas_record(a.rec[c], a.level, ST_SINGULAR, 0, 0, 0.0);
+    if (a.fbasis)
+        for (int i = threadIdx.x; i < a.P.M1; i += NT) a.fbasis[(long long)c * a.P.M1 + i] = -1;
+}
+
 template <int NT>
 __global__ __launch_bounds__(NT) void feas_kernel(FeasArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -116,21 +139,7 @@ __global__ __launch_bounds__(NT) void feas_kernel(FeasArgs a) {
     const DevTol tl = dev_tol64(O);
 
     if (a.licq_fail && a.licq_fail[c]) {
-        // rows of S linearly dependent (LICQ screen): no LP, no children
-        if (tid == 0) {
-            DevRecord &R = a.rec[c];
-            R.level = a.level;
-            R.feas_status = ST_SINGULAR;
-            R.feas_iters = R.feasible = 0;
-            R.z_feas = 0.0;
-            R.p1_status = R.p1_iters = R.kkt_feasible = R.p1_warm = 0;
-            R.p2_status = R.p2_iters = R.final_set = 0;
-            R.z1 = R.z2 = 0.0;
-            R.repivots = 0;
-            R.p1_clean = 0;
-        }
-        if (a.fbasis)
-            for (int i = tid; i < M; i += NT) a.fbasis[(long long)c * M + i] = -1;
+        feas_dependent<NT>(a, c);
         return;
     }
     for (int w = tid; w < nw; w += NT) inS[w] = 0u;
@@ -219,19 +228,7 @@ __global__ __launch_bounds__(NT) void feas_kernel(FeasArgs a) {
         ++iters;
     }
 
-    if (tid == 0) {
-        DevRecord &R = a.rec[c];
-        R.level = a.level;
-        R.feas_status = status;
-        R.feas_iters = iters;
-        R.feasible = feasible;
-        R.z_feas = z;
-        R.p1_status = R.p1_iters = R.kkt_feasible = R.p1_warm = 0;
-        R.p2_status = R.p2_iters = R.final_set = 0;
-        R.z1 = R.z2 = 0.0;
-        R.repivots = 0;
-        R.p1_clean = 0;
-    }
+    if (tid == 0) feas_record(a.rec[c], a.level, status, iters, feasible, z);
     if (a.fbasis)
         for (int i = tid; i < M; i += NT) a.fbasis[(long long)c * M + i] = basis[i];
     if (a.store && feasible) {
@@ -621,6 +618,7 @@ struct P2Pred {  // min_idx_kernel_optimal, batched_simplex.cu:343-344
 
 #include "opt_kernel.hpp"
 #include "reg_kernel.hpp"
+#include "feas_reg.hpp"
 
 // ---------------------------------------------------------------------
 // Root: S = {} KKT basis tableau (one workgroup, tableau in global memory)

@@ -92,6 +92,13 @@ const std::vector<RegConfig> &reg_configs() {
     return c;
 }
 
+const std::vector<FeasConfig> &feas_configs() {
+#define MPQP_CFG(part, ...) feas_config_part##part(),
+    static const std::vector<FeasConfig> c = {MPQP_FEAS_PARTS(MPQP_CFG)};
+#undef MPQP_CFG
+    return c;
+}
+
 // The feasibility kernel at a workgroup size the autotuner may choose.
 void launch_feas(int nt, int grid, size_t lds, hipStream_t st, const FeasArgs &fa) {
     switch (nt) {
@@ -671,6 +678,7 @@ struct Run {
     long long fstride = 0, flds = 0, ostride = 0, lds64 = 0, lds32 = 0;
     bool gt64 = false, gt32 = false;
     int R64 = 0, R32 = 0;  // rows of a split tableau kept in LDS
+    const FeasConfig *freg = nullptr;  // feasibility tableau in registers (null: LDS)
     int S = 1, feas_nt = 256, opt_nt = OPT_NT, cap64 = 0, cap32 = 0;
     int w32 = 2, w64 = 1;                // workgroups per CU a split tableau is sized for
     size_t gtab64_max = 0, gtab32_max = 0;  // global rows of the largest variant
@@ -919,6 +927,20 @@ struct Run {
         if (reg64) gt64 = false;
         S = red_slots(std::max(M2, N2 - in.n_eqs));
         feas_nt = feas_threads_for(M1, K1);
+        // Registers from 4,800 entries: LDS holds a smaller tableau as many
+        // times as a CU has waves for, and its one wave per decision is no
+        // worse (91 x 39, 70,376 LPs: 2.25 ms against 2.90; 92 x 45, 73,227:
+        // 2.90 against 3.01; 100 x 49, 98,855: 5.20 against 4.36; 124 x 61,
+        // 5,887: 0.63 against 0.41; 112 x 97, 5,051: 0.97 against 0.59;
+        // 144 x 73, 288,101: 67.3 against 24.8).
+        freg = nullptr;
+        for (const FeasConfig &c : feas_configs())
+            if ((M1 + 1) * (K1 + 1) > 4800 && M1 <= c.rows() && K1 <= c.columns()) {
+                freg = &c;
+                feas_nt = c.threads();
+                flds = reg64_lds_bytes(c.nw, c.rw, c.cs, 0, M1, K1, M1 + K1);
+                break;
+            }
         // 1024 threads only where every optimality kernel of the call splits its tableau
         const bool all_split = gt64 && (gt32 || o.precision != MPQP_MIXED);
         const int nt0 = o.opt_threads == 1024 ? (all_split ? 1024 : OPT_NT)
@@ -945,7 +967,7 @@ struct Run {
         if (o.autotune && o.batching == MPQP_PERSISTENT && o.opt_threads == 0 && (!tuned_split || o.split_wgs == 0)) {
             auto it = C.tuned.find(tkey);
             if (it != C.tuned.end()) {
-                feas_nt = it->second[0];
+                if (!freg) feas_nt = it->second[0];
                 select_variant(it->second[1], it->second[2], it->second[3]);
             } else {
                 tune_pending = true;
@@ -1193,7 +1215,7 @@ struct Run {
         // (or of the last level), time each workgroup size; the real
         // launches below overwrite what the trials wrote
         const bool tune_here = tune_pending && (n >= 2048 || level == last_lvl);
-        if (tune_here) {
+        if (tune_here && !freg) {
             FeasArgs ft = fa;
             ft.n = std::min(n, 8192);
             float best = INFINITY;
@@ -1212,7 +1234,8 @@ struct Run {
             }
         }
         HIP_OK(hipEventRecord(e0, st));
-        launch_feas(feas_nt, n, (size_t)flds, st, fa);
+        if (freg) hipLaunchKernelGGL(freg->fn, dim3(n), dim3(feas_nt), (size_t)flds, st, fa);
+        else launch_feas(feas_nt, n, (size_t)flds, st, fa);
         HIP_OK(hipGetLastError());
         HIP_OK(hipEventRecord(e1, st));
 

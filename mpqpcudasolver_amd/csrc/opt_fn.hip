@@ -7,7 +7,23 @@
 #define MPQP_CAT_(a, b) a##b
 #define MPQP_CAT(a, b) MPQP_CAT_(a, b)
 
-#if MPQP_PART >= 8
+#if MPQP_PART >= 20
+
+template <int P>
+struct Part;
+#define MPQP_PICK(part, nw_, rw_, cs_, ex_, eu_)                                    \
+    template <>                                                                     \
+    struct Part<part> {                                                             \
+        static constexpr int nw = nw_, rw = rw_, cs = cs_, ex = ex_, eu = eu_;      \
+    };
+MPQP_FEAS_PARTS(MPQP_PICK)
+
+FeasConfig MPQP_CAT(feas_config_part, MPQP_PART)() {
+    typedef Part<MPQP_PART> P;
+    return FeasConfig{P::nw, P::rw, P::cs, P::ex, P::eu, &feas_reg<P::nw, P::rw, P::cs, P::ex, P::eu>};
+}
+
+#elif MPQP_PART >= 8
 
 template <int P>
 struct Part;

@@ -38,6 +38,25 @@ MPQP_OPT_PARTS(MPQP_DECL)
     X(18, false, 8, 32, 0, 2, 8, 6, 2)     \
     X(19, false, 8, 42, 11, 3, 4, 6, 2)
 
+// Feasibility LPs with the tableau in registers (parts 20 ..): waves, rows
+// per wave, column slots, extra columns, waves per SIMD.
+#define MPQP_FEAS_PARTS(X)   \
+    X(20, 4, 32, 1, 0, 4)    \
+    X(21, 4, 40, 1, 12, 3)   \
+    X(22, 4, 40, 2, 0, 2)
+
+struct FeasConfig {
+    int nw, rw, cs, ex, eu;
+    void (*fn)(FeasArgs);
+    int rows() const { return nw * rw; }
+    int columns() const { return 64 * cs + ex; }
+    int threads() const { return nw * 64; }
+};
+
+#define MPQP_DECL(part, ...) __attribute__((visibility("hidden"))) FeasConfig feas_config_part##part();
+MPQP_FEAS_PARTS(MPQP_DECL)
+#undef MPQP_DECL
+
 struct RegConfig {
     bool fp32;
     int nw, rw, lw, cs, ex, sn, eu;
