@@ -271,7 +271,7 @@ def roofline(st: dict, st64: dict | None, lps, lds_peak: float, fp32: bool) -> d
     if st64 is None and "per_problem_pivots" not in st:
         return {"bound": None, "kernel": None, "note": "no pivot counts for this workload without --compare"}
     if ms_opt >= st["ms_feas"]:
-        name = "opt_kernel32 (FP32 pivots + FP64 certification)" if fp32 else "opt_kernel64"
+        name = "reg_kernel32 (FP32 pivots + FP64 certification)" if fp32 else "reg_kernel64"
         launches = st["launches_opt"] - st["launches_fallback"]
         s = 4.0 if fp32 else 8.0
         # per problem: the FP64 path's phase-1 / phase-2 pivots at this element size
@@ -320,7 +320,8 @@ def roofline(st: dict, st64: dict | None, lps, lds_peak: float, fp32: bool) -> d
         bound = "hbm" if in_global else "lds"
         note = ("HBM3E 8 TB/s: the tableau exceeds one workgroup's LDS and lives in global memory"
                 if in_global else
-                f"LDS read bandwidth measured on this device by mpqp_measure_lds_bandwidth "
+                f"a tableau in registers or LDS, priced at the LDS read bandwidth measured on this device by "
+                f"mpqp_measure_lds_bandwidth "
                 f"(nominal 256 CU x 128 B/clk x 2.4 GHz = {LDS_NOMINAL / 1e12:.1f} TB/s)")
     return {
         "bound": bound,
@@ -494,8 +495,8 @@ def main() -> int:
                              "speedup": h["value"] / h["v64"] if h["v64"] > 0 else None, **h["cmp"]}
         out["fp64_persistent_autotuned"] = {"value": h["v64p"], "ms_per_step": h["dt64p"] / args.steps * 1e3,
                                             "speedup": h["value"] / h["v64p"] if h["v64p"] > 0 else None}
-    if (out["roofline"]["kernel"] or "").startswith("opt_kernel"):
-        kname = "opt_kernel32" if fp32 else "opt_kernel64"
+    if (out["roofline"]["kernel"] or "").startswith("reg_kernel"):
+        kname = "reg_kernel32" if fp32 else "reg_kernel64"
         variant = f"{args.precision}_{args.batching}"
         out["roofline"]["traffic"] = profiled_traffic(kname, args.config, variant)
         if out["roofline"]["traffic"] is not None:

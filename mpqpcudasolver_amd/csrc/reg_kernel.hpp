@@ -35,8 +35,10 @@
 // n=60 m=120 p=12.  The LDS and split kernels (opt_kernel.hpp) spend the same
 // chain and a pass over the tableau: n=60 m=120 p=12 |S|<=3 mixed 822 -> 571 ms
 // with the FP32 tableau and -> 486 ms with the re-solves' FP64 too; FP64
-// |S|<=2 at that size 57 -> 25 ms of kernel time, n=30 m=62 p=8 |S|<=3 18.4
-// -> 8.5 ms, n=6 m=28 p=4 |S|<=6 6.4 -> 3.1 ms.
+// |S|<=2 at that size 57 -> 24.5 ms of kernel time, n=30 m=62 p=8 |S|<=3 18.4
+// -> 7.8 ms, n=6 m=28 p=4 |S|<=6 6.4 -> 2.9 ms.  An FP64 update takes 2,800
+// cycles at 171 x 102 and 5,500 at 325 x 194, where the vector unit's issue
+// bounds it (two waves per SIMD, four cycles an instruction).
 #pragma once
 #include <type_traits>
 #include <utility>
