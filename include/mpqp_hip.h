@@ -247,6 +247,8 @@ int mpqp_get_stats(MpqpStats *stats);
 
 /* Workgroup sizes (threads per LP) of the feasibility and optimality kernels
  * used by the last mpqp() call (chosen by the autotuner in persistent mode).
+ * An optimality tableau in registers has a workgroup of its own, which is not
+ * chosen: opt_threads is then the size that an LDS tableau would have had.
  * No counterpart in the reference. */
 int mpqp_get_tuning(int *feas_threads, int *opt_threads);
 
