@@ -1864,6 +1864,11 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     const long long chunk_cap = std::max<long long>(1, std::min<long long>(1 << 16, ((long long)256 << 20) /
                                                                                        (long long)(per_set * 8 + 64)));
     const int max_iter = 20 * (m0 + 2 * p + 2) + 1000;
+    // 128 threads up to 2,000 entries of the Chebyshev LP's tableau, whose
+    // pivots then leave half of 256 idle (3,000 sets, device ms at 128 / 256:
+    // 25 x 7 0.030 / 0.047, 61 x 23 0.338 / 0.421, 79 x 19 0.332 / 0.339,
+    // 145 x 27 1.92 / 1.37)
+    const bool small = (long long)(m0 + 1) * (2 * p + 3) <= 2000;
     std::vector<DevRegion> info((size_t)in.n_sets);
     const bool any_out = out.par_A || out.par_b || out.lam_A || out.lam_b || out.cr_A || out.cr_b || out.center;
     CopyBack back(C.staging, st, C.device,
@@ -1905,7 +1910,8 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
         ra.info = reinterpret_cast<DevRegion *>(dout.as<unsigned char>() + off);
         segs.push_back({off, (size_t)n * sizeof(DevRegion), info.data() + s0});
         HIP_OK(hipEventRecord(C.ev[2], st));
-        hipLaunchKernelGGL(region_kernel<256>, dim3((unsigned)n), dim3(256), (size_t)lds, st, ra);
+        if (small) hipLaunchKernelGGL(region_kernel<128>, dim3((unsigned)n), dim3(128), (size_t)lds, st, ra);
+        else hipLaunchKernelGGL(region_kernel<256>, dim3((unsigned)n), dim3(256), (size_t)lds, st, ra);
         HIP_OK(hipGetLastError());
         HIP_OK(hipEventRecord(C.ev[3], st));
         back.copy(dout.as<unsigned char>(), segs);
