@@ -33,6 +33,7 @@
 #include <cstring>
 #include <map>
 #include <condition_variable>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -216,19 +217,30 @@ class CopyBack {
         size_t off, bytes;  // in the device buffer
         void *dst;
     };
-    CopyBack(Staging &s, hipStream_t stream, int device, size_t total) : S(s), st(stream) {
-        if (total < 2 * Staging::SLOT) return;
+    CopyBack(Staging &s, hipStream_t stream) : S(s), st(stream) {}
+    // The threads share the object and are not joined: one that starts behind
+    // a busy CPU (up to the scheduler's tick, 4 ms) finds the copies ended and
+    // goes, and the caller does not wait for it.
+    static std::shared_ptr<CopyBack> start(Staging &s, hipStream_t stream, size_t total) {
+        std::shared_ptr<CopyBack> c = std::make_shared<CopyBack>(s, stream);
+        if (total < 2 * Staging::SLOT) return c;
         try {
             for (int t = 0; t < 4; ++t)
-                th.emplace_back([this, device] {
-                    if (hipSetDevice(device) != hipSuccess) return;  // the caller empties what is left
-                    while (drain_one(true)) {}
-                });
+                std::thread([c] {
+                    while (c->drain_one(true)) {}
+                }).detach();
         } catch (const std::exception &) {
             // fewer threads, or none
         }
+        return c;
     }
-    ~CopyBack() { stop(); }
+    // no block is taken any more, and none is being emptied
+    void stop() {
+        std::unique_lock<std::mutex> lk(m);
+        ended = true;
+        cv.notify_all();
+        cv.wait(lk, [this] { return taken == drained; });
+    }
     // segs (ascending) of the buffer at dev, read in stream order
     void copy(const unsigned char *dev, const std::vector<Seg> &segs) {
         size_t i = 0;
@@ -243,6 +255,7 @@ class CopyBack {
     }
     // every copy is in its array
     void finish() {
+        while (arrive()) {}
         while (drain_one(false)) {}
         std::unique_lock<std::mutex> lk(m);
         cv.wait(lk, [this] { return drained == issued; });
@@ -256,12 +269,11 @@ class CopyBack {
     };
     Staging &S;
     hipStream_t st;
-    std::vector<std::thread> th;
     std::mutex m;
     std::condition_variable cv;
     std::vector<Part> parts[Staging::SLOTS];
     bool busy[Staging::SLOTS] = {};
-    long long issued = 0, taken = 0, drained = 0;
+    long long issued = 0, ready = 0, taken = 0, drained = 0;
     bool ended = false;
     hipError_t err = hipSuccess;
 
@@ -276,7 +288,7 @@ class CopyBack {
                     continue;
                 }
             }
-            drain_one(false);
+            if (!arrive()) drain_one(false);
         }
         unsigned char *p = S.slot(b);
         std::vector<Part> ps;
@@ -293,33 +305,36 @@ class CopyBack {
         ++issued;
         cv.notify_all();
     }
-    // Empties the oldest block not yet taken; wait: until there is one or the
-    // copies have ended.  False: none left.
-    bool drain_one(bool wait) {
-        int b;
-        {
-            std::unique_lock<std::mutex> lk(m);
-            if (wait) cv.wait(lk, [this] { return taken < issued || ended; });
-            if (taken == issued) return false;
-            b = (int)(taken++ % Staging::SLOTS);
-        }
-        const hipError_t e = hipEventSynchronize(S.ev[b]);
-        if (e == hipSuccess)
-            for (const Part &q : parts[b]) std::memcpy(q.dst, S.p[b] + q.src, q.bytes);
+    // Waits for the next copy (the caller's thread only: a wait for an event
+    // spins) and hands its block to the threads.  False: none left.
+    bool arrive() {
+        if (ready == issued) return false;
+        const hipError_t e = hipEventSynchronize(S.ev[ready % Staging::SLOTS]);
         std::lock_guard<std::mutex> lk(m);
         if (e != hipSuccess) err = e;
+        ++ready;
+        cv.notify_all();
+        return true;
+    }
+    // Empties the oldest block that has arrived and is not taken; wait: until
+    // there is one or the copies have ended.  False: none left.
+    bool drain_one(bool wait) {
+        int b;
+        bool good;
+        {
+            std::unique_lock<std::mutex> lk(m);
+            if (wait) cv.wait(lk, [this] { return taken < ready || ended; });
+            if (taken == ready || ended) return false;
+            b = (int)(taken++ % Staging::SLOTS);
+            good = err == hipSuccess;
+        }
+        if (good)
+            for (const Part &q : parts[b]) std::memcpy(q.dst, S.p[b] + q.src, q.bytes);
+        std::lock_guard<std::mutex> lk(m);
         busy[b] = false;
         ++drained;
         cv.notify_all();
         return true;
-    }
-    void stop() {
-        {
-            std::lock_guard<std::mutex> lk(m);
-            ended = true;
-            cv.notify_all();
-        }
-        for (std::thread &t : th) t.join();
     }
 };
 
@@ -1871,8 +1886,11 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     const bool small = (long long)(m0 + 1) * (2 * p + 3) <= 2000;
     std::vector<DevRegion> info((size_t)in.n_sets);
     const bool any_out = out.par_A || out.par_b || out.lam_A || out.lam_b || out.cr_A || out.cr_b || out.center;
-    CopyBack back(C.staging, st, C.device,
-                  (size_t)in.n_sets * (sizeof(DevRegion) + (any_out ? per_set * 8 : (size_t)0)));
+    const std::shared_ptr<CopyBack> back = CopyBack::start(C.staging, st, (size_t)in.n_sets * (sizeof(DevRegion) + (any_out ? per_set * 8 : (size_t)0)));
+    struct CopyEnd {
+        CopyBack &c;
+        ~CopyEnd() { c.stop(); }
+    } copy_end{*back};
     float ms = 0.f;
     for (long long s0 = 0; s0 < in.n_sets; s0 += chunk_cap) {
         const int n = (int)std::min<long long>(chunk_cap, in.n_sets - s0);
@@ -1914,13 +1932,13 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
         else hipLaunchKernelGGL(region_kernel<256>, dim3((unsigned)n), dim3(256), (size_t)lds, st, ra);
         HIP_OK(hipGetLastError());
         HIP_OK(hipEventRecord(C.ev[3], st));
-        back.copy(dout.as<unsigned char>(), segs);
+        back->copy(dout.as<unsigned char>(), segs);
         HIP_OK(hipEventSynchronize(C.ev[3]));
         HIP_OK(hipEventElapsedTime(&ms, C.ev[2], C.ev[3]));
         rs.ms_sets += ms;
         rs.launches += 1;
     }
-    back.finish();
+    back->finish();
     HIP_OK(hipEventSynchronize(C.ev[1]));
     HIP_OK(hipEventElapsedTime(&ms, C.ev[0], C.ev[1]));
     rs.ms_prep = ms;
