@@ -938,6 +938,7 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
     bool stall = false;
     for (;;) {
         int r = -1, q = -1, act = ACT_PIVOT;
+        int ec = 0;  // the leaving row's wave: use count of the entering variable
         bool pert = false;
         for (;;) {
             if (stall) { act = ACT_STOP; res.status = ST_STALL; break; }
@@ -1073,7 +1074,13 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
                     qk = reg_tree<NS>(v, id, cnt_of, K, lane, DratioPred{mode});
                 }
                 qk = rfl(qk);
-                if (qk >= 0) reg_publish(R, L, al, lr, qk);
+                if (qk >= 0) {
+                    // read before the barrier: behind it the last wave's first
+                    // thread writes the bookkeeping, whenever it gets there
+                    const int nv = L.nonb[qk];
+                    reg_publish(R, L, al, lr, qk);
+                    ec = L.bcnt[nv];
+                }
                 if (lane == 0) sh.q = qk;
                 MPQP_PRIO_LO();
             }
@@ -1105,11 +1112,19 @@ __device__ __forceinline__ P1Result reg_phase1(RegTab<Re, NW, RW, CS, EX, LW> &R
             ++n_same;
         }
         stall = n_same > O.stall_exit;
-        // the bookkeeping's reads pass while the tableau is updated
-        const int bv = L.basis[r], nv = L.nonb[q], bc = L.bcnt[bv], nc = L.nbcnt[nv], ec = L.bcnt[nv];
+        // Up to the closing barrier the bookkeeping is one thread's alone; its
+        // reads pass while the tableau is updated.
+        const bool keeper = threadIdx.x == (NW - 1) * MPQP_WAVE;
+        int bv = 0, nv = 0, bc = 0, nc = 0;
+        if (keeper) {
+            bv = L.basis[r];
+            nv = L.nonb[q];
+            bc = L.bcnt[bv];
+            nc = L.nbcnt[nv];
+        }
         reg_update(R, L, r, q);
         R.cb = fresh_lane() == r - wave * RW ? ec : R.cb;
-        if (threadIdx.x == (NW - 1) * MPQP_WAVE) {
+        if (keeper) {
             L.bcnt[bv] = bc + 1;
             L.nbcnt[nv] = nc + 1;
             L.basis[r] = nv;
