@@ -32,7 +32,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <condition_variable>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -40,6 +39,7 @@
 #include <vector>
 
 #include "../../include/mpqp_hip.h"
+#include "copy_back.hpp"
 #include "kernels.hpp"
 #include "opt_fn.hpp"
 #include "regions.hpp"
@@ -58,10 +58,6 @@ static_assert(sizeof(MpqpStats) == 160, "MpqpStats layout");
 static __device__ __align__(256) unsigned char scratch[MPQP_SCRATCH_BYTES];
 
 namespace {
-
-struct HipError {
-    std::string msg;
-};
 
 // Threads per feasibility LP when the autotuner does not choose: about 16
 // tableau entries per thread, one wave for a small LP, at most 512.
@@ -149,13 +145,6 @@ int split_rows_for(int M, int K, int N2, bool cert, long long budget) {
     return R;
 }
 
-#define HIP_OK(expr)                                                                   \
-    do {                                                                               \
-        hipError_t e_ = (expr);                                                        \
-        if (e_ != hipSuccess)                                                          \
-            throw HipError{std::string(#expr) + ": " + hipGetErrorString(e_)};         \
-    } while (0)
-
 // A view of a device buffer.
 struct BufView {
     void *p = nullptr;
@@ -186,156 +175,6 @@ struct Arena {
     virtual void set_levels(int nl) { (void)nl; }
     // a new chunk of `level` starts: its previous chunk's buffers are dead
     virtual void begin_level(int level) { (void)level; }
-};
-
-// Pinned host memory for copies to and from the caller's arrays, SLOTS blocks
-// allocated when first used and kept (32 MiB in all), with an event each.
-struct Staging {
-    static constexpr size_t SLOT = (size_t)4 << 20;
-    static constexpr int SLOTS = 8;
-    unsigned char *p[SLOTS] = {};
-    hipEvent_t ev[SLOTS] = {};
-    unsigned char *slot(int i) {
-        if (!p[i]) {
-            HIP_OK(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming));
-            HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&p[i]), SLOT));
-        }
-        return p[i];
-    }
-};
-
-// Copies from device memory into the caller's arrays through the staging
-// blocks.  A direct copy into pageable memory moves 16 GB/s into pages in use
-// and far less into new ones, which it faults in one by one: the 82 MB of
-// 3,000 regions at n=60 m=120 p=12 took 7 of the call's 8.4 ms, now 3 of 4.5.  Here the
-// device writes pinned blocks (54 GB/s) while up to four threads empty the
-// earlier ones, faults included; a call of less than two blocks' bytes is
-// emptied by the caller's thread.
-class CopyBack {
-  public:
-    struct Seg {
-        size_t off, bytes;  // in the device buffer
-        void *dst;
-    };
-    CopyBack(Staging &s, hipStream_t stream) : S(s), st(stream) {}
-    // The threads share the object and are not joined: one that starts behind
-    // a busy CPU (up to the scheduler's tick, 4 ms) finds the copies ended and
-    // goes, and the caller does not wait for it.
-    static std::shared_ptr<CopyBack> start(Staging &s, hipStream_t stream, size_t total) {
-        std::shared_ptr<CopyBack> c = std::make_shared<CopyBack>(s, stream);
-        if (total < 2 * Staging::SLOT) return c;
-        try {
-            for (int t = 0; t < 4; ++t)
-                std::thread([c] {
-                    while (c->drain_one(true)) {}
-                }).detach();
-        } catch (const std::exception &) {
-            // fewer threads, or none
-        }
-        return c;
-    }
-    // no block is taken any more, and none is being emptied
-    void stop() {
-        std::unique_lock<std::mutex> lk(m);
-        ended = true;
-        cv.notify_all();
-        cv.wait(lk, [this] { return taken == drained; });
-    }
-    // segs (ascending) of the buffer at dev, read in stream order
-    void copy(const unsigned char *dev, const std::vector<Seg> &segs) {
-        size_t i = 0;
-        while (i < segs.size()) {
-            // a run of adjacent segments
-            size_t j = i, end = segs[i].off + segs[i].bytes;
-            while (j + 1 < segs.size() && segs[j + 1].off == end) end += segs[++j].bytes;
-            for (size_t a = segs[i].off; a < end; a += Staging::SLOT)
-                issue(dev, a, std::min(Staging::SLOT, end - a), segs, i, j);
-            i = j + 1;
-        }
-    }
-    // every copy is in its array
-    void finish() {
-        while (arrive()) {}
-        while (drain_one(false)) {}
-        std::unique_lock<std::mutex> lk(m);
-        cv.wait(lk, [this] { return drained == issued; });
-        if (err != hipSuccess) throw HipError{std::string("copy to the host failed: ") + hipGetErrorString(err)};
-    }
-
-  private:
-    struct Part {
-        size_t src, bytes;
-        unsigned char *dst;
-    };
-    Staging &S;
-    hipStream_t st;
-    std::mutex m;
-    std::condition_variable cv;
-    std::vector<Part> parts[Staging::SLOTS];
-    bool busy[Staging::SLOTS] = {};
-    long long issued = 0, ready = 0, taken = 0, drained = 0;
-    bool ended = false;
-    hipError_t err = hipSuccess;
-
-    void issue(const unsigned char *dev, size_t a, size_t bytes, const std::vector<Seg> &segs, size_t i, size_t j) {
-        const int b = (int)(issued % Staging::SLOTS);
-        for (;;) {
-            {
-                std::unique_lock<std::mutex> lk(m);
-                if (!busy[b]) break;
-                if (taken == issued) {  // a thread is at it
-                    cv.wait(lk);
-                    continue;
-                }
-            }
-            if (!arrive()) drain_one(false);
-        }
-        unsigned char *p = S.slot(b);
-        std::vector<Part> ps;
-        for (size_t k = i; k <= j; ++k) {
-            const size_t lo = std::max(a, segs[k].off), hi = std::min(a + bytes, segs[k].off + segs[k].bytes);
-            if (lo < hi)
-                ps.push_back(Part{lo - a, hi - lo, static_cast<unsigned char *>(segs[k].dst) + (lo - segs[k].off)});
-        }
-        HIP_OK(hipMemcpyAsync(p, dev + a, bytes, hipMemcpyDeviceToHost, st));
-        HIP_OK(hipEventRecord(S.ev[b], st));
-        std::lock_guard<std::mutex> lk(m);
-        parts[b].swap(ps);
-        busy[b] = true;
-        ++issued;
-        cv.notify_all();
-    }
-    // Waits for the next copy (the caller's thread only: a wait for an event
-    // spins) and hands its block to the threads.  False: none left.
-    bool arrive() {
-        if (ready == issued) return false;
-        const hipError_t e = hipEventSynchronize(S.ev[ready % Staging::SLOTS]);
-        std::lock_guard<std::mutex> lk(m);
-        if (e != hipSuccess) err = e;
-        ++ready;
-        cv.notify_all();
-        return true;
-    }
-    // Empties the oldest block that has arrived and is not taken; wait: until
-    // there is one or the copies have ended.  False: none left.
-    bool drain_one(bool wait) {
-        int b;
-        bool good;
-        {
-            std::unique_lock<std::mutex> lk(m);
-            if (wait) cv.wait(lk, [this] { return taken < ready || ended; });
-            if (taken == ready || ended) return false;
-            b = (int)(taken++ % Staging::SLOTS);
-            good = err == hipSuccess;
-        }
-        if (good)
-            for (const Part &q : parts[b]) std::memcpy(q.dst, S.p[b] + q.src, q.bytes);
-        std::lock_guard<std::mutex> lk(m);
-        busy[b] = false;
-        ++drained;
-        cv.notify_all();
-        return true;
-    }
 };
 
 // Grow-only hipMalloc'd buffers kept across calls (mpqp()).
@@ -433,6 +272,7 @@ struct Ctx {
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     LevelMail *mail = nullptr;  // pinned host memory that the level kernels write
     Staging staging;            // copies of mpqp_regions()
+    CopyThreads copy_threads;
     MpqpOptions opt{};
     bool opt_set = false;
     std::string err;
@@ -551,6 +391,7 @@ void ensure_ready() {
     c.scratch_ptr[c.device] = static_cast<unsigned char *>(sp);
     c.scratch_arena.base = static_cast<unsigned char *>(sp);
     c.scratch_arena.cap = MPQP_SCRATCH_BYTES;
+    c.copy_threads.make(4);
     c.ready = true;
 }
 
@@ -1829,9 +1670,10 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     double *dA = din.as<double>(), *dQ = dA + nA, *dW = dQ + nQ, *db = dW + nW, *dF = db + n_c, *dCA = dF + nF,
            *dCb = dCA + nCA, *dY = dCb + n_cp, *dGX = dY + nW;
     std::vector<double> big;
-    const bool fits = up + nS <= Staging::SLOT;
+    C.staging.make();
+    const bool fits = C.staging.ok && up + nS <= Staging::SLOT;
     if (!fits) big.resize(up / 8);
-    double *hp = fits ? reinterpret_cast<double *>(C.staging.slot(0)) : big.data();
+    double *hp = fits ? reinterpret_cast<double *>(C.staging.p[0]) : big.data();
     auto put = [&](double *&h, const double *src, size_t cnt) {
         if (cnt) std::memcpy(h, src, cnt * 8);
         h += cnt;
@@ -1851,8 +1693,9 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
         put(h, in.CRb, n_cp);
         if (fits && nS) std::memcpy(h, in.sets, nS);
     }
-    // (declared after `big`, destroyed before it: whatever ends the call, the
-    // host memory of the copies stays until the stream is done with it)
+    std::vector<DevRegion> info((size_t)in.n_sets);
+    // (declared after `big` and `info`, destroyed before them: whatever ends the
+    // call, the host memory of the copies stays until the stream is done with it)
     struct StreamEnd {
         hipStream_t st;
         ~StreamEnd() { (void)hipStreamSynchronize(st); }
@@ -1884,9 +1727,9 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     // 25 x 7 0.030 / 0.047, 61 x 23 0.338 / 0.421, 79 x 19 0.332 / 0.339,
     // 145 x 27 1.92 / 1.37)
     const bool small = (long long)(m0 + 1) * (2 * p + 3) <= 2000;
-    std::vector<DevRegion> info((size_t)in.n_sets);
     const bool any_out = out.par_A || out.par_b || out.lam_A || out.lam_b || out.cr_A || out.cr_b || out.center;
-    const std::shared_ptr<CopyBack> back = CopyBack::start(C.staging, st, (size_t)in.n_sets * (sizeof(DevRegion) + (any_out ? per_set * 8 : (size_t)0)));
+    const std::shared_ptr<CopyBack> back = std::make_shared<CopyBack>(
+        C.staging, C.copy_threads, st, (size_t)in.n_sets * (sizeof(DevRegion) + (any_out ? per_set * 8 : (size_t)0)));
     struct CopyEnd {
         CopyBack &c;
         ~CopyEnd() { c.stop(); }
