@@ -391,7 +391,8 @@ void ensure_ready() {
     c.scratch_ptr[c.device] = static_cast<unsigned char *>(sp);
     c.scratch_arena.base = static_cast<unsigned char *>(sp);
     c.scratch_arena.cap = MPQP_SCRATCH_BYTES;
-    c.copy_threads.make(4);
+    c.staging.make();
+    if (c.staging.ok) c.copy_threads.make(4);
     c.ready = true;
 }
 
@@ -1670,7 +1671,6 @@ int run_regions(const RegionIn &in, const RegionOut &out) {
     double *dA = din.as<double>(), *dQ = dA + nA, *dW = dQ + nQ, *db = dW + nW, *dF = db + n_c, *dCA = dF + nF,
            *dCb = dCA + nCA, *dY = dCb + n_cp, *dGX = dY + nW;
     std::vector<double> big;
-    C.staging.make();
     const bool fits = C.staging.ok && up + nS <= Staging::SLOT;
     if (!fits) big.resize(up / 8);
     double *hp = fits ? reinterpret_cast<double *>(C.staging.p[0]) : big.data();

@@ -8,7 +8,7 @@ import subprocess
 
 import pytest
 
-from conftest import TESTS
+from conftest import ROOT, TESTS
 
 SOURCE = os.path.join(TESTS, "host", "copy_back_test.cpp")
 SCENARIOS = ["copies", "no_staging", "late_helper", "held_up_helper", "failed_copy", "joined", "forked"]
@@ -30,3 +30,14 @@ def test_scenario(binary, scenario):
         pytest.skip("the sanitizer does not follow a fork of a process with threads")
     r = subprocess.run([path, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr[-3000:]
+
+
+def test_blocks_and_threads_are_made_by_warm_up():
+    """The first regions call of a process is as fast as the others only if
+    neither the pinned blocks nor the threads are made in it."""
+    with open(os.path.join(ROOT, "mpqpcudasolver_amd", "csrc", "mpqp_hip.hip")) as f:
+        src = f.read()
+    body = src[src.index("void ensure_ready()"):]
+    body = body[:body.index("\n}\n")]
+    for call in ("staging.make(", "copy_threads.make("):
+        assert src.count(call) == 1 and call in body, call
