@@ -240,7 +240,16 @@ typedef struct MpqpStats {
     /* rows of the optimality tableau held in LDS (M2 when it fits there; for a
        split tableau the others are global rows whose phase-1 / phase-2 updates
        are applied in batches of lazy_batch pivots) of the FP64 and FP32 kernels */
-    int split_rows_fp64, split_rows_fp32, lazy_batch, reserved_stats;
+    int split_rows_fp64, split_rows_fp32, lazy_batch;
+    /* tableaus held in registers, 8 bits each from the lowest: FP64 optimality,
+       FP32 optimality, feasibility LP.  0: in LDS (or split, or not run), else the
+       kernel's shape, from 1, by its rows x columns (threads):
+         FP64  48x64 (128), 80x64 (128), 128x72 (256), 176x128 (256), 256x136 (512),
+               336x196 (512)
+         FP32  88x68 (128), 128x72 (128), 176x128 (256), 256x136 (256), 352x196 (512),
+               352x256 (512)
+         feasibility  128x64 (256), 160x76 (256), 160x128 (256) */
+    int register_shapes;
 } MpqpStats;
 
 int mpqp_get_stats(MpqpStats *stats);
@@ -248,7 +257,8 @@ int mpqp_get_stats(MpqpStats *stats);
 /* Workgroup sizes (threads per LP) of the feasibility and optimality kernels
  * used by the last mpqp() call (chosen by the autotuner in persistent mode).
  * An optimality tableau in registers has a workgroup of its own, which is not
- * chosen: opt_threads is then the size that an LDS tableau would have had.
+ * chosen (MpqpStats.register_shapes): opt_threads is then the size that an LDS
+ * tableau would have had.
  * No counterpart in the reference. */
 int mpqp_get_tuning(int *feas_threads, int *opt_threads);
 

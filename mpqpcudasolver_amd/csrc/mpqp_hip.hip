@@ -96,6 +96,17 @@ const std::vector<FeasConfig> &feas_configs() {
     return c;
 }
 
+// Place of a register shape among those of its kernel, from 1 (0: none).
+int shape_of(const RegConfig *r) {
+    int n = 0;
+    for (const RegConfig &c : reg_configs()) {
+        if (r && c.fp32 == r->fp32) ++n;
+        if (&c == r) return n;
+    }
+    return 0;
+}
+int shape_of(const FeasConfig *f) { return f ? (int)(f - feas_configs().data()) + 1 : 0; }
+
 // The feasibility kernel at a workgroup size the autotuner may choose.
 void launch_feas(int nt, int grid, size_t lds, hipStream_t st, const FeasArgs &fa) {
     switch (nt) {
@@ -1408,6 +1419,7 @@ struct Run {
         C.stats.split_rows_fp64 = gt64 ? R64 : in.M2;
         C.stats.split_rows_fp32 = gt32 ? R32 : in.M2;
         C.stats.lazy_batch = MPQP_LAZY_KE;
+        C.stats.register_shapes = shape_of(reg64) | shape_of(reg32) << 8 | shape_of(freg) << 16;
         C.last_feas_nt = feas_nt;
         C.last_opt_nt = opt_nt;
         HIP_OK(hipStreamSynchronize(st));
@@ -1519,6 +1531,7 @@ void add_stats(MpqpStats &d, const MpqpStats &s) {
     d.split_rows_fp64 = s.split_rows_fp64;
     d.split_rows_fp32 = s.split_rows_fp32;
     d.lazy_batch = s.lazy_batch;
+    d.register_shapes = s.register_shapes;
     d.ms_fallback += s.ms_fallback;
     d.bytes_fallback += s.bytes_fallback;
     d.flops_fallback += s.flops_fallback;

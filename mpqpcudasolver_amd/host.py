@@ -152,7 +152,7 @@ class MpqpStats(ctypes.Structure):
         ("split_rows_fp64", ctypes.c_int),
         ("split_rows_fp32", ctypes.c_int),
         ("lazy_batch", ctypes.c_int),
-        ("reserved_stats", ctypes.c_int),
+        ("register_shapes", ctypes.c_int),
     ]
 
     def as_dict(self) -> dict:
@@ -639,9 +639,10 @@ class MpqpLib:
                 for key, val in st.items():
                     if key == "tableau_global":
                         tot[key] |= val
-                    elif key != "precision_used":
+                    elif key not in ("precision_used", "register_shapes"):
                         tot[key] += val
-                tot["precision_used"] = st["precision_used"]
+                for key in ("precision_used", "register_shapes"):
+                    tot[key] = st[key]
         return runs, tot or {}
 
 
