@@ -9,9 +9,6 @@ from concurrent.futures import ThreadPoolExecutor
 
 _DIR = os.path.dirname(os.path.abspath(__file__))
 _CSRC = os.path.join(_DIR, "csrc")
-DEPS = [os.path.join(_CSRC, f) for f in ("lp_engine.hpp", "kernels.hpp", "opt_kernel.hpp", "reg_kernel.hpp", "opt_fn.hpp",
-                                         "regions.hpp")] + [
-    os.path.join(os.path.dirname(_DIR), "include", "mpqp_hip.h")]
 # (source, extra flags): the library's host code and small kernels, then the
 # groups of optimality kernels (csrc/opt_fn.hpp), longest compilations first
 UNITS = [(os.path.join(_CSRC, "opt_fn.hip"), [f"-DMPQP_PART={p}"]) for p in (2, 3, 6, 7, 1, 0, 13, 12, 5, 4, 11, 10, 9, 8, 19, 18, 17, 16, 15, 14, 22, 21, 20)] + [

@@ -1,7 +1,7 @@
 // opt_fn.hip — one group of optimality kernels (see opt_fn.hpp).
 #include <hip/hip_runtime.h>
 
-#include "kernels.hpp"
+#include "lp_kernels.hpp"
 #include "opt_fn.hpp"
 
 #define MPQP_CAT_(a, b) a##b
