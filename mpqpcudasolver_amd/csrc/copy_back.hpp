@@ -138,13 +138,16 @@ class CopyThreads {
 // A thread that loses its CPU in mid-piece holds up the call, by a scheduler's
 // slice and more where the program's other threads keep the CPUs busy (those
 // of a BLAS spin for tens of milliseconds after a product).  So the threads
-// stop once SHARE % of the bytes are handed out: the caller copies the rest
-// meanwhile, and waits only for a thread that is inside a piece or a range
-// even then.  A thread that comes later finds the call ended and touches
-// nothing.  3,000 regions at n=60 m=120 p=12 (82 MB; ms a call on the same
-// data / on each of six new problems): 50% 4.1 / 4.0 to 5.5, 70% 3.9 / 3.9 to
-// 12, 100% 3.5 / 3.6 to 13, none 4.7 / 4.6 to 7.6; direct copies 9.8 / 10.4.
-// Pieces of 4 MiB instead of 1: the same / up to 12.
+// stop before the last half of the bytes, or the last ALONE of more: the
+// caller copies those meanwhile, and waits only for a thread that is inside a
+// piece or a range even then.  A thread that comes later finds the call ended
+// and touches nothing.  n=60 m=120 p=12 (27.6 KB a set), ms a call on the same
+// data / on each of several new problems:
+//   3,000 sets, the threads stop at 50% 4.1 / 4.0 to 5.5, at 70% 3.9 / 3.9 to
+//   12, never 3.5 / 3.6 to 13, at once 4.7 / 4.6 to 7.6; direct copies 9.8 /
+//   10.4; pieces of 4 MiB instead of 1 at 70% the same / up to 12;
+//   110,415 sets, at 50% 178 / 205, 64 MiB before the end 118 / 147; direct
+//   337 / 334.
 class CopyBack : public std::enable_shared_from_this<CopyBack> {
   public:
     struct Seg {
@@ -153,7 +156,7 @@ class CopyBack : public std::enable_shared_from_this<CopyBack> {
     };
     // total: bytes of all the copies to come
     CopyBack(Staging &s, CopyThreads &t, hipStream_t stream, size_t total)
-        : S(s), T(t), st(stream), help_from(total >= 2 * Staging::SLOT), limit(total / 100 * SHARE) {}
+        : S(s), T(t), st(stream), help_from(total >= 2 * Staging::SLOT), limit(total - std::min(total / 2, ALONE)) {}
     // segs (ascending) of the buffer at dev, read in stream order
     void copy(const unsigned char *dev, const std::vector<Seg> &segs) {
         if (!S.ok) {
@@ -219,7 +222,7 @@ class CopyBack : public std::enable_shared_from_this<CopyBack> {
 
   private:
     static constexpr size_t PIECE = (size_t)1 << 20, RANGE = (size_t)2 << 20;  // RANGE: a huge page
-    static constexpr size_t SHARE = 50;
+    static constexpr size_t ALONE = (size_t)64 << 20;
     struct Part {
         size_t src, bytes;
         unsigned char *dst;
