@@ -261,6 +261,17 @@ def pivot_bytes(M, K, s):
     return 2.0 * (M + 1) * (K + 1) * s + (M + K + 2) * s
 
 
+def register_shape(st: dict, which: str) -> int:
+    """Shape of a kernel with its tableau in registers, 0: it has it elsewhere."""
+    return st["register_shapes"] >> {"fp64": 0, "fp32": 8, "feas": 16}[which] & 255
+
+
+def threads_per_lp(tuning: dict, st: dict, fp32: bool) -> dict:
+    """Workgroup sizes of the kernels that ran (a register shape has its own)."""
+    shape = register_shape(st, "fp32" if fp32 else "fp64")
+    return {**tuning, "optimality": (128, 128, 256, 256, 512, 512)[shape - 1]} if shape else tuning
+
+
 def roofline(st: dict, st64: dict | None, lps, lds_peak: float, fp32: bool) -> dict:
     """Dominant kernel: the optimality kernel (the FP32 launches of a mixed
     run, fallback launches excluded) or the feasibility kernel, whichever
@@ -271,7 +282,8 @@ def roofline(st: dict, st64: dict | None, lps, lds_peak: float, fp32: bool) -> d
     if st64 is None and "per_problem_pivots" not in st:
         return {"bound": None, "kernel": None, "note": "no pivot counts for this workload without --compare"}
     if ms_opt >= st["ms_feas"]:
-        name = "reg_kernel32 (FP32 pivots + FP64 certification)" if fp32 else "reg_kernel64"
+        held = "reg" if register_shape(st, "fp32" if fp32 else "fp64") else "opt"
+        name = f"{held}_kernel32 (FP32 pivots + FP64 certification)" if fp32 else f"{held}_kernel64"
         launches = st["launches_opt"] - st["launches_fallback"]
         s = 4.0 if fp32 else 8.0
         # per problem: the FP64 path's phase-1 / phase-2 pivots at this element size
@@ -296,7 +308,7 @@ def roofline(st: dict, st64: dict | None, lps, lds_peak: float, fp32: bool) -> d
                     t_hbm += cnt * 2.0 * (lp.M2 - R) * (kk + 1) * s / kb / HBM_PEAK
             split = {"rows_lds": R, "lazy_batch": kb, "t_lds_s": t_lds, "t_hbm_s": t_hbm}
     else:
-        name = "feas_kernel"
+        name = "feas_reg" if register_shape(st, "feas") else "feas_kernel"
         launches, ms = st["launches_feas"], st["ms_feas"]
         byts = flops = 0.0
         for lp, pf in zip(lps, (st64 or st)["per_problem_feas_pivots"]):
@@ -486,7 +498,7 @@ def main() -> int:
                    "checks_per_step": st["candidates"], "problems": len(h["lps"]),
                    "precision_used": "mixed" if st["precision_used"] else "fp64",
                    "fallbacks_fp64": st["fallbacks"], "optimality_lps": st["opt_lps"],
-                   "threads_per_lp": h["tuning"]},
+                   "threads_per_lp": threads_per_lp(h["tuning"], st, fp32)},
         "roofline": roofline(st, h["st64"], h["lps"], lds_peak, fp32),
         "stats": st,
     }
@@ -495,8 +507,8 @@ def main() -> int:
                              "speedup": h["value"] / h["v64"] if h["v64"] > 0 else None, **h["cmp"]}
         out["fp64_persistent_autotuned"] = {"value": h["v64p"], "ms_per_step": h["dt64p"] / args.steps * 1e3,
                                             "speedup": h["value"] / h["v64p"] if h["v64p"] > 0 else None}
-    if (out["roofline"]["kernel"] or "").startswith("reg_kernel"):
-        kname = "reg_kernel32" if fp32 else "reg_kernel64"
+    if (out["roofline"]["kernel"] or "").startswith(("reg_kernel", "opt_kernel")):
+        kname = out["roofline"]["kernel"].split()[0]
         variant = f"{args.precision}_{args.batching}"
         out["roofline"]["traffic"] = profiled_traffic(kname, args.config, variant)
         if out["roofline"]["traffic"] is not None:
