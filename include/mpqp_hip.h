@@ -44,8 +44,10 @@ typedef struct GPUResults {
 } GPUResults;
 
 /* Replaces the reference's warm_up() (bound at main.py:60, no argtypes /
- * restype): creates the HIP context and stream on device 0 and loads the
- * kernels.  Returns 0 on success (the reference ignores the return). */
+ * restype): creates the HIP context and stream on device 0, loads the
+ * kernels, and makes the pinned blocks (32 MiB) and the parked threads that
+ * mpqp_regions() copies with.  Returns 0 on success (the reference ignores the
+ * return). */
 int warm_up(void);
 
 /* Replaces mpqp() of mpqp_cuda.so (argtypes main.py:28-49, call main.py:144).

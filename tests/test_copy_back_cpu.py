@@ -20,6 +20,8 @@ def binary(request, tmp_path_factory):
     flags = ["-fsanitize=thread"] if request.param == "thread" else []
     subprocess.run(["g++", "-std=c++17", "-O2", "-g", "-Wall", "-pthread", "-I" + os.path.join(TESTS, "host"), *flags,
                     SOURCE, "-o", out], check=True)
+    if flags and subprocess.run([out], capture_output=True, timeout=120).returncode != 2:
+        pytest.skip("the thread sanitizer does not start here")  # (without a scenario the program ends with 2)
     return request.param, out
 
 
